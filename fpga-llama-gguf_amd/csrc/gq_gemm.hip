@@ -1,52 +1,77 @@
 // Batched GEMV for gfx950: n_tok tokens share every weight read (prefill, speculative or multi-sequence decode; the
 // batched path the reference plans in ROADMAP.md:78-96). Token t's output row is the single-token GEMV's bit for
 // bit: the same Q8_0 activation quantizer (gemvq_ref.h:236-245, with a per-token RMS norm folded in as the deferred
-// norm of gemvqc16.h:52-59), the same exact block terms floor(sumi * fp16(d_w) * d_x * 2^40) summed in int64 and
-// rounded to FP32 once (gemvqw_engine.h:352-445), the same epilogs. Only the block sums change hands: one int8
-// v_mfma_i32_16x16x32_i8 per 32-weight block gives them for 16 rows x 16 tokens. A block's 32 quants may be
-// permuted as long as the weight and the activation operands agree, so lane group g (lanes 16g..16g+15) takes quants
-// 4g..4g+3 and 16+4g..16+4g+3: Q4_0 and Q4_1 pack exactly those as the low and high nibbles of quant bytes 4g..4g+3,
-// Q8_0 holds them as bytes 4g..4g+3 of its two 16-byte halves, and the activation quantizer stores them in that
-// order. Q4_1 adds the term floor(m_w * s_x * 2^40) with the Q8_1 s_x of each activation block (gemvq_ref.h:194-229).
+// norm of gemvqc16.h:52-59), the same exact block terms floor(sumi * fp16(d_w) * d_x * 2^40) summed exactly and
+// rounded to FP32 once (gemvqw_engine.h:352-445), the same epilogs. Per 32-weight block and 16 rows x 16 tokens the
+// matrix cores do two products:
+//   - one v_mfma_i32_16x16x32_i8 for the block sums. A block's 32 quants may be permuted as long as the weight and the
+//     activation operands agree, so lane group g (lanes 16g..16g+15) takes quants 4g..4g+3 and 16+4g..16+4g+3: Q4_0
+//     and Q4_1 pack exactly those as the low and high nibbles of quant bytes 4g..4g+3, Q8_0 holds them as bytes
+//     4g..4g+3 of its two 16-byte halves, and the activation quantizer stores them in that order. Q4_0 enters as
+//     16 * (q - 8), the nibble moved to the top of its byte (three instructions a block instead of nine for q - 8);
+//   - one v_mfma_f32_16x16x16_f16 for the scale products d_w * d_x of the block: A holds the scales of 16 blocks as
+//     they lie in memory, B the token's scale of this block at the block's place and zeros elsewhere, so every
+//     product comes out alone, exact in FP32, already where the block sums' rows and tokens are.
+// The vector ALUs then do three FP64 instructions a term: both values converted, and one fused multiply-add into an
+// accumulator near 1.5 * 2^52 LSB in the round-toward-minus-infinity mode. There the accumulator's last place is the
+// LSB 2^-40, so that one rounding is the term's floor, and the sum of the floors is exact while it stays within 2^51
+// LSB (checked per 16 blocks; past it the terms go to int64 one by one). The accumulator's bits less those of
+// 1.5 * 2^52 LSB are the integer sum.
+// Q4_1 adds the term floor(m_w * s_x * 2^40) with the Q8_1 s_x of each activation block (gemvq_ref.h:194-229), its
+// product by one more FP16 matrix product of the same form.
 #include "gq_gemv_impl.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace gq {
 namespace {
 
-constexpr int GT = 16;                 // rows and tokens per MFMA tile
-constexpr int GU = 16;                 // blocks per round of a workgroup (each wave sums GU / NWAVES of them)
-constexpr int GW = GU / NWAVES;        // blocks per wave per round
-constexpr int ROW_LDS = GU * 16 + 16;  // LDS bytes per staged row: 16 quant bytes per block, padded so that the 16
-                                       // rows of an operand read fall in distinct banks
+constexpr int GT = 16;             // rows and tokens per MFMA tile
+constexpr int GS = 16;             // blocks per step of a wave
+constexpr int GNW = 8;             // waves per workgroup; wave w sums steps w, w + GNW, ..
+constexpr int GNT = GNW * WAVE;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));  // native vectors (promoted to registers, unlike uint4)
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
-// Activation scratch: token t's block b, 8-byte group g (quants 4g..4g+3 and 16+4g..16+4g+3) at byte
-// ((t * 4 + g) * nb + b) * 8, so a lane's groups of consecutive blocks are contiguous.
-__device__ __forceinline__ size_t act_group(int tok, int g, int nb, int b) {
-    return ((size_t(tok) * 4 + g) * nb + b) * 8;
+// Activation scratch, in the order the waves of gemm_kernel read it (16 consecutive bytes a lane, 1 KiB an
+// instruction): per tile of 16 tokens and step of 16 blocks, the pairs of blocks in turn, lane (r, g) = 16 g + r holding
+// token r's 8-byte groups g (quants 4g..4g+3 and 16+4g..16+4g+3) of the pair's two blocks.
+__device__ __forceinline__ size_t act_group(int tok, int g, int ns, int b) {
+    return ((size_t(tok >> 4) * ns + (b >> 4)) * 8 + (b >> 1 & 7)) * 1024 + size_t(g * 16 + (tok & 15)) * 16 + (b & 1) * 8;
+}
+// Its fp16 scales (and Q8_1 sums): per tile and step, lane (r, g) holds token r's blocks 4g .. 4g + 3.
+__device__ __forceinline__ size_t act_scale(int tok, int ns, int b) {
+    return (size_t(tok >> 4) * ns + (b >> 4)) * 256 + size_t((b >> 2 & 3) * 16 + (tok & 15)) * 4 + (b & 3);
+}
+// And each step's part of the term bound, per tile and step one value a token.
+__device__ __forceinline__ size_t act_bound(int tok, int ns, int step) {
+    return (size_t(tok >> 4) * ns + step) * 16 + (tok & 15);
 }
 
 // ---- activation: token rows -> Q8_0 blocks in operand order ----
 // Workgroup t quantizes token t exactly as the single-token prologue: thread i holds the 16-float items i, i + NT,
 // ... (the two halves of a block in adjacent lanes), the norm scale is the canonical pairwise tree over the row, and
-// v = (x * scale) * w.
+// v = (x * scale) * w. Beside each step of 16 blocks goes its part of the term bound: the sum over the blocks of
+// d_x * 2^40 * (sum of |quants|) / (32 * 127), which times a matrix's wbound bounds the step's terms.
 __global__ __launch_bounds__(NT) void gemm_quant_kernel(GemmQuantArgs a) {
     __shared__ Lds s;
-    const int tok = blockIdx.x, nb = a.cols / 32, n16 = a.cols / 16;
+    const int tok = blockIdx.x, nb = a.cols / 32, ns = nb / GS, n16 = a.cols / 16;
     int8_t * q = a.q;
-    float * d40 = a.d40 + size_t(tok) * nb, * s40 = a.s40 + size_t(tok) * nb;
     if (tok >= a.n_tok) {  // padding tokens: zero quants and scales, whose terms are exactly zero
-        uint4 * z = reinterpret_cast<uint4 *>(q + act_group(tok, 0, nb, 0));
-        for (int i = threadIdx.x; i < n16; i += NT) z[i] = make_uint4(0u, 0u, 0u, 0u);  // 4 groups x nb x 8 bytes
-        for (int i = threadIdx.x; i < nb; i += NT) d40[i] = s40[i] = 0.0f;
+        for (int i = threadIdx.x; i < 2 * nb; i += NT)  // 4 groups of a pair of blocks
+            *reinterpret_cast<uint4 *>(q + act_group(tok, i & 3, ns, i >> 2 << 1)) = make_uint4(0u, 0u, 0u, 0u);
+        for (int i = threadIdx.x; i < nb; i += NT) a.d[act_scale(tok, ns, i)] = a.s[act_scale(tok, ns, i)] = 0;
+        for (int i = threadIdx.x; i < ns; i += NT) a.bound[act_bound(tok, ns, i)] = 0.0f;
         return;
     }
     const float * x = a.x + size_t(tok) * a.x_stride;
     const float sc = a.norm ? block_norm_scale(x, a.cols, a.eps, a.norm_l2, s) : 1.0f;
-    for (int i = threadIdx.x; i < n16; i += NT) {  // n16 is even: both lanes of a pair run every round
+    for (int i = threadIdx.x; i < n16; i += NT) {  // n16 is a multiple of 32: whole steps of lanes run every round
         float v[16];
         load16(x + size_t(i) * 16, v);
         if (a.norm_w) {
@@ -63,69 +88,78 @@ __global__ __launch_bounds__(NT) void gemm_quant_kernel(GemmQuantArgs a) {
         const float d = quantize_half_core(v, packed, sum);
         // half h of block b: its word g (quants 16h + 4g .. 16h + 4g + 3) is word h of group g
         const int b = i >> 1, h = i & 1;
+        uint32_t mag = 0;  // sum of |quants| of the half
 #pragma unroll
-        for (int g = 0; g < 4; ++g) *reinterpret_cast<uint32_t *>(q + act_group(tok, g, nb, b) + 4 * h) = packed[g];
-        if (h == 0) {
-            d40[b] = h2f(f2h(d)) * 1099511627776.0f;                   // * 2^40, exact
-            s40[b] = h2f(f2h(float(sum) * d)) * 1099511627776.0f;      // ggml quantize_row_q8_1: fp16(sum * d)
+        for (int g = 0; g < 4; ++g) {
+            *reinterpret_cast<uint32_t *>(q + act_group(tok, g, ns, b) + 4 * h) = packed[g];
+            mag = __builtin_amdgcn_sad_u8(packed[g] ^ 0x80808080u, 0x80808080u, mag);  // |q + 128 - 128| per byte
         }
+        const uint32_t dh = f2h(d);
+        if (h == 0) {
+            a.d[act_scale(tok, ns, b)] = uint16_t(dh);
+            a.s[act_scale(tok, ns, b)] = uint16_t(f2h(float(sum) * d));  // ggml quantize_row_q8_1: fp16(sum * d)
+        }
+        float bs = h2f(dh) * (1099511627776.0f / 4064.0f) * float(mag);
+        bs = pair_sum_lanes<32>(bs);  // the 32 halves of the step's 16 blocks
+        if ((i & 31) == 0) a.bound[act_bound(tok, ns, i >> 5)] = bs;
     }
 }
 
-// Per-block scale words: fp16 d (Q4_0 in region b, Q8_0 in region c), or d | m << 16 (Q4_1, region b).
+// ---- weights ----
+// One step of one 16-row tile as a wave loads it: lane l takes row l / 4; of its 16 blocks the quants of blocks 4c + l % 4
+// (instruction c: 64 contiguous bytes of a row by four neighbouring lanes; Q8_0 twice) and the scales of blocks
+// 4 (l % 4) .. + 3 as they lie in memory. Weight bytes are read once per launch: the non-temporal hint keeps them from
+// displacing the activations in L2.
 template <int TYPE>
-__device__ __forceinline__ uint32_t load_scale(const WeightView & w, size_t blk) {
-    if constexpr (TYPE == T_Q4_1) return *reinterpret_cast<const uint32_t *>(w.b + blk * 4);
-    return *reinterpret_cast<const uint16_t *>((TYPE == T_Q4_0 ? w.b : w.c) + blk * 2);
-}
-
-// One round's weights as loaded by the workgroup: thread t takes block t % 16 of the round in row t / 16 of the tile
-// (its 16 quant bytes, or 32 for Q8_0, and its fp16 scale), so 16 consecutive threads read 256 contiguous bytes of
-// one row.
-// (Named members rather than arrays: the register allocator keeps them in VGPRs.)
-template <int TYPE, bool PAIR>
-struct WRound {
-    v4u g0, g1, u0, u1;  // quant bytes (g1 / u1: the high halves of Q8_0 blocks) of the matrix and of u
-    uint32_t gd, ud;       // fp16 scales
+struct WStep {
+    v4u q[4];
+    v4u q2[TYPE == T_Q8_0 ? 4 : 1];  // the high halves of Q8_0 blocks
+    typename std::conditional<TYPE == T_Q4_1, v4u, v2u>::type s;  // Q4_1: four (d, m) pairs; others: four d
 };
 
-template <int TYPE, bool PAIR>
-__device__ __forceinline__ void load_wround(const GemmArgs & a, int nb, int row, int rd, WRound<TYPE, PAIR> & o) {
-    const size_t blk = size_t(row) * nb + rd * GU + (threadIdx.x & 15);
-    o.g0 = *reinterpret_cast<const v4u *>(a.w.a + blk * 16);
-    if constexpr (TYPE == T_Q8_0) o.g1 = *reinterpret_cast<const v4u *>(a.w.b + blk * 16);
-    o.gd = load_scale<TYPE>(a.w, blk);
-    if constexpr (PAIR) {
-        o.u0 = *reinterpret_cast<const v4u *>(a.w2.a + blk * 16);
-        if constexpr (TYPE == T_Q8_0) o.u1 = *reinterpret_cast<const v4u *>(a.w2.b + blk * 16);
-        o.ud = load_scale<TYPE>(a.w2, blk);
+// blk: the first block of the step in row l / 4
+template <int TYPE>
+__device__ __forceinline__ void load_wstep(const WeightView & w, size_t blk, int part, WStep<TYPE> & o) {
+    const v4u * p = reinterpret_cast<const v4u *>(w.a + (blk + part) * 16);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.q[c] = __builtin_nontemporal_load(p + 4 * c);
+    if constexpr (TYPE == T_Q8_0) {
+        const v4u * p2 = reinterpret_cast<const v4u *>(w.b + (blk + part) * 16);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o.q2[c] = __builtin_nontemporal_load(p2 + 4 * c);
+    }
+    const size_t sb = blk + 4 * part;
+    if constexpr (TYPE == T_Q4_1) {
+        o.s = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(w.b + sb * 4));
+    } else {
+        o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>((TYPE == T_Q4_0 ? w.b : w.c) + sb * 2));
     }
 }
+
+// A wave's step in its part of LDS, which turns the load order into the operand order: the 16-byte quants of (row r,
+// block 4c + b) at slot 4r + (b + r / 4) % 4 of KiB c (the 16 rows' words of one block then lie in distinct banks), the
+// scales of (row r, blocks 4g .. 4g + 3) at lane (r, g).
+template <int TYPE>
+struct WLds {
+    static constexpr int QH = TYPE == T_Q8_0 ? 2 : 1;
+    uint32_t q[QH][4][256];
+    uint32_t s[WAVE * (TYPE == T_Q4_1 ? 4 : 2)];
+};
 
 template <int TYPE>
-__device__ __forceinline__ uint32_t scale_word(uint32_t sw) {
-    return TYPE == T_Q4_1 ? sw : __float_as_uint(h2f(sw & 0xffffu));
-}
-
-// Thread t's part of a round into an LDS buffer: its 16 quant bytes of every matrix-half at row t / 16, block t % 16
-// (rows padded to ROW_LDS bytes), and its scale word: Q4_0 / Q8_0 the fp16 scale as FP32 bits (converted once here,
-// not once per token lane), Q4_1 the fp16 pair (d, m) as loaded.
-template <int TYPE, bool PAIR>
-__device__ __forceinline__ void stage(const WRound<TYPE, PAIR> & w, uint8_t * lq, uint32_t * ld) {
-    constexpr int QH = TYPE == T_Q8_0 ? 2 : 1, QBUF = GT * ROW_LDS;
-    const int t = threadIdx.x, o = (t >> 4) * ROW_LDS + (t & 15) * 16, od = (t >> 4) * GU + (t & 15);
-    *reinterpret_cast<v4u *>(lq + o) = w.g0;
-    if constexpr (QH == 2) *reinterpret_cast<v4u *>(lq + QBUF + o) = w.g1;
-    ld[od] = scale_word<TYPE>(w.gd);
-    if constexpr (PAIR) {
-        *reinterpret_cast<v4u *>(lq + QH * QBUF + o) = w.u0;
-        if constexpr (QH == 2) *reinterpret_cast<v4u *>(lq + 3 * QBUF + o) = w.u1;
-        ld[GT * GU + od] = scale_word<TYPE>(w.ud);
+__device__ __forceinline__ void stage(const WStep<TYPE> & w, int lane, WLds<TYPE> & l) {
+    const int row = lane >> 2, part = lane & 3, slot = 4 * (4 * row + ((part + (row >> 2)) & 3));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][c][slot]) = w.q[c];
+    if constexpr (TYPE == T_Q8_0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[WLds<TYPE>::QH - 1][c][slot]) = w.q2[c];
     }
+    if constexpr (TYPE == T_Q4_1) *reinterpret_cast<v4u *>(&l.s[4 * (part * 16 + row)]) = w.s;
+    else *reinterpret_cast<v2u *>(&l.s[2 * (part * 16 + row)]) = w.s;
 }
 
-// The A operand of one block: Q4_0 nibbles (low: quants 4g..4g+3, high: 16+4g..) minus 8 in every byte; Q4_1 the
-// nibbles as they are; Q8_0 its two words as they are.
+// The i8 operand of one block from its quant word(s).
 template <int TYPE>
 __device__ __forceinline__ long a_operand(uint32_t lo, uint32_t hi) {
     uint32_t w0 = lo, w1 = hi;
@@ -133,259 +167,350 @@ __device__ __forceinline__ long a_operand(uint32_t lo, uint32_t hi) {
         w0 = lo & 0x0F0F0F0Fu;
         w1 = (lo >> 4) & 0x0F0F0F0Fu;
     }
-    if constexpr (TYPE == T_Q4_0) {
-        const uint32_t n0 = lo & 0x0F0F0F0Fu, n1 = (lo >> 4) & 0x0F0F0F0Fu;
-        // per byte: ((v | 0x80) - 8) ^ 0x80 = v - 8 as int8 for 0 <= v <= 15, no borrow between bytes
-        w0 = ((n0 | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-        w1 = ((n1 | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+    if constexpr (TYPE == T_Q4_0) {  // 16 (q - 8) as int8: the nibble at the top of the byte, its sign bit flipped
+        w0 = ((lo << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
+        w1 = (lo & 0xF0F0F0F0u) ^ 0x80808080u;
     }
     return long((uint64_t(w1) << 32) | w0);
 }
 
-// A lane's activation operands of one round: its token's groups g of the wave's GW blocks (GW * 8 contiguous bytes)
-// and their d * 2^40.
-template <int T>
-struct XRound {
-    v4u q[T][GW / 2];
-    v4f d[T];
-    v4f s[T];  // Q4_1 only
+// The launch as the kernel reads it: the members of a group (one, of a SwiGLU pair) by index, their 16-row tiles after
+// one another.
+struct GemmMember {
+    WeightView w;
+    float * y;
+    const float * res;
+    int rows, y_stride, res_stride, epi, tile0;
+    float wbound;
+};
+struct GemmLaunch {
+    const int8_t * q;
+    const uint16_t * d, * s;
+    const float * bound;
+    int cols, n_tok, n_members, n_tiles;
+    WeightView w2;  // u of a SwiGLU pair
+    GemmMember m[GEMM_MAX_MORE + 1];
+};
+// The member of tile b: the last whose first tile is <= b.
+__device__ __forceinline__ int member_of(const GemmLaunch & a, int b) {
+    int mi = 0;
+    for (int i = 1; i < a.n_members; ++i) mi = b >= a.m[i].tile0 ? i : mi;
+    return mi;
+}
+
+// A lane's activation operands of one step: group g of token r's 16 blocks, and (lane group g) the scales of the
+// token's blocks 4g .. 4g + 3; the step's part of the term bound.
+template <int TYPE, int T>
+struct XStep {
+    v4u q[T][GS / 2];
+    v2u d[T];
+    v2u s[TYPE == T_Q4_1 ? T : 1];
+    float bound;  // the largest over the token tiles
 };
 
 template <int TYPE, int T>
-__device__ __forceinline__ void load_xround(const GemmArgs & a, int nb, int r, int g, int b, XRound<T> & o) {
+__device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lane, int step, XStep<TYPE, T> & o) {
+    float bd[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const int tok = t * GT + r;
-        const v4u * p = reinterpret_cast<const v4u *>(a.q + act_group(tok, g, nb, b));
+        const size_t at = size_t(t) * ns + step;
+        const v4u * p = reinterpret_cast<const v4u *>(a.q + at * 8192) + lane;
 #pragma unroll
-        for (int k = 0; k < GW / 2; ++k) o.q[t][k] = p[k];
-        o.d[t] = *reinterpret_cast<const v4f *>(a.d40 + size_t(tok) * nb + b);
-        if constexpr (TYPE == T_Q4_1) o.s[t] = *reinterpret_cast<const v4f *>(a.s40 + size_t(tok) * nb + b);
+        for (int k = 0; k < GS / 2; ++k) o.q[t][k] = p[k * WAVE];
+        o.d[t] = reinterpret_cast<const v2u *>(a.d + at * 256)[lane];
+        if constexpr (TYPE == T_Q4_1) o.s[t] = reinterpret_cast<const v2u *>(a.s + at * 256)[lane];
+        bd[t] = a.bound[at * 16 + (lane & 15)];
     }
+    o.bound = 0.0f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) o.bound = bd[t] <= o.bound ? o.bound : bd[t];  // a NaN stays
+    if constexpr (T == 2) o.bound = bd[0] != bd[0] ? bd[0] : o.bound;
 }
 
-__device__ __forceinline__ float lane_of(const v4f & v, int j) { return v[j]; }
-
-
-// Whether a round needs the int64 path: some lane's wbound * (largest sum of |d_x * 2^40| over a token's GW blocks)
-// reaches 2^52 (one ballot, so the branch on it is uniform over the wave).
-template <int T>
-__device__ __forceinline__ bool round_needs_exact(const XRound<T> & x, float wbound) {
-    float dm = 0.0f;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        float ds = 0.0f;
-#pragma unroll
-        for (int c = 0; c < GW; ++c) ds += fabsf(lane_of(x.d[t], c));
-        dm = fmaxf(dm, ds);
-    }
-    return __builtin_amdgcn_ballot_w64(!(wbound * dm < 4503599627370496.0f)) != 0;
+// The FP16 operand of one block: the token's scale at the block's place c of lane group gb, zeros elsewhere.
+__device__ __forceinline__ v4h one_scale(const v2u & d, int c, bool mine) {
+    const uint32_t v = mine ? (c & 1 ? d[c >> 1] & 0xffff0000u : d[c >> 1] & 0xffffu) : 0u;
+    const v2u o = c < 2 ? v2u{v, 0u} : v2u{0u, v};
+    return __builtin_bit_cast(v4h, o);
 }
 
-// The wave's GW blocks of a staged round: per block and token tile one MFMA gives the lane's 4 sums (rows 4g + i,
-// token r); each term is floor(sumi * s) with s = fp16(d_w) * d_x * 2^40 exact in FP32 and the product exact in FP64;
-// the GW terms are summed in FP64 and moved to the int64 totals. The FP64 sum is exact while it stays below 2^53 LSB:
-// |term| <= wbound * |d_x * 2^40| (wbound: the member's largest |d_w| times its type's largest |sum of products|),
-// so a round where a lane's wbound * sum |d_x * 2^40| over a token's GW blocks reaches 2^52 (a factor 2 of margin)
-// adds every term of the wave to the int64 totals directly (EXACT).
-template <int TYPE, bool PAIR, int T, bool EXACT>
-__device__ __forceinline__ void round_terms_k(const uint8_t * lq, const uint32_t * ld, int wave, int r, int g,
-                                              const XRound<T> & x, long long (*tot)[4], long long (*totu)[4]) {
-    constexpr int NM = PAIR ? 2 : 1, QH = TYPE == T_Q8_0 ? 2 : 1;
-    constexpr int QBUF = GT * ROW_LDS, DBUF = GT * GU;  // bytes of one matrix-half's quants, scales of one matrix
-    double acc[NM][T][4];
+// 1.5 * 2^52 LSB: the FP64 accumulator's base. Q4_0 block sums carry a factor 16, so the LSB is 2^-36 there.
+template <int TYPE>
+constexpr double acc_base() { return TYPE == T_Q4_0 ? 98304.0 : 6144.0; }
+
+// One step into the accumulators acc[t][i] (row 4g + i, token r of token tile t).
+template <int TYPE, int T>
+__device__ __forceinline__ void step_terms(const WLds<TYPE> & l, const XStep<TYPE, T> & x, int lane, double (*acc)[4]) {
+    const int r = lane & 15, g = lane >> 4;
+    v2u dw, mw;
+    if constexpr (TYPE == T_Q4_1) {  // (d, m) words -> the four d and the four m
+        const v4u s = *reinterpret_cast<const v4u *>(&l.s[4 * lane]);
+        dw = v2u{__builtin_amdgcn_perm(s[1], s[0], 0x05040100u), __builtin_amdgcn_perm(s[3], s[2], 0x05040100u)};
+        mw = v2u{__builtin_amdgcn_perm(s[1], s[0], 0x07060302u), __builtin_amdgcn_perm(s[3], s[2], 0x07060302u)};
+    } else {
+        dw = *reinterpret_cast<const v2u *>(&l.s[2 * lane]);
+    }
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int c = 0; c < 4; ++c) {
+        __builtin_amdgcn_sched_barrier(0);  // four blocks in work at a time: their products must fit in registers
 #pragma unroll
-        for (int t = 0; t < T; ++t)
+        for (int gb = 0; gb < 4; ++gb) {
+            // block 4c + gb: its scales are lane group c's, at place gb
+            const int at = 4 * (4 * r + ((gb + (r >> 2)) & 3)) + g;
+            const long aop = a_operand<TYPE>(l.q[0][c][at], TYPE == T_Q8_0 ? l.q[WLds<TYPE>::QH - 1][c][at] : 0u);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[m][t][i] = 0.0;
-    v4u dw[NM][4];  // scale words of rows 4g + i for the wave's GW = 4 blocks
+            for (int t = 0; t < T; ++t) {
+                const v4u qv = x.q[t][2 * c + (gb >> 1)];
+                const long bx = (gb & 1) ? long((uint64_t(qv[3]) << 32) | qv[2]) : long((uint64_t(qv[1]) << 32) | qv[0]);
+                const v4i zi = {0, 0, 0, 0};
+                const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
+                const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
+                const v4f sc = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, dw),
+                                                                     one_scale(x.d[t], gb, g == c), zf, 0, 0, 0);
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+                for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fma(double(sm[i]), double(sc[i]), acc[t][i]);
+                if constexpr (TYPE == T_Q4_1) {
+                    const v4f ms = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, mw),
+                                                                         one_scale(x.s[t], gb, g == c), zf, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dw[m][i] = *reinterpret_cast<const v4u *>(ld + m * DBUF + (4 * g + i) * GU + wave * GW);
-#pragma unroll
-    for (int j = 0; j < GW; ++j) {
-        const int blk = wave * GW + j;
-        long aop[NM];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const uint8_t * p = lq + (m * QH) * QBUF + r * ROW_LDS + blk * 16 + 4 * g;
-            const uint32_t lo = *reinterpret_cast<const uint32_t *>(p);
-            const uint32_t hi = QH == 2 ? *reinterpret_cast<const uint32_t *>(p + QBUF) : 0u;
-            aop[m] = a_operand<TYPE>(lo, hi);
-        }
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const v4u qv = x.q[t][j >> 1];
-            const long bx = (j & 1) ? long((uint64_t(qv[3]) << 32) | qv[2]) : long((uint64_t(qv[1]) << 32) | qv[0]);
-            const float dx = lane_of(x.d[t], j);
-            const v4i zero = {0, 0, 0, 0};
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop[m], bx, zero, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t sw = dw[m][i][j];
-                    const float sc = (TYPE == T_Q4_1 ? h2f(sw & 0xffffu) : __uint_as_float(sw)) * dx;
-                    double term = floor(double(sm[i]) * double(sc));
-                    if constexpr (TYPE == T_Q4_1)  // + floor(m * s_x * 2^40), the product of two fp16 values exact
-                        term += floor(double(h2f(sw >> 16) * lane_of(x.s[t], j)));
-                    if constexpr (EXACT) {
-                        if (m == 0) tot[t][i] += dint_to_i64(term);
-                        else totu[PAIR ? t : 0][i] += dint_to_i64(term);
-                    } else {
-                        acc[m][t][i] += term;
-                    }
+                    for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] + double(ms[i]);
                 }
             }
         }
     }
-    if constexpr (!EXACT) {
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                tot[t][i] += dint_to_i64(acc[0][t][i]);
-                if constexpr (PAIR) totu[t][i] += dint_to_i64(acc[PAIR ? 1 : 0][t][i]);
-            }
-    }
 }
 
-// The GW blocks of a round through one of two loops, chosen once per round (not per term, which kept the compiler
-// from scheduling the round as one block): the FP64-sum loop, or, where the bound says an FP64 partial could pass
-// 2^53 LSB, the one adding every term to the int64 totals.
-template <int TYPE, bool PAIR, int T>
-__device__ __forceinline__ void round_terms(const uint8_t * lq, const uint32_t * ld, int wave, int r, int g,
-                                            const XRound<T> & x, float wbound, long long (*tot)[4],
-                                            long long (*totu)[4]) {
-    if (round_needs_exact<T>(x, wbound)) round_terms_k<TYPE, PAIR, T, true>(lq, ld, wave, r, g, x, tot, totu);
-    else round_terms_k<TYPE, PAIR, T, false>(lq, ld, wave, r, g, x, tot, totu);
+__device__ __forceinline__ void add_total(long long * p, long long v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Workgroup b: rows 16b .. 16b + 15 (clamped loads past the last row, nothing stored for them), the whole K range in
-// rounds of GU blocks. Round rd + 2's weights are requested while round rd is summed (two rounds in flight) and
-// round rd + 1's are staged in LDS for the next; wave w sums blocks w * GW .. of each round, and wave 0 adds the
-// other waves' int64 totals (exact in any order), applies the epilog and stores token t's row at y + t * y_stride.
-// Loads past the last round repeat the last round (cache hits), so every load is unconditional and the waits stay
-// exact.
-// A group's workgroups are dealt to its members by tile: the member of tile b is the last whose first tile is <= b,
-// and its fields replace the first member's (the activation, columns and tokens are shared).
-template <int TYPE, bool PAIR, int T>
-__global__ __launch_bounds__(NT) void gemm_kernel(GemmArgs a0) {
-    constexpr int NM = PAIR ? 2 : 1, QH = TYPE == T_Q8_0 ? 2 : 1;
-    constexpr int QBUF = GT * ROW_LDS, DBUF = GT * GU;
-    __shared__ __align__(16) uint8_t lq[2][NM * QH * QBUF];
-    __shared__ __align__(16) uint32_t ld[2][NM * DBUF];
-    __shared__ long long red[NWAVES - 1][NM][T][4][WAVE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// One step with every term formed alone and added to the int64 totals: for steps whose terms could pass the
+// accumulators' 2^51 LSB (activation outliers in the thousands) or whose scales are not finite. Block by block in a
+// rolled loop that reads its activation operands again where they lie, so that it takes no registers from step_terms.
+// tot[t][i][lane]: row 4g + i, token r of token tile t.
+template <int TYPE, int T>
+__device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLds<TYPE> & l, int ns, int lane, int step,
+                                                 long long (*tot)[4][WAVE]) {
     const int r = lane & 15, g = lane >> 4;
-    GemmArgs a = a0;
-    int tile0 = 0;
-    float wbd = a0.wbound[0];  // the member's term bound
-    if (!PAIR) {
-        int mi = -1;
-        for (int i = 0; i < a0.n_more; ++i)
-            if (int(blockIdx.x) >= a0.more[i].tile0) mi = i;
-        if (mi >= 0) {
-            wbd = a0.wbound[mi + 1];
-            const GemmMore & o = a0.more[mi];
-            a.w = o.w;
-            a.y = o.y;
-            a.res = o.res;
-            a.rows = o.rows;
-            a.y_stride = o.y_stride;
-            a.res_stride = o.res_stride;
-            a.epi = o.epi;
-            tile0 = o.tile0;
-        }
-    }
-    const int r0 = (int(blockIdx.x) - tile0) * GT;
-    const int nb = a.cols / 32, nr = nb / GU;
-    const int lrow = min(r0 + (tid >> 4), a.rows - 1);
-    long long tot[T][4], totu[PAIR ? T : 1][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t)
+    const uint16_t * sc = reinterpret_cast<const uint16_t *>(l.s);
+    constexpr int SW = TYPE == T_Q4_1 ? 2 : 1;  // halves per scale
+#pragma unroll 1
+    for (int j = 0; j < GS; ++j) {
+        const int c = j >> 2, gb = j & 3, blk = step * GS + j;
+        const int at = 4 * (4 * r + ((gb + (r >> 2)) & 3)) + g;
+        const long aop = a_operand<TYPE>(l.q[0][c][at], TYPE == T_Q8_0 ? l.q[WLds<TYPE>::QH - 1][c][at] : 0u);
+        float dw[4], mw[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            tot[t][i] = 0;
-            totu[PAIR ? t : 0][i] = 0;
+            const int k = ((c * 16 + 4 * g + i) * 4 + gb) * SW;
+            dw[i] = h2f(sc[k]);
+            mw[i] = TYPE == T_Q4_1 ? h2f(sc[k + SW - 1]) : 0.0f;
         }
-    // rounds alternate between two LDS buffers and two register slots, so every load lands in a free slot
-    WRound<TYPE, PAIR> w0, wa, wb;
-    XRound<T> xa, xb;
-    load_wround<TYPE, PAIR>(a, nb, lrow, 0, w0);
-    load_wround<TYPE, PAIR>(a, nb, lrow, min(1, nr - 1), wb);
-    load_xround<TYPE, T>(a, nb, r, g, wave * GW, xa);
-    stage<TYPE, PAIR>(w0, lq[0], ld[0]);
-    __syncthreads();
-    int rd = 0;
-    for (; rd + 1 < nr; rd += 2) {
-        // round rd from buffer 0 and xa; round rd + 1's weights (wb) go to buffer 1
-        load_xround<TYPE, T>(a, nb, r, g, (rd + 1) * GU + wave * GW, xb);
-        load_wround<TYPE, PAIR>(a, nb, lrow, min(rd + 2, nr - 1), wa);
-        round_terms<TYPE, PAIR, T>(lq[0], ld[0], wave, r, g, xa, wbd, tot, totu);
-        stage<TYPE, PAIR>(wb, lq[1], ld[1]);
-        __syncthreads();
-        // round rd + 1 from buffer 1 and xb; round rd + 2's weights (wa) go to buffer 0
-        load_xround<TYPE, T>(a, nb, r, g, min(rd + 2, nr - 1) * GU + wave * GW, xa);
-        load_wround<TYPE, PAIR>(a, nb, lrow, min(rd + 3, nr - 1), wb);
-        round_terms<TYPE, PAIR, T>(lq[1], ld[1], wave, r, g, xb, wbd, tot, totu);
-        stage<TYPE, PAIR>(wa, lq[0], ld[0]);
-        __syncthreads();
-    }
-    if (rd < nr) round_terms<TYPE, PAIR, T>(lq[0], ld[0], wave, r, g, xa, wbd, tot, totu);  // an odd last round
-    if (wave > 0) {
 #pragma unroll
-        for (int t = 0; t < T; ++t)
+        for (int t = 0; t < T; ++t) {
+            const int tok = t * GT + r;
+            const long bx = *reinterpret_cast<const long *>(a.q + act_group(tok, g, ns, blk));
+            const v4i zi = {0, 0, 0, 0};
+            const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
+            const float d40 = h2f(a.d[act_scale(tok, ns, blk)]) * 1099511627776.0f;  // * 2^40, exact
+            const float s40 = TYPE == T_Q4_1 ? h2f(a.s[act_scale(tok, ns, blk)]) * 1099511627776.0f : 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                red[wave - 1][0][t][i][lane] = tot[t][i];
-                if constexpr (PAIR) red[wave - 1][PAIR ? 1 : 0][t][i][lane] = totu[t][i];
+                const double sum = TYPE == T_Q4_0 ? double(sm[i]) * 0.0625 : double(sm[i]);
+                long long v = dint_to_i64(floor(sum * double(dw[i] * d40)));
+                if constexpr (TYPE == T_Q4_1) v += dint_to_i64(floor(double(mw[i] * s40)));
+                add_total(&tot[t][i][lane], v);
             }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int tok = t * GT + r;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            long long sw = tot[t][i], su = 0;
-#pragma unroll
-            for (int k = 0; k < NWAVES - 1; ++k) sw += red[k][0][t][i][lane];
-            if constexpr (PAIR) {
-                su = totu[t][i];
-#pragma unroll
-                for (int k = 0; k < NWAVES - 1; ++k) su += red[k][PAIR ? 1 : 0][t][i][lane];
-            }
-            const int row = r0 + 4 * g + i;
-            if (row >= a.rows || tok >= a.n_tok) continue;
-            const float v = fixed_to_float(sw);
-            float out = v;
-            if (PAIR && a.epi == EPI_SWIGLU) {
-                out = (v / (1.0f + expf_(-v))) * fixed_to_float(su);  // gemvqc_ops.h:88-92
-            } else if (a.epi == EPI_ADD) {
-                out = v + a.res[size_t(tok) * a.res_stride + row];  // gemvqc16.cpp:282-301
-            } else if (a.epi == EPI_SILU) {
-                out = silu_(v);
-            }
-            a.y[size_t(tok) * a.y_stride + row] = out;
         }
     }
+}
+
+// A matrix whose bound is not known (the caller's own memory, never scanned): the largest |scale| of the step's
+// blocks over the wave, as the host's weight_bound forms it.
+template <int TYPE>
+__device__ __forceinline__ float step_bound(const WLds<TYPE> & l, int lane) {
+    uint32_t dm = 0, mm = 0;
+    constexpr int N = TYPE == T_Q4_1 ? 4 : 2;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const uint32_t v = l.s[N * lane + k];
+        dm = max(dm, TYPE == T_Q4_1 ? v & 0x7fffu : max(v & 0x7fffu, v >> 16 & 0x7fffu));
+        mm = max(mm, v >> 16 & 0x7fffu);
+    }
+#pragma unroll
+    for (int s = 1; s < WAVE; s <<= 1) {
+        dm = max(dm, uint32_t(__shfl_xor(int(dm), s, WAVE)));
+        mm = max(mm, uint32_t(__shfl_xor(int(mm), s, WAVE)));
+    }
+    constexpr float smax = TYPE == T_Q4_0 ? 32.0f * 8 * 127 : TYPE == T_Q4_1 ? 32.0f * 15 * 127 : 32.0f * 128 * 127;
+    return h2f(dm) * smax + (TYPE == T_Q4_1 ? h2f(mm) * (32.0f * 127) : 0.0f);
+}
+
+// FP64 round mode (MODE bits 3:2; 0 nearest even, 2 toward minus infinity). FP32 arithmetic keeps its own. As asm: the
+// compiler, which takes the default mode for granted, sets it back ahead of FP64 instructions after a builtin's switch.
+#define GQ_ROUND_F64(mode) asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), " #mode "\n\ts_nop 3" ::: "memory")
+
+// A workgroup takes the tiles of 16 rows b, b + gridDim.x, .. of all members, each against T tiles of 16 tokens; of a
+// SwiGLU pair the same rows of both matrices in turn. Its wave w sums the steps of 16 blocks w, w + 8, .. of every tile.
+// The launch is a stream of weight bytes, so the weights move past activations that stay: with up to 8 steps (4096
+// columns; HOLD = 1) or, for one token tile, 24 (12288 columns; HOLD = 3) a wave holds the activation operands of its
+// steps in registers for the whole launch, and requests the weights of its next step, or of the next tile's first,
+// before it sums the current one. Every load instruction reads whole 64-byte (activation: 1 KiB) runs; the operand
+// order comes from the wave's own part of LDS, without a workgroup barrier. The waves' sums meet in int64 totals in LDS
+// (exact in any order; two sets in turn, so one barrier a tile).
+// Measured (events, Q4_0, MI355X) against four waves sharing one staged tile, two rounds of 16 blocks in flight, seven
+// vector instructions a term: gate/up pair 2 x 12288 x 4096 17.1 us at 16 tokens and 27 at 32 (57 MB: 3.3 and 2.1 TB/s),
+// 12352 x 4096 group 13.2 and 20, 4096 x 12288 12.0 and 16.5, 4096 x 4096 5.8 and 8.1; the average launch of a layer 12.0
+// instead of 17.9 and 17.7 instead of 29.8. Loads whose neighbouring lanes lay in different rows (the operand order read
+// straight from memory) took 20.5 and 30.5: the address unit then works a line per lane.
+template <int TYPE, bool PAIR, int T, int HOLD>
+__global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(T == 1 && HOLD == 1 ? 4 : 2)))
+void gemm_kernel(GemmLaunch a) {
+    constexpr int NM = PAIR ? 2 : 1;
+    __shared__ WLds<TYPE> ws[GNW];
+    __shared__ long long tot[2][NM][T][4][WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lrow = lane >> 2, part = lane & 3;
+    const int nb = a.cols / 32, ns = nb / GS;
+    const int per_wave = (ns + GNW - 1) / GNW;
+    const float limit = 1125899906842624.0f / float(per_wave);  // 2^50 LSB over the wave's steps (half of what fits)
+    const bool mine = wave < ns;
+    WLds<TYPE> & wl = ws[wave];
+    int mi = member_of(a, blockIdx.x);
+    WStep<TYPE> wn;
+    XStep<TYPE, T> x[HOLD ? HOLD : 1];
+    const auto first_block = [&](int b, int mb) {  // of this lane's row of tile b
+        return size_t(min((b - a.m[mb].tile0) * GT + lrow, a.m[mb].rows - 1)) * nb;
+    };
+    if (mine) {
+        if constexpr (HOLD > 0) {
+#pragma unroll
+            for (int h = 0; h < HOLD; ++h)
+                if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, wave + GNW * h, x[h]);
+        }
+        load_wstep<TYPE>(a.m[mi].w, first_block(blockIdx.x, mi) + size_t(wave) * GS, part, wn);
+    }
+    for (int i = tid; i < 2 * NM * T * 4 * WAVE; i += GNT) (&tot[0][0][0][0][0])[i] = 0;
+    __syncthreads();
+    GQ_ROUND_F64(2);
+    double acc[T][4];
+#pragma unroll
+    for (int k = 0; k < T; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[k][i] = acc_base<TYPE>();
+            asm volatile("" : "+v"(acc[k][i]));  // the sums stay behind the mode switch
+        }
+    int set = 0;
+    for (int b = blockIdx.x; b < a.n_tiles; b += gridDim.x, set ^= 1) {
+        const int bn = b + int(gridDim.x);
+        const int next = bn < a.n_tiles ? member_of(a, bn) : mi;
+        if (mine) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                const WeightView & w = PAIR && m ? a.w2 : a.m[mi].w;
+                const auto one = [&](int step, XStep<TYPE, T> & xs) {
+                    if constexpr (HOLD == 0) load_xstep<TYPE, T>(a, ns, lane, step, xs);
+                    stage<TYPE>(wn, lane, wl);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    if (step + GNW < ns) load_wstep<TYPE>(w, first_block(b, mi) + size_t(step + GNW) * GS, part, wn);
+                    else if (m + 1 < NM) load_wstep<TYPE>(a.w2, first_block(b, mi) + size_t(wave) * GS, part, wn);
+                    else if (bn < a.n_tiles) load_wstep<TYPE>(a.m[next].w, first_block(bn, next) + size_t(wave) * GS, part, wn);
+                    // (opaque: the blocks' scale operands are formed where they are used, not held for the launch)
+#pragma unroll
+                    for (int k = 0; k < T; ++k) {
+                        asm volatile("" : "+v"(xs.d[k]));
+                        if constexpr (TYPE == T_Q4_1) asm volatile("" : "+v"(xs.s[k]));
+                    }
+                    const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
+                    if (__builtin_amdgcn_ballot_w64(!(wb * xs.bound < limit)) != 0)
+                        step_terms_exact<TYPE, T>(a, wl, ns, lane, step, tot[set][m]);
+                    else step_terms<TYPE, T>(wl, xs, lane, acc);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                };
+                if constexpr (HOLD > 0) {
+#pragma unroll
+                    for (int h = 0; h < HOLD; ++h)
+                        if (wave + GNW * h < ns) one(wave + GNW * h, x[h]);
+                } else {
+                    for (int step = wave; step < ns; step += GNW) one(step, x[0]);
+                }
+#pragma unroll
+                for (int k = 0; k < T; ++k)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        add_total(&tot[set][m][k][i][lane],
+                                  __builtin_bit_cast(long long, acc[k][i]) - __builtin_bit_cast(long long, acc_base<TYPE>()));
+                        acc[k][i] = acc_base<TYPE>();
+                    }
+            }
+        }
+        __syncthreads();
+        // thread e: row e % 16 of token e / 16 (consecutive rows are stored together); the total is cleared for the
+        // tile after next, whose sums start behind the next barrier
+        if (tid < T * GT * GT) {
+            const int tok = tid >> 4, rr = tid & 15, src = (rr >> 2) * 16 + (tok & 15);
+            long long sum[NM];
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                long long * p = &tot[set][m][tok >> 4][rr & 3][src];
+                sum[m] = *p;
+                *p = 0;
+            }
+            const GemmMember & t = a.m[mi];
+            const int row = (b - t.tile0) * GT + rr;
+            if (row < t.rows && tok < a.n_tok) {
+                const float v = fixed_to_float(sum[0]);
+                float out = v;
+                if (PAIR) {
+                    out = (v / (1.0f + expf_(-v))) * fixed_to_float(sum[NM - 1]);  // gemvqc_ops.h:88-92
+                } else if (t.epi == EPI_ADD) {
+                    out = v + t.res[size_t(tok) * t.res_stride + row];  // gemvqc16.cpp:282-301
+                } else if (t.epi == EPI_SILU) {
+                    out = silu_(v);
+                }
+                t.y[size_t(tok) * t.y_stride + row] = out;
+            }
+        }
+        mi = next;
+    }
+#pragma unroll
+    for (int k = 0; k < T; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[k][i]));
+    GQ_ROUND_F64(0);
+}
+
+template <int TYPE, bool PAIR, int T, int HOLD>
+void launch_one(const GemmLaunch & a, hipStream_t st) {
+    // as many workgroups as the 256 CUs hold at once (two of 8 waves each where the registers allow)
+    const int grid = std::min(a.n_tiles, T == 1 && HOLD == 1 ? 512 : 256);
+    GQ_LAUNCH((gemm_kernel<TYPE, PAIR, T, HOLD>), dim3(grid), dim3(GNT), 0, st, a);
 }
 
 template <int TYPE, bool PAIR>
-hipError_t launch_tiles(const GemmArgs & a, hipStream_t st) {
-    int tiles = (a.rows + GT - 1) / GT;
-    for (int i = 0; i < a.n_more; ++i) {  // members follow each other, every one at least a tile
-        if (a.more[i].tile0 != tiles || a.more[i].rows < 1) return hipErrorInvalidValue;
-        tiles += (a.more[i].rows + GT - 1) / GT;
+hipError_t launch_tiles(const GemmArgs & g, hipStream_t st) {
+    GemmLaunch a{g.q, g.d, g.s, g.bound, g.cols, g.n_tok, 1 + g.n_more, 0, g.w2, {}};
+    for (int i = 0; i <= g.n_more; ++i) {  // members follow each other, every one at least a tile
+        const GemmMore f{g.w, g.y, g.res, g.rows, g.y_stride, g.res_stride, g.epi};
+        const GemmMore & o = i ? g.more[i - 1] : f;
+        if (o.rows < 1) return hipErrorInvalidValue;
+        a.m[i] = GemmMember{o.w, o.y, o.res, o.rows, o.y_stride, o.res_stride, o.epi, a.n_tiles, g.wbound[i]};
+        a.n_tiles += (o.rows + GT - 1) / GT;
     }
-    const dim3 grid(tiles);
-    if (a.n_tok <= GT) GQ_LAUNCH((gemm_kernel<TYPE, PAIR, 1>), grid, dim3(NT), 0, st, a);
-    else GQ_LAUNCH((gemm_kernel<TYPE, PAIR, 2>), grid, dim3(NT), 0, st, a);
+    const int steps = a.cols / (32 * GS);
+    if (a.n_tok <= GT) {
+        if (steps <= GNW) launch_one<TYPE, PAIR, 1, 1>(a, st);
+        else if (steps <= 3 * GNW) launch_one<TYPE, PAIR, 1, 3>(a, st);
+        else launch_one<TYPE, PAIR, 1, 0>(a, st);
+    } else if (steps <= GNW) {
+        launch_one<TYPE, PAIR, 2, 1>(a, st);
+    } else {
+        launch_one<TYPE, PAIR, 2, 0>(a, st);
+    }
     return hipGetLastError();
 }
 

@@ -226,9 +226,10 @@ struct NextTokenArgs {
 struct GemmQuantArgs {
     const float * x;       // token t's row at x + t * x_stride
     const float * norm_w;  // per-token RMS norm folded into the quantization: its weight (NULL: none)
-    int8_t * q;            // [n_pad][cols]
-    float * d40;           // [n_pad][cols / 32]
-    float * s40;           // [n_pad][cols / 32]: the Q8_1 s = fp16(sum of the block's quants * d), times 2^40
+    int8_t * q;            // [n_pad * cols]
+    uint16_t * d;          // [n_pad * cols / 32]: the blocks' fp16 scales (orders of all: gq_gemm.hip)
+    uint16_t * s;          // [n_pad * cols / 32]: the Q8_1 s = fp16(sum of the block's quants * d)
+    float * bound;         // [n_pad * cols / 512]: per 16 blocks, the sum of d * 2^40 * (sum of |quants|) / (32 * 127)
     int n_tok, n_pad, cols, x_stride;
     int norm, norm_l2;
     float eps;
@@ -241,15 +242,15 @@ struct GemmMore {  // a further member of a GEMM group: its own matrix, output r
     float * y;
     const float * res;
     int rows, y_stride, res_stride, epi;
-    int tile0;  // its first 16-row tile in the group's grid
 };
 
 struct GemmArgs {
     WeightView w;       // matrix (g of a SwiGLU pair)
     WeightView w2;      // u of a SwiGLU pair
     const int8_t * q;   // the quantized activation (GemmQuantArgs)
-    const float * d40;
-    const float * s40;  // Q4_1 weights: the activation blocks' Q8_1 s * 2^40
+    const uint16_t * d;
+    const uint16_t * s;  // Q4_1 weights: the activation blocks' Q8_1 s
+    const float * bound;
     float * y;          // token t, row r at y[t * y_stride + r]
     const float * res;  // ADD: res[t * res_stride + r]
     int rows, cols, n_tok, y_stride, res_stride;

@@ -118,8 +118,9 @@ struct gemvq_ctx {
     uint32_t * gdn_fault = nullptr;  // host word the fused launch sets when a wait for its heads ran out of polls
     unsigned xch_polls = 0;          // that wait's bound in polls (set at creation)
     int8_t * gemm_q = nullptr;    // a batched GEMV's quantized activation rows (GEMM_MAX_TOK x GEMV_MAXK)
-    float * gemm_d = nullptr;     // and their block scales
-    float * gemm_s = nullptr;     // and their Q8_1 block sums (for Q4_1 weights)
+    uint16_t * gemm_d = nullptr;  // and their block scales
+    uint16_t * gemm_s = nullptr;  // and their Q8_1 block sums (for Q4_1 weights)
+    float * gemm_b = nullptr;     // and their parts of the term bounds
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
     int arith = GEMVQ_ARITH_CANONICAL;  // the arithmetic lists are compiled in (gemvq_set_arith)
     int last_launches = 0;
@@ -982,8 +983,9 @@ struct Compiler {
         q.x = A(k[6]);
         q.norm_w = normw ? A(k2[5]) : nullptr;
         q.q = c->gemm_q;
-        q.d40 = c->gemm_d;
-        q.s40 = c->gemm_s;
+        q.d = c->gemm_d;
+        q.s = c->gemm_s;
+        q.bound = c->gemm_b;
         q.n_tok = int(ntok);
         q.n_pad = int((ntok + 15) / 16 * 16);
         q.cols = int(cols);
@@ -992,8 +994,9 @@ struct Compiler {
         q.norm_l2 = (nflags & GEMVQ_NORM_L2) ? 1 : 0;
         q.eps = bits_f(k2[6]);
         g.q = c->gemm_q;
-        g.d40 = c->gemm_d;
-        g.s40 = c->gemm_s;
+        g.d = c->gemm_d;
+        g.s = c->gemm_s;
+        g.bound = c->gemm_b;
         const bool same = lastq.on && lastq.x_off == k[6] && lastq.x_len == x_len && lastq.q.n_tok == q.n_tok &&
                           lastq.q.cols == q.cols && lastq.q.x_stride == q.x_stride && lastq.q.norm == q.norm &&
                           lastq.q.norm_l2 == q.norm_l2 && lastq.q.norm_w == q.norm_w && lastq.q.eps == q.eps;
@@ -1112,7 +1115,6 @@ struct Compiler {
         const R ny = span(g.y, g.y_stride, g.rows);
         const bool nres = g.epi == EPI_ADD;
         const R nr = nres ? span(g.res, g.res_stride, g.rows) : R{0, 0};
-        int tiles = 0;
         for (int m = 0; m <= p->a.n_more; ++m) {
             const bool first = m == 0;
             const GemmMore * o = first ? nullptr : &p->a.more[m - 1];
@@ -1121,10 +1123,9 @@ struct Compiler {
             const R res = epi == EPI_ADD ? (first ? span(p->a.res, p->a.res_stride, p->a.rows) : span(o->res, o->res_stride, o->rows))
                                          : R{0, 0};
             if (meet(ny, y) || (epi == EPI_ADD && meet(ny, res)) || (nres && meet(nr, y))) return false;
-            tiles += ((first ? p->a.rows : o->rows) + 15) / 16;
         }
         p->a.wbound[p->a.n_more + 1] = g.wbound[0];
-        p->a.more[p->a.n_more++] = GemmMore{g.w, g.y, g.res, g.rows, g.y_stride, g.res_stride, g.epi, tiles};
+        p->a.more[p->a.n_more++] = GemmMore{g.w, g.y, g.res, g.rows, g.y_stride, g.res_stride, g.epi};
         spans.back().second = i + used - spans.back().first;
         return true;
     }
@@ -1450,8 +1451,9 @@ gemvq_ctx * gemvq_ctx_create(int device, size_t act_floats, size_t weight_bytes,
     if (e == hipSuccess) e = hipHostMalloc(&c->gdn_fault, sizeof(uint32_t), hipHostMallocCoherent);
     if (e == hipSuccess) *c->gdn_fault = 0;
     if (e == hipSuccess) e = hipMalloc(&c->gemm_q, size_t(GEMM_MAX_TOK) * GEMV_MAXK);
-    if (e == hipSuccess) e = hipMalloc(&c->gemm_d, size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 32) * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&c->gemm_s, size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 32) * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&c->gemm_d, size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 32) * sizeof(uint16_t));
+    if (e == hipSuccess) e = hipMalloc(&c->gemm_s, size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 32) * sizeof(uint16_t));
+    if (e == hipSuccess) e = hipMalloc(&c->gemm_b, size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 512) * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&c->ref_x, size_t(GEMM_MAX_TOK + 1) * GEMV_MAXK * sizeof(float));
     if (e == hipSuccess && state_rows) e = hipMemset(c->state, 0, state_rows * 128 * sizeof(float));
     if (e != hipSuccess) {
@@ -1491,6 +1493,7 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->gemm_q);
     hipFree(c->gemm_d);
     hipFree(c->gemm_s);
+    hipFree(c->gemm_b);
     hipFree(c->ref_x);
     hipFree(c->dbg);
     if (c->stream) hipStreamDestroy(c->stream);

@@ -16,8 +16,8 @@ namespace {
 
 constexpr size_t Q_BYTES = size_t(GEMM_MAX_TOK) * GEMV_MAXK;          // quants of up to 32 token rows
 constexpr size_t BLOCKS = size_t(GEMM_MAX_TOK) * (GEMV_MAXK / 32);    // their per-block scale words
-constexpr size_t SCRATCH_BYTES = Q_BYTES + 2 * BLOCKS * sizeof(float);  // 640 KiB
-static_assert(SCRATCH_BYTES == GEMVQ_STATIC_SCRATCH_BYTES, "scratch size in the header");
+constexpr size_t SCRATCH_BYTES = GEMVQ_STATIC_SCRATCH_BYTES;          // 640 KiB
+static_assert(Q_BYTES + 2 * BLOCKS * sizeof(uint16_t) + BLOCKS / 16 * sizeof(float) <= SCRATCH_BYTES, "scratch size in the header");
 
 __device__ __align__(256) uint8_t scratch[SCRATCH_BYTES];
 
@@ -60,8 +60,9 @@ extern "C" int gemvq_gemm_static(int type, int rows, int cols, const void * w, c
     q.x = x;
     q.norm_w = nullptr;
     q.q = reinterpret_cast<int8_t *>(base);
-    q.d40 = reinterpret_cast<float *>(base + Q_BYTES);
-    q.s40 = q.d40 + BLOCKS;
+    q.d = reinterpret_cast<uint16_t *>(base + Q_BYTES);
+    q.s = q.d + BLOCKS;
+    q.bound = reinterpret_cast<float *>(q.s + BLOCKS);
     q.n_tok = n_tok;
     q.n_pad = (n_tok + 15) / 16 * 16;  // the quantizer writes the padding rows too: nothing needs clearing
     q.cols = cols;
@@ -69,15 +70,16 @@ extern "C" int gemvq_gemm_static(int type, int rows, int cols, const void * w, c
     GemmArgs g{};
     g.w = weight_view(static_cast<const uint8_t *>(w), type, rows, cols);
     g.q = q.q;
-    g.d40 = q.d40;
-    g.s40 = q.s40;
+    g.d = q.d;
+    g.s = q.s;
+    g.bound = q.bound;
     g.y = y;
     g.rows = rows;
     g.cols = cols;
     g.n_tok = n_tok;
     g.y_stride = y_stride;
     g.epi = EPI_PLAIN;
-    g.wbound[0] = INFINITY;  // the caller's matrix was never scanned: every round's terms are summed in int64
+    g.wbound[0] = INFINITY;  // the caller's matrix was never scanned: each step's bound is formed from its scales
     const hipStream_t s = static_cast<hipStream_t>(stream);
     e = launch_gemm_quant(q, s);
     if (e == hipSuccess) e = launch_gemm(g, type, s);

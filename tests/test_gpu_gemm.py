@@ -352,3 +352,25 @@ def test_q4_1_sum_on_fp16_tie(gq, orc, ctx):
         assert_bits(y[t], want, f"GEMM token {t}")
         assert ctx.run(gq.gemv(3, rows, cols, off, t * cols, 16384)) == 0, ctx.error()
         assert_bits(ctx.read(16384, rows), want, f"GEMV token {t}")
+
+
+@pytest.mark.parametrize("fmt", [2, 3, 8])
+@pytest.mark.parametrize("rows,cols,ntok", [(1, 512, 16), (8209, 512, 17), (17, 12288, 16), (40, 12800, 5),
+                                            (40, 16384, 32), (16400, 1024, 7)])
+def test_gemm_tiles_and_held_steps(gq, orc, ctx, fmt, rows, cols, ntok):
+    """The edges of the weight pass: one row and one step; more tiles than workgroups (513 and 1025 tiles, a partial
+    last one); activations held for the launch (up to 4096 columns, and 12288 for one token tile) and read again for
+    every tile (wider, and two token tiles past 4096 columns); waves without a step. Token rows bit for bit."""
+    w = gq.matrix(fmt, min(rows, 512), cols, 5, 70 + fmt, std=0.02)
+    w = np.resize(w, rows * gq.row_bytes(fmt, cols))
+    off = ctx.upload(fmt, rows, cols, w)
+    x = gq.normal(5, 71, ntok * cols)
+    ys = up16(rows)
+    X, Y = 0, ntok * cols
+    ctx.write(X, x)
+    print(f"[gemm] held steps fmt {fmt} rows {rows} cols {cols} tokens {ntok}", flush=True)
+    assert ctx.run(gq.gemm(fmt, rows, cols, off, X, Y, ntok, cols, ys)) == 0, ctx.error()
+    y = ctx.read(Y, ntok * ys).reshape(ntok, ys)[:, :rows]
+    for t in sorted({0, ntok // 2, ntok - 1}):
+        want = orc.fx_gemv(fmt, w[:min(rows, 512) * gq.row_bytes(fmt, cols)], x[t * cols:(t + 1) * cols], min(rows, 512), cols)
+        assert_bits(y[t], np.resize(want, rows), f"token {t}")
