@@ -9,8 +9,8 @@
 //     and Q4_1 pack exactly those as the low and high nibbles of quant bytes 4g..4g+3, Q8_0 holds them as bytes
 //     4g..4g+3 of its two 16-byte halves, and the activation quantizer stores them in that order. Q4_0 enters as
 //     16 * (q - 8), the nibble moved to the top of its byte (three instructions a block instead of nine for q - 8);
-//   - one v_mfma_f32_16x16x16_f16 for the scale products d_w * d_x of the block: A holds the scales of 16 blocks as
-//     they lie in memory, B the token's scale of this block at the block's place and zeros elsewhere, so every
+//   - one v_mfma_f32_16x16x16_f16 for the scale products d_w * d_x of the block: B holds the tokens' scales of 16
+//     blocks as they lie in memory, A the row's scale of this block at the block's place and zeros elsewhere, so every
 //     product comes out alone, exact in FP32, already where the block sums' rows and tokens are.
 // The vector ALUs then do three FP64 instructions a term: both values converted, and one fused multiply-add into an
 // accumulator near 1.5 * 2^52 LSB in the round-toward-minus-infinity mode. There the accumulator's last place is the
@@ -198,7 +198,7 @@ __device__ __forceinline__ int member_of(const GemmLaunch & a, int b) {
     return mi;
 }
 
-// A lane's activation operands of one step: group g of token r's 16 blocks, and (lane group g) the scales of the
+// A lane's activation operands of one step (token tiles tile, tile + 1, ..): group g of token r's 16 blocks, and (lane group g) the scales of the
 // token's blocks 4g .. 4g + 3; the step's part of the term bound.
 template <int TYPE, int T>
 struct XStep {
@@ -209,11 +209,11 @@ struct XStep {
 };
 
 template <int TYPE, int T>
-__device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lane, int step, XStep<TYPE, T> & o) {
+__device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lane, int tile, int step, XStep<TYPE, T> & o) {
     float bd[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const size_t at = size_t(t) * ns + step;
+        const size_t at = size_t(tile + t) * ns + step;
         const v4u * p = reinterpret_cast<const v4u *>(a.q + at * 8192) + lane;
 #pragma unroll
         for (int k = 0; k < GS / 2; ++k) o.q[t][k] = p[k * WAVE];
@@ -223,11 +223,11 @@ __device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lan
     }
     o.bound = 0.0f;
 #pragma unroll
-    for (int t = 0; t < T; ++t) o.bound = bd[t] <= o.bound ? o.bound : bd[t];  // a NaN stays
-    if constexpr (T == 2) o.bound = bd[0] != bd[0] ? bd[0] : o.bound;
+    for (int t = 0; t < T; ++t) o.bound = bd[t] <= o.bound || o.bound != o.bound ? o.bound : bd[t];  // a NaN stays
 }
 
-// The FP16 operand of one block: the token's scale at the block's place c of lane group gb, zeros elsewhere.
+// The FP16 operand of one block: the row's scale at the block's place c of the lane group that it is mine of, zeros
+// elsewhere.
 __device__ __forceinline__ v4h one_scale(const v2u & d, int c, bool mine) {
     const uint32_t v = mine ? (c & 1 ? d[c >> 1] & 0xffff0000u : d[c >> 1] & 0xffffu) : 0u;
     const v2u o = c < 2 ? v2u{v, 0u} : v2u{0u, v};
@@ -258,6 +258,7 @@ __device__ __forceinline__ void step_terms(const WLds<TYPE> & l, const XStep<TYP
             // block 4c + gb: its scales are lane group c's, at place gb
             const int at = 4 * (4 * r + ((gb + (r >> 2)) & 3)) + g;
             const long aop = a_operand<TYPE>(l.q[0][c][at], TYPE == T_Q8_0 ? l.q[WLds<TYPE>::QH - 1][c][at] : 0u);
+            const v4h dw1 = one_scale(dw, gb, g == c), mw1 = one_scale(TYPE == T_Q4_1 ? mw : dw, gb, g == c);
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 const v4u qv = x.q[t][2 * c + (gb >> 1)];
@@ -265,13 +266,11 @@ __device__ __forceinline__ void step_terms(const WLds<TYPE> & l, const XStep<TYP
                 const v4i zi = {0, 0, 0, 0};
                 const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
                 const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
-                const v4f sc = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, dw),
-                                                                     one_scale(x.d[t], gb, g == c), zf, 0, 0, 0);
+                const v4f sc = __builtin_amdgcn_mfma_f32_16x16x16f16(dw1, __builtin_bit_cast(v4h, x.d[t]), zf, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[t][i] = __builtin_fma(double(sm[i]), double(sc[i]), acc[t][i]);
                 if constexpr (TYPE == T_Q4_1) {
-                    const v4f ms = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, mw),
-                                                                         one_scale(x.s[t], gb, g == c), zf, 0, 0, 0);
+                    const v4f ms = __builtin_amdgcn_mfma_f32_16x16x16f16(mw1, __builtin_bit_cast(v4h, x.s[t]), zf, 0, 0, 0);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] + double(ms[i]);
                 }
@@ -289,7 +288,7 @@ __device__ __forceinline__ void add_total(long long * p, long long v) {
 // rolled loop that reads its activation operands again where they lie, so that it takes no registers from step_terms.
 // tot[t][i][lane]: row 4g + i, token r of token tile t.
 template <int TYPE, int T>
-__device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLds<TYPE> & l, int ns, int lane, int step,
+__device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLds<TYPE> & l, int ns, int lane, int tile, int step,
                                                  long long (*tot)[4][WAVE]) {
     const int r = lane & 15, g = lane >> 4;
     const uint16_t * sc = reinterpret_cast<const uint16_t *>(l.s);
@@ -308,7 +307,7 @@ __device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLd
         }
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            const int tok = t * GT + r;
+            const int tok = (tile + t) * GT + r;
             const long bx = *reinterpret_cast<const long *>(a.q + act_group(tok, g, ns, blk));
             const v4i zi = {0, 0, 0, 0};
             const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
@@ -386,7 +385,7 @@ void gemm_kernel(GemmLaunch a) {
         if constexpr (HOLD > 0) {
 #pragma unroll
             for (int h = 0; h < HOLD; ++h)
-                if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, wave + GNW * h, x[h]);
+                if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, 0, wave + GNW * h, x[h]);
         }
         load_wstep<TYPE>(a.m[mi].w, first_block(blockIdx.x, mi) + size_t(wave) * GS, part, wn);
     }
@@ -410,7 +409,7 @@ void gemm_kernel(GemmLaunch a) {
             for (int m = 0; m < NM; ++m) {
                 const WeightView & w = PAIR && m ? a.w2 : a.m[mi].w;
                 const auto one = [&](int step, XStep<TYPE, T> & xs) {
-                    if constexpr (HOLD == 0) load_xstep<TYPE, T>(a, ns, lane, step, xs);
+                    if constexpr (HOLD == 0) load_xstep<TYPE, T>(a, ns, lane, 0, step, xs);
                     stage<TYPE>(wn, lane, wl);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -418,15 +417,9 @@ void gemm_kernel(GemmLaunch a) {
                     if (step + GNW < ns) load_wstep<TYPE>(w, first_block(b, mi) + size_t(step + GNW) * GS, part, wn);
                     else if (m + 1 < NM) load_wstep<TYPE>(a.w2, first_block(b, mi) + size_t(wave) * GS, part, wn);
                     else if (bn < a.n_tiles) load_wstep<TYPE>(a.m[next].w, first_block(bn, next) + size_t(wave) * GS, part, wn);
-                    // (opaque: the blocks' scale operands are formed where they are used, not held for the launch)
-#pragma unroll
-                    for (int k = 0; k < T; ++k) {
-                        asm volatile("" : "+v"(xs.d[k]));
-                        if constexpr (TYPE == T_Q4_1) asm volatile("" : "+v"(xs.s[k]));
-                    }
                     const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
                     if (__builtin_amdgcn_ballot_w64(!(wb * xs.bound < limit)) != 0)
-                        step_terms_exact<TYPE, T>(a, wl, ns, lane, step, tot[set][m]);
+                        step_terms_exact<TYPE, T>(a, wl, ns, lane, 0, step, tot[set][m]);
                     else step_terms<TYPE, T>(wl, xs, lane, acc);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -484,6 +477,134 @@ void gemm_kernel(GemmLaunch a) {
     GQ_ROUND_F64(0);
 }
 
+// ---- more than 32 tokens: bound by the vector instructions of the terms, no longer by the weight bytes ----
+// The (token group of 64, tile of 16 rows) pairs of the launch, in this order, are dealt to the workgroups in equal
+// contiguous runs, each summed in batches of up to WTB tile products whose int64 totals lie in LDS. A batch goes through the
+// columns in chunks of 4096 (128 blocks): wave w holds the activation operands of the chunk's blocks 16 w .. 16 w + 15 for
+// all 64 tokens in registers while the batch's weights stream past, four token tiles to every weight operand formed, and
+// adds its part of each tile to the totals. (Held operands: read per tile instead, 64 tokens' would need four times the
+// weights' bandwidth from L2.)
+// Measured (trace, Q4_0, 511 tokens, MI355X): gate/up pair 2 x 12288 x 4096 290 us, 12352 x 4096 group 140 us, 4096 x 12288
+// 140-190 us; a layer's launches 0.66 ms, where 16 chunks of 32 tokens took 1.1 ms. At 16.4 cycles per 64 terms (the
+// matrix product, two conversions and the multiply-add in a loop of their own) the pair's terms alone are 172 us.
+constexpr int WT = 4;   // token tiles
+constexpr int WTB = 8;  // tile products per batch (64 KiB of totals)
+
+template <int TYPE, bool PAIR>
+__global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(GemmLaunch a, int n_tg) {
+    constexpr int NM = PAIR ? 2 : 1, TB = WTB / NM;  // row tiles per batch
+    __shared__ WLds<TYPE> ws[GNW];
+    __shared__ long long tot[WTB][WT][4][WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lrow = lane >> 2, part = lane & 3;
+    const int nb = a.cols / 32, ns = nb / GS, chunks = (ns + GNW - 1) / GNW;
+    WLds<TYPE> & wl = ws[wave];
+    const int total = n_tg * a.n_tiles;
+    const int begin = int((long long)(blockIdx.x) * total / gridDim.x), end = int((long long)(blockIdx.x + 1) * total / gridDim.x);
+    const auto first_block = [&](int b, int mb) {  // of this lane's row of tile b
+        return size_t(min((b - a.m[mb].tile0) * GT + lrow, a.m[mb].rows - 1)) * nb;
+    };
+    WStep<TYPE> wn;
+    XStep<TYPE, WT> x;
+    int held = -1;  // the token group whose only chunk x holds
+    if (begin < end && wave < ns) {
+        const int b = begin % a.n_tiles, mi = member_of(a, b);
+        load_wstep<TYPE>(a.m[mi].w, first_block(b, mi) + size_t(wave) * GS, part, wn);
+    }
+    for (int at = begin; at < end;) {
+        const int tg = at / a.n_tiles, t0 = at % a.n_tiles, n = min(min(TB, end - at), a.n_tiles - t0);
+        for (int i = tid; i < n * NM * WT * 4 * WAVE; i += GNT) (&tot[0][0][0][0])[i] = 0;
+        __syncthreads();
+        GQ_ROUND_F64(2);
+        for (int kc = 0; kc < chunks; ++kc) {
+            const int step = kc * GNW + wave;
+            if (step >= ns) break;
+            if (chunks > 1 || held != tg) load_xstep<TYPE, WT>(a, ns, lane, tg * WT, step, x);
+            held = tg;
+            for (int j = 0; j < n; ++j) {
+                const int mi = member_of(a, t0 + j);
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    stage<TYPE>(wn, lane, wl);
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    // the next product's weights: u of the pair, the next tile, the batch's first of the next chunk, or
+                    // the next batch's first
+                    if (m + 1 < NM) {
+                        load_wstep<TYPE>(a.w2, first_block(t0 + j, mi) + size_t(step) * GS, part, wn);
+                    } else {
+                        int b = t0 + j + 1, st = step;
+                        bool more = true;
+                        if (j + 1 == n) {
+                            if (step + GNW < ns) {
+                                b = t0;
+                                st = step + GNW;
+                            } else {
+                                more = at + n < end;
+                                b = (at + n) % a.n_tiles;
+                                st = wave;
+                            }
+                        }
+                        if (more) {
+                            const int mb = member_of(a, b);
+                            load_wstep<TYPE>(a.m[mb].w, first_block(b, mb) + size_t(st) * GS, part, wn);
+                        }
+                    }
+                    const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
+                    long long (*tt)[4][WAVE] = tot[j * NM + m];
+                    if (__builtin_amdgcn_ballot_w64(!(wb * x.bound < 1125899906842624.0f)) != 0) {  // 2^50 LSB
+                        step_terms_exact<TYPE, WT>(a, wl, ns, lane, tg * WT, step, tt);
+                    } else {
+                        double acc[WT][4];
+#pragma unroll
+                        for (int k = 0; k < WT; ++k)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                acc[k][i] = acc_base<TYPE>();
+                                asm volatile("" : "+v"(acc[k][i]));  // the sums stay between the mode switches
+                            }
+                        step_terms<TYPE, WT>(wl, x, lane, acc);
+#pragma unroll
+                        for (int k = 0; k < WT; ++k)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                asm volatile("" : "+v"(acc[k][i]));
+                                add_total(&tt[k][i][lane], __builtin_bit_cast(long long, acc[k][i]) -
+                                                               __builtin_bit_cast(long long, acc_base<TYPE>()));
+                            }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+        }
+        GQ_ROUND_F64(0);
+        __syncthreads();
+        // element e: row e % (16 TB) of the batch, token e / (16 TB) of the group: consecutive rows are stored together
+        for (int e = tid; e < TB * GT * WT * GT; e += GNT) {
+            const int q = e % (TB * GT), tk = e / (TB * GT), j = q / GT, rr = q % GT;
+            const int tok = tg * WT * GT + tk, src = (rr >> 2) * 16 + (tk & 15);
+            if (j >= n || tok >= a.n_tok) continue;
+            const GemmMember & t = a.m[member_of(a, t0 + j)];
+            const int row = (t0 + j - t.tile0) * GT + rr;
+            if (row >= t.rows) continue;
+            const float v = fixed_to_float(tot[j * NM][tk >> 4][rr & 3][src]);
+            float out = v;
+            if (PAIR) {
+                out = (v / (1.0f + expf_(-v))) * fixed_to_float(tot[j * NM + NM - 1][tk >> 4][rr & 3][src]);
+            } else if (t.epi == EPI_ADD) {
+                out = v + t.res[size_t(tok) * t.res_stride + row];
+            } else if (t.epi == EPI_SILU) {
+                out = silu_(v);
+            }
+            t.y[size_t(tok) * t.y_stride + row] = out;
+        }
+        __syncthreads();
+        at += n;
+    }
+}
+
 template <int TYPE, bool PAIR, int T, int HOLD>
 void launch_one(const GemmLaunch & a, hipStream_t st) {
     // as many workgroups as the 256 CUs hold at once (two of 8 waves each where the registers allow)
@@ -502,7 +623,10 @@ hipError_t launch_tiles(const GemmArgs & g, hipStream_t st) {
         a.n_tiles += (o.rows + GT - 1) / GT;
     }
     const int steps = a.cols / (32 * GS);
-    if (a.n_tok <= GT) {
+    if (a.n_tok > 2 * GT) {
+        const int n_tg = (a.n_tok + WT * GT - 1) / (WT * GT);
+        GQ_LAUNCH((gemm_wide_kernel<TYPE, PAIR>), dim3(std::min(n_tg * a.n_tiles, 256)), dim3(GNT), 0, st, a, n_tg);
+    } else if (a.n_tok <= GT) {
         if (steps <= GNW) launch_one<TYPE, PAIR, 1, 1>(a, st);
         else if (steps <= 3 * GNW) launch_one<TYPE, PAIR, 1, 3>(a, st);
         else launch_one<TYPE, PAIR, 1, 0>(a, st);
@@ -522,7 +646,7 @@ hipError_t launch_type(const GemmArgs & a, hipStream_t st) {
 }  // namespace
 
 hipError_t launch_gemm_quant(const GemmQuantArgs & a, hipStream_t s) {
-    if (a.n_tok < 1 || a.n_pad < a.n_tok || a.n_pad % GT || a.n_pad > GEMM_MAX_TOK || a.cols % 512 ||
+    if (a.n_tok < 1 || a.n_pad != gemm_pad(a.n_tok) || a.n_tok > GEMM_WIDE_TOK || a.cols % 512 ||
         a.cols > GEMV_MAXK || a.x_stride < a.cols || a.x_stride % 16)
         return hipErrorInvalidValue;
     GQ_LAUNCH(gemm_quant_kernel, dim3(a.n_pad), dim3(NT), 0, s, a);
@@ -530,8 +654,8 @@ hipError_t launch_gemm_quant(const GemmQuantArgs & a, hipStream_t s) {
 }
 
 hipError_t launch_gemm(const GemmArgs & a, int type, hipStream_t s) {
-    // shapes the kernels assume: whole rounds of GU blocks per wave, at most two token tiles
-    if (a.rows < 1 || a.n_tok < 1 || a.n_tok > GEMM_MAX_TOK || a.cols % 512 || a.cols > GEMV_MAXK ||
+    // shapes the kernels assume: whole steps of GS blocks
+    if (a.rows < 1 || a.n_tok < 1 || a.n_tok > GEMM_WIDE_TOK || a.cols % 512 || a.cols > GEMV_MAXK ||
         a.y_stride < a.rows || (a.epi == EPI_ADD && a.res_stride < a.rows) || a.n_more < 0 || a.n_more > GEMM_MAX_MORE ||
         (a.n_more && a.epi == EPI_SWIGLU))
         return hipErrorInvalidValue;

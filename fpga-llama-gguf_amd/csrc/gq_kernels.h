@@ -285,7 +285,10 @@ struct TokArgs {
 };
 
 constexpr int GEMV_MAXK = 16384;  // GEMV columns at most
-constexpr int GEMM_MAX_TOK = 32;  // tokens of one batched GEMV (two tiles of 16)
+constexpr int GEMM_MAX_TOK = 32;  // tokens of one GEMM command (two tiles of 16)
+constexpr int GEMM_WIDE_TOK = 512;  // tokens of a batched GEMV in the model driver's own lists (prompt chunks)
+// Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
+constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 : (n_tok + 15) / 16 * 16; }
 constexpr int ATTN_CHUNK = 64;
 constexpr int ATTN_MAXG = 8;  // q heads per KV head
 constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command

@@ -121,6 +121,8 @@ struct gemvq_ctx {
     uint16_t * gemm_d = nullptr;  // and their block scales
     uint16_t * gemm_s = nullptr;  // and their Q8_1 block sums (for Q4_1 weights)
     float * gemm_b = nullptr;     // and their parts of the term bounds
+    uint8_t * wide = nullptr;     // the same for a list of the model driver's prompt chunks (up to GEMM_WIDE_TOK rows)
+    int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
     int arith = GEMVQ_ARITH_CANONICAL;  // the arithmetic lists are compiled in (gemvq_set_arith)
     int last_launches = 0;
@@ -600,7 +602,7 @@ struct Compiler {
                 // z rows are packed (hv * 128 floats apart)
                 const uint32_t ntok = gates && k3[2] ? k3[2] : 1, sq = ntok > 1 ? k3[3] : 0, sg = ntok > 1 ? k3[4] : 0;
                 const uint64_t yz = uint64_t(hv) * 128 * (ntok - 1);
-                if (ntok > GEMVQ_GEMM_MAX_TOK || (ntok > 1 && (sq % 16 || sg % 16))) return reject(i, "GDN tokens");
+                if (ntok > uint32_t(c->max_tok) || (ntok > 1 && (sq % 16 || sg % 16))) return reject(i, "GDN tokens");
                 if (!range(k[2], uint64_t(sq) * (ntok - 1) + hk * 128) || !range(k[3], uint64_t(sq) * (ntok - 1) + hk * 128) ||
                     !range(k[4], uint64_t(sq) * (ntok - 1) + hv * 128) || !range(k[5], uint64_t(sg) * (ntok - 1) + hv) ||
                     !range(k[6], uint64_t(sg) * (ntok - 1) + hv) || !range(k[7], yz + hv * 128))
@@ -703,7 +705,7 @@ struct Compiler {
                 const uint32_t ch = k[1], ntok = (k[7] >> 16) ? (k[7] >> 16) : 1;  // packed token rows
                 const bool seqs = k[7] & GEMVQ_CONV_SEQS;  // token t of sequence t: windows packed, 3 ch apart
                 const uint64_t sw = 3ull * ch * (seqs ? ntok : 1);
-                if (ch == 0 || ch % 16 || ntok > GEMVQ_GEMM_MAX_TOK || !range(k[2], uint64_t(ch) * ntok) ||
+                if (ch == 0 || ch % 16 || ntok > uint32_t(c->max_tok) || !range(k[2], uint64_t(ch) * ntok) ||
                     !range(k[3], 4ull * ch) || !range(k[4], uint64_t(ch) * ntok) || !range(k[5], sw) ||
                     !range(k[6], sw))
                     return reject(i, "CONV range");
@@ -802,10 +804,11 @@ struct Compiler {
             }
             case GEMVQ_OP_GET_ROWS: {
                 const int type = int(k[1] & 0xffu), rows = int(k[2]), cols = int(k[3]);
-                const uint32_t ntok = (k[1] >> 16) & 0xffu ? (k[1] >> 16) & 0xffu : 1;  // ids 16 floats apart
+                const uint32_t tw = (k[1] >> 16) & (c->max_tok > GEMM_MAX_TOK ? 0xffffu : 0xffu);
+                const uint32_t ntok = tw ? tw : 1;  // ids 16 floats apart
                 const uint64_t woff = uint64_t(k[4]) | (uint64_t(k[5]) << 32);
                 if (type != T_Q6_K && type != T_Q4_0 && type != T_Q8_0) return reject(i, "GET_ROWS type");
-                if (ntok > GEMVQ_GEMM_MAX_TOK) return reject(i, "GET_ROWS tokens");
+                if (ntok > uint32_t(c->max_tok)) return reject(i, "GET_ROWS tokens");
                 if (!weight(woff, type, rows, cols)) return reject(i, "GET_ROWS weight");
                 if (!range(k[6], 16ull * (ntok - 1) + 1) || !range(k[7], uint64_t(cols) * ntok)) return reject(i, "GET_ROWS range");
                 GetRowsArgs a{weight_view(c->warena + woff, type, rows, cols), reinterpret_cast<const int32_t *>(A(k[6])),
@@ -875,6 +878,16 @@ struct Compiler {
         return true;
     }
 
+    // The activation scratch of a launch with more than GEMM_MAX_TOK tokens, one allocation (WIDE_BYTES).
+    static constexpr size_t WIDE_Q = size_t(GEMM_WIDE_TOK) * GEMV_MAXK, WIDE_BLOCKS = WIDE_Q / 32;
+    static constexpr size_t WIDE_BYTES = WIDE_Q + 2 * WIDE_BLOCKS * sizeof(uint16_t) + WIDE_BLOCKS / 16 * sizeof(float);
+    void wide_scratch(GemmQuantArgs & q) const {
+        q.q = reinterpret_cast<int8_t *>(c->wide);
+        q.d = reinterpret_cast<uint16_t *>(c->wide + WIDE_Q);
+        q.s = q.d + WIDE_BLOCKS;
+        q.bound = reinterpret_cast<float *>(q.s + WIDE_BLOCKS);
+    }
+
     // A batched GEMV at command i (two slots; a SwiGLU g takes its u command too): the activation rows are
     // quantized once into the context's scratch rows, then every weight row is read once for all the tokens.
     bool gemm(const uint32_t * cmds, unsigned n, unsigned i, unsigned & used) {
@@ -889,7 +902,7 @@ struct Compiler {
             return reject(i, "GEMM flags");
         if (kq && ((flags & GEMVQ_GEMV_SWIGLU) || !gemv_tok_ok(t, int(cols), 1, false)))
             return reject(i, "GEMM on K-quant weights: no SwiGLU pair, at most 12288 columns");
-        if (ntok < 1 || ntok > GEMVQ_GEMM_MAX_TOK) return reject(i, "GEMM token count");
+        if (ntok < 1 || ntok > uint32_t(c->max_tok) || (ntok > GEMVQ_GEMM_MAX_TOK && (kq || ref()))) return reject(i, "GEMM token count");
         if (xs % 16 || xs < cols || ys % 16 || ys < uint32_t(rows)) return reject(i, "GEMM strides");
         const uint64_t woff = uint64_t(k[4]) | (uint64_t(k[5]) << 32);
         const Weight * gw = weight(woff, t, rows, int(cols));
@@ -982,21 +995,25 @@ struct Compiler {
         GemmQuantArgs q{};
         q.x = A(k[6]);
         q.norm_w = normw ? A(k2[5]) : nullptr;
-        q.q = c->gemm_q;
-        q.d = c->gemm_d;
-        q.s = c->gemm_s;
-        q.bound = c->gemm_b;
+        if (ntok > GEMVQ_GEMM_MAX_TOK) {
+            wide_scratch(q);
+        } else {
+            q.q = c->gemm_q;
+            q.d = c->gemm_d;
+            q.s = c->gemm_s;
+            q.bound = c->gemm_b;
+        }
         q.n_tok = int(ntok);
-        q.n_pad = int((ntok + 15) / 16 * 16);
+        q.n_pad = gemm_pad(int(ntok));
         q.cols = int(cols);
         q.x_stride = int(xs);
         q.norm = norm ? 1 : 0;
         q.norm_l2 = (nflags & GEMVQ_NORM_L2) ? 1 : 0;
         q.eps = bits_f(k2[6]);
-        g.q = c->gemm_q;
-        g.d = c->gemm_d;
-        g.s = c->gemm_s;
-        g.bound = c->gemm_b;
+        g.q = q.q;
+        g.d = q.d;
+        g.s = q.s;
+        g.bound = q.bound;
         const bool same = lastq.on && lastq.x_off == k[6] && lastq.x_len == x_len && lastq.q.n_tok == q.n_tok &&
                           lastq.q.cols == q.cols && lastq.q.x_stride == q.x_stride && lastq.q.norm == q.norm &&
                           lastq.q.norm_l2 == q.norm_l2 && lastq.q.norm_w == q.norm_w && lastq.q.eps == q.eps;
@@ -1494,6 +1511,7 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->gemm_d);
     hipFree(c->gemm_s);
     hipFree(c->gemm_b);
+    hipFree(c->wide);
     hipFree(c->ref_x);
     hipFree(c->dbg);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -1690,6 +1708,24 @@ int gemvq_run(gemvq_ctx * c, const uint32_t * cmds, unsigned n) {
         c->dbg_used = false;
     }
     return e == hipSuccess ? 0 : fail(c, e, "run");
+}
+
+// Whether the lists compiled from now on may hold commands of up to GEMM_WIDE_TOK tokens (GEMM, CONV, GDN, GET_ROWS): for
+// the prompt chunks of the model driver, which switches it on around its own lists. A caller's lists keep the limits of
+// the header.
+__attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int on) {
+    if (!c) return GEMVQ_EINVAL;
+    if (on && !c->wide) {
+        if (!c->usable) return unusable(c);
+        hipSetDevice(c->device);
+        const hipError_t e = hipMalloc(&c->wide, Compiler::WIDE_BYTES);
+        if (e != hipSuccess) {
+            c->wide = nullptr;
+            return fail(c, e, "prompt chunk scratch");
+        }
+    }
+    c->max_tok = on ? GEMM_WIDE_TOK : GEMM_MAX_TOK;
+    return 0;
 }
 
 int gemvq_graph_create(gemvq_ctx * c, const uint32_t * cmds, unsigned n, int * graph) {

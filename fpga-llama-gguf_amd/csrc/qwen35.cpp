@@ -23,6 +23,8 @@ namespace {
 
 constexpr int F32 = 0, T_Q4_0 = 2, T_Q4_1 = 3, T_Q8_0 = 8, T_Q5_K = 13, T_Q6_K = 14;  // ggml type ids
 
+constexpr size_t PROMPT_CHUNK = 512;  // prompt tokens per chunk at most (GEMM_WIDE_TOK of gq_kernels.h)
+
 uint32_t fb(float f) {
     uint32_t b;
     std::memcpy(&b, &f, 4);
@@ -54,7 +56,9 @@ struct gemvq_qwen35 {
              logits = 0, rope = 0, prompt = 0, out = 0;
     std::vector<uint32_t> conv_state;  // per layer
     size_t act_floats = 0;
-    // batched prefill: rows of up to GEMVQ_GEMM_MAX_TOK prompt tokens (token ids and positions one per 16 floats)
+    // batched prefill: rows of up to `chunk` prompt tokens (token ids, and the positions of the attention's batches of
+    // GEMVQ_GEMM_MAX_TOK tokens, one per 16 floats)
+    uint32_t chunk = GEMVQ_GEMM_MAX_TOK;
     bool can_batch = false;
     std::string batch_why;
     uint32_t bh = 0, bqkv = 0, bcqkv = 0, bz = 0, bbeta = 0, balpha = 0, by = 0, bqg = 0, bk = 0, bv = 0, batt = 0,
@@ -116,7 +120,11 @@ size_t layout(gemvq_qwen35 & m, const gemvq_tensor_desc * tab, int n) {
     m.att = take(size_t(c.n_head) * c.head_dim);
     m.ffn = take(c.n_ff);
     m.logits = take(c.n_vocab);
-    const size_t B = GEMVQ_GEMM_MAX_TOK;
+    // A prompt chunk of a single sequence: as much of the context as the widest batched GEMV takes. Longer chunks read the
+    // weights and start launches less often, and past 32 tokens the batched GEMV is bound by its arithmetic.
+    const size_t most = size_t(c.n_ctx + 31) / 32 * 32;
+    m.chunk = m.n_seq > 1 ? GEMVQ_GEMM_MAX_TOK : uint32_t(std::max<size_t>(GEMVQ_GEMM_MAX_TOK, std::min<size_t>(most, PROMPT_CHUNK)));
+    const size_t B = m.chunk;
     m.bh = take(B * c.n_embd);
     m.bqkv = take(B * ch);
     m.bcqkv = take(B * ch);
@@ -130,7 +138,7 @@ size_t layout(gemvq_qwen35 & m, const gemvq_tensor_desc * tab, int n) {
     m.batt = take(B * c.n_head * c.head_dim);
     m.bffn = take(B * c.n_ff);
     m.bid = take(B * 16);
-    m.bpos = take(16);
+    m.bpos = take(B / GEMVQ_GEMM_MAX_TOK * 16);
     if (m.n_seq > 1) {
         m.skey = take(ns * 16);
         m.spos = take(ns * 16);
@@ -210,11 +218,16 @@ bool build_chunk(const gemvq_qwen35 & m, uint32_t ntok, std::vector<uint32_t> & 
             e.gemm(*W(p + "attn_q.weight"), m.bh, E, m.bqg, qrow, ntok, 0, 0, 0, an, eps);
             e.gemm(*W(p + "attn_k.weight"), m.bh, E, m.bk, kvrow, ntok, 0, 0, 0, an, eps);
             e.gemm(*W(p + "attn_v.weight"), m.bh, E, m.bv, kvrow, ntok, 0, 0, 0, an, eps);
-            // the chunk's tokens at positions act[bpos] + i, packed rows (q + gate, k, v, output)
-            e.cmd({GEMVQ_OP_ATTN, uint32_t(c.n_head) | (uint32_t(c.n_head_kv) << 16), m.bqg, uint32_t(m.kv[il]), m.batt,
-                   hd | (uint32_t(c.n_rot) << 16), m.bpos, 1u | (ntok << 16)});
-            e.cmd({m.bk, m.bv, fb(1.0f / std::sqrt(float(c.head_dim))), fb(eps), W(p + "attn_q_norm.weight")->act_off,
-                   W(p + "attn_k_norm.weight")->act_off, m.rope, m.bqg + hd});
+            // batches of up to GEMVQ_GEMM_MAX_TOK of the chunk's tokens, batch b's at positions act[bpos + 16 b] + i, packed
+            // rows (q + gate, k, v, output)
+            for (uint32_t t0 = 0; t0 < ntok; t0 += GEMVQ_GEMM_MAX_TOK) {
+                const uint32_t nt = std::min(GEMVQ_GEMM_MAX_TOK, ntok - t0);
+                e.cmd({GEMVQ_OP_ATTN, uint32_t(c.n_head) | (uint32_t(c.n_head_kv) << 16), m.bqg + t0 * qrow, uint32_t(m.kv[il]),
+                       m.batt + t0 * arow, hd | (uint32_t(c.n_rot) << 16), m.bpos + t0 / GEMVQ_GEMM_MAX_TOK * 16, 1u | (nt << 16)});
+                e.cmd({m.bk + t0 * kvrow, m.bv + t0 * kvrow, fb(1.0f / std::sqrt(float(c.head_dim))), fb(eps),
+                       W(p + "attn_q_norm.weight")->act_off, W(p + "attn_k_norm.weight")->act_off, m.rope,
+                       m.bqg + t0 * qrow + hd});
+            }
             e.gemm(*W(p + "attn_output.weight"), m.batt, arow, m.bh, E, ntok, GEMVQ_GEMV_ADD, m.bh, E);
         } else {
             // the four projections of the normed rows back to back (one quantization), then the conv
@@ -382,6 +395,7 @@ bool build_commands(gemvq_qwen35 & m, std::string & err) {
 }  // namespace
 
 extern "C" void gq_set_error(gemvq_ctx * ctx, const char * what);  // gq_runtime.hip
+extern "C" int gq_wide_lists(gemvq_ctx * ctx, int on);
 
 namespace {
 int set_err(gemvq_ctx * ctx, const std::string & what) {
@@ -538,19 +552,24 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
     if (st) return st;
     const int np = int(m->prompt_ids.size());
     if (pos < 0 || pos + n > np - 1) return set_err(ctx, "gemvq_qwen35_prefill: positions past the last prompt token but one");
+    // chunks of the layout's rows; the reference arithmetic runs its commands token by token and keeps their limit
+    const int most = gemvq_arith(ctx) == GEMVQ_ARITH_REFERENCE ? int(GEMVQ_GEMM_MAX_TOK) : int(m->chunk);
+    if (most > int(GEMVQ_GEMM_MAX_TOK)) st = gq_wide_lists(ctx, 1);
     std::vector<uint32_t> w;
     for (int p0 = pos; p0 < pos + n && !st;) {
-        const int nt = std::min<int>(GEMVQ_GEMM_MAX_TOK, pos + n - p0);
-        std::vector<int32_t> slots(size_t(16) * GEMVQ_GEMM_MAX_TOK, 0);  // ids, one per 16 floats
+        const int nt = std::min<int>(most, pos + n - p0);
+        std::vector<int32_t> slots(size_t(16) * nt, 0);  // ids, one per 16 floats
         for (int i = 0; i < nt; ++i) slots[size_t(16) * i] = m->prompt_ids[size_t(p0 + i)];
         st = gemvq_act_write(ctx, m->bid, slots.data(), slots.size());
-        if (!st) st = gemvq_act_write(ctx, m->bpos, &p0, 1);  // the chunk's first position
-        if (!st && nt == int(GEMVQ_GEMM_MAX_TOK)) {
-            // full chunks replay one captured list: it reads the chunk's ids and first position from the slots
-            // just written (the write waits for the previous replay; the replay follows it on the same stream)
+        std::vector<int32_t> first(size_t(nt + GEMVQ_GEMM_MAX_TOK - 1) / GEMVQ_GEMM_MAX_TOK * 16, 0);  // the batches' first positions
+        for (size_t i = 0; i < first.size(); i += 16) first[i] = p0 + int(i / 16 * GEMVQ_GEMM_MAX_TOK);
+        if (!st) st = gemvq_act_write(ctx, m->bpos, first.data(), first.size());
+        if (!st && nt == most) {
+            // full chunks replay one captured list: it reads the chunk's ids and positions from the slots just written
+            // (the write waits for the previous replay; the replay follows it on the same stream)
             if (m->chunk_graph < 0) {
                 w.clear();
-                build_chunk(*m, GEMVQ_GEMM_MAX_TOK, w);
+                build_chunk(*m, uint32_t(most), w);
                 st = gemvq_graph_create(ctx, w.data(), unsigned(w.size() / GEMVQ_CMD_WORDS), &m->chunk_graph);
             }
             if (!st) st = gemvq_graph_replay(ctx, m->chunk_graph, 1);
@@ -561,6 +580,7 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
         }
         p0 += nt;
     }
+    if (most > int(GEMVQ_GEMM_MAX_TOK)) gq_wide_lists(ctx, 0);
     if (!st) st = gemvq_sync(ctx);
     if (st) return st;
     // what the steps' NEXT_TOKEN would have left: the next prompt token at the next position, the ids so far

@@ -47,8 +47,8 @@ int gemvq_qwen35_reset(gemvq_qwen35 * m, const int32_t * prompt, int n);
 /* Enqueues n decode steps (replays of the per-token graph, captured by the first step after create or after a
  * reset with a new prompt length); asynchronous. */
 int gemvq_qwen35_step(gemvq_qwen35 * m, int n);
-/* Runs the next n prompt positions (all before the last prompt token) in chunks of up to GEMVQ_GEMM_MAX_TOK tokens
- * per weight read (GEMM commands; the reference plans this batched path, ROADMAP.md:78-96, and has no counterpart):
+/* Runs the next n prompt positions (all before the last prompt token) in chunks of up to 512 tokens (as much
+ * of them as n_ctx holds; GEMVQ_GEMM_MAX_TOK in the reference arithmetic) per weight read (GEMM commands; the reference plans this batched path, ROADMAP.md:78-96, and has no counterpart):
  * afterwards the model is where n decode steps would have left it (states, KV cache, position, token ids), bit for
  * bit, without the logits. GEMVQ_EINVAL when a projection has no batched form (Q4_0 / Q4_1 / Q8_0 with columns a
  * multiple of 512; decode steps then do the same work) or the positions pass the last prompt token but one; synchronizes. */

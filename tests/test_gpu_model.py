@@ -252,3 +252,38 @@ def test_batched_prefill_declines_unbatchable_models(gq, q35):
         assert not m.prefill(5)
         m.step(9)
         assert m.tokens(10)[9] >= 0
+
+
+@pytest.mark.parametrize("wtype,n_prompt,outliers", [("q4_0", 34, False), ("q4_1", 66, False), ("q8_0", 130, False),
+                                                     ("q4_0", 517, False), ("q4_0", 100, True), ("q8_0", 66, True)])
+def test_prompt_chunks_of_many_tokens_equal_decode_steps(gq, q35, wtype, n_prompt, outliers):
+    """Prompt chunks past 32 tokens (the batched GEMV over groups of 64 tokens, the token-parallel conv, attention in
+    batches of 32): one token past a batch or group, two and more groups, a full chunk of 512 and a remainder; with
+    activation outliers (norm weights of 2e3 in some columns) the steps that sum term by term. States, cache, ids and the
+    generation after it equal the decode steps' bit for bit."""
+    cfg = q35.Config(n_layer=4, n_embd=1024, n_ff=1536, n_vocab=1040, n_head=4, n_head_kv=1, head_dim=128, n_rot=32,
+                     ssm_k_heads=2, ssm_v_heads=4, n_ctx=n_prompt + 8, wtype=getattr(gq, wtype.upper()))
+    blob = q35.generate(cfg, seed=3)
+    if outliers:
+        for il in range(cfg.n_layer):
+            for name in ("attn_norm", "post_attention_norm"):
+                nw = blob.tensor(f"blk.{il}.{name}.weight").view(np.float32)
+                nw[[5, 700]] = 2e3  # ffn_down's steps pass 2^50 LSB; rows stay within the fixed point's 2^63
+    prompt = q35.prompt_ids(cfg, n_prompt, seed=3)
+    with q35.Model(blob) as m:
+        m.reset(prompt)
+        m.step(n_prompt - 1)
+        want = _decode_state(m, cfg, n_prompt - 1)
+        m.step(4)
+        t_steps, l_steps = m.tokens(n_prompt + 4), m.logits()
+        m.reset(prompt)
+        print(f"[prompt] {wtype} {n_prompt} outliers {outliers}", flush=True)
+        assert m.prefill(n_prompt - 1)
+        got = _decode_state(m, cfg, n_prompt - 1)
+        assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32)), "DeltaNet states"
+        for a, b in zip(got[1], want[1]):
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), "KV cache"
+        assert np.array_equal(got[2], want[2]), "token ids"
+        m.step(4)
+        assert np.array_equal(m.tokens(n_prompt + 4), t_steps)
+        assert np.array_equal(m.logits().view(np.uint32), l_steps.view(np.uint32))
