@@ -17,6 +17,10 @@
 // LSB 2^-40, so that one rounding is the term's floor, and the sum of the floors is exact while it stays within 2^51
 // LSB (checked per 16 blocks; past it the terms go to int64 one by one). The accumulator's bits less those of
 // 1.5 * 2^52 LSB are the integer sum.
+// Q6_K (super-blocks of 256 weights on Q8_K activations) has one term per super-block, of the sum of its 16 sub-block
+// sums times their int8 scales: the sub-block sums come from the same matrix product with half of each operand zeroed (an
+// operand's low and high words belong to different sub-blocks), the scales multiply them in the vector ALUs, and the
+// super-block's scale product, 11 by 24 bits, is exact in FP64; the fused multiply-add then floors as above.
 // Q4_1 adds the term floor(m_w * s_x * 2^40) with the Q8_1 s_x of each activation block (gemvq_ref.h:194-229), its
 // product by one more FP16 matrix product of the same form.
 #include "gq_gemv_impl.h"
@@ -105,6 +109,43 @@ __global__ __launch_bounds__(NT) void gemm_quant_kernel(GemmQuantArgs a) {
     }
 }
 
+// The same for K-quant weights: Q8_K super-blocks (gemvq_ref.h:62-81) by the single-token prologue's quantizer, the quants
+// in the same order, the FP32 scales (subnormals as zero, as the block terms take them) per tile and step as two rows of 16
+// tokens, and the step's sum of |d_x| * (sum of |quants|) * 2^40.
+__device__ __forceinline__ float * act_kscale(uint16_t * d, int tok, int ns, int sb) {
+    return reinterpret_cast<float *>(d) + (size_t(tok >> 4) * ns + (sb >> 1)) * 32 + (sb & 1) * 16 + (tok & 15);
+}
+
+__global__ __launch_bounds__(NT) void gemm_quant_k_kernel(GemmQuantArgs a) {
+    __shared__ Lds s;
+    const int tok = blockIdx.x, nb = a.cols / 32, ns = nb / GS, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool pad = tok >= a.n_tok;  // padding tokens: zero quants and scales
+    if (!pad) {
+        const float * x = a.x + size_t(tok) * a.x_stride;
+        const float sc = a.norm ? block_norm_scale(x, a.cols, a.eps, a.norm_l2, s) : 1.0f;
+        quantize_q8_K(x, a.cols, a.norm != 0, a.norm_w, sc, s.xq, s.bs, s.info);
+        __syncthreads();
+    }
+    const uint32_t * q = reinterpret_cast<const uint32_t *>(s.xq);
+    for (int i = threadIdx.x; i < nb * 4; i += NT) {  // block b, group g
+        const int b = i >> 2, g = i & 3;
+        *reinterpret_cast<v2u *>(a.q + act_group(tok, g, ns, b)) = pad ? v2u{0u, 0u} : v2u{q[b * 8 + g], q[b * 8 + 4 + g]};
+    }
+    for (int step = wave; step < ns; step += NWAVES) {
+        const int sb = step * 2 + (lane >> 5);  // lane l: 16 quants of super-block l / 32 of the step
+        uint32_t mag = 0, bits = 0;
+        if (!pad) {
+            bits = s.info[sb];
+            if ((bits & 0x7f800000u) == 0) bits = 0;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) mag = __builtin_amdgcn_sad_u8(q[step * 128 + 2 * lane + k] ^ 0x80808080u, 0x80808080u, mag);
+        }
+        const float bs = pair_sum_lanes<64>(fabsf(__uint_as_float(bits)) * float(mag));
+        if ((lane & 31) == 0) *act_kscale(a.d, tok, ns, sb) = __uint_as_float(bits);
+        if (lane == 0) a.bound[act_bound(tok, ns, step)] = bs * 1099511627776.0f;
+    }
+}
+
 // ---- weights ----
 // One step of one 16-row tile as a wave loads it: lane l takes row l / 4; of its 16 blocks the quants of blocks 4c + l % 4
 // (instruction c: 64 contiguous bytes of a row by four neighbouring lanes; Q8_0 twice) and the scales of blocks
@@ -115,6 +156,15 @@ struct WStep {
     v4u q[4];
     v4u q2[TYPE == T_Q8_0 ? 4 : 1];  // the high halves of Q8_0 blocks
     typename std::conditional<TYPE == T_Q4_1, v4u, v2u>::type s;  // Q4_1: four (d, m) pairs; others: four d
+};
+
+// Q6_K: of the row's two super-blocks the 16 low-bit pieces as the quants above, the high-bit pieces 4c + l % 4 (unit
+// l % 4 of super-block c), 8 of the 32 sub-block scales, and both d.
+template <>
+struct WStep<T_Q6_K> {
+    v4u q[4], h[2];
+    v2u s;
+    uint32_t d;
 };
 
 // blk: the first block of the step in row l / 4
@@ -134,6 +184,18 @@ __device__ __forceinline__ void load_wstep(const WeightView & w, size_t blk, int
     } else {
         o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>((TYPE == T_Q4_0 ? w.b : w.c) + sb * 2));
     }
+}
+
+template <>
+__device__ __forceinline__ void load_wstep<T_Q6_K>(const WeightView & w, size_t blk, int part, WStep<T_Q6_K> & o) {
+    const v4u * p = reinterpret_cast<const v4u *>(w.a + (blk + part) * 16);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.q[c] = __builtin_nontemporal_load(p + 4 * c);
+    const v4u * h = reinterpret_cast<const v4u *>(w.b + blk * 8) + part;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) o.h[c] = __builtin_nontemporal_load(h + 4 * c);
+    o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(w.c + blk * 2) + part);
+    o.d = *reinterpret_cast<const uint32_t *>(w.d + blk / 4);
 }
 
 // A wave's step in its part of LDS, which turns the load order into the operand order: the 16-byte quants of (row r,
@@ -174,6 +236,32 @@ __device__ __forceinline__ long a_operand(uint32_t lo, uint32_t hi) {
     return long((uint64_t(w1) << 32) | w0);
 }
 
+// Q6_K: the high-bit pieces as the quants; the sub-block scales as integers, those of unit u of super-block c in row r at
+// (4c + u) * 16 + r; d as loaded.
+template <>
+struct WLds<T_Q6_K> {
+    uint32_t q[1][4][256], h[2][256];
+    int s[8 * 16][4];
+    uint32_t d[16];
+};
+
+template <>
+__device__ __forceinline__ void stage<T_Q6_K>(const WStep<T_Q6_K> & w, int lane, WLds<T_Q6_K> & l) {
+    const int row = lane >> 2, part = lane & 3, slot = 4 * (4 * row + ((part + (row >> 2)) & 3));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][c][slot]) = w.q[c];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) *reinterpret_cast<v4u *>(&l.h[c][slot]) = w.h[c];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {  // scales 8 part .. + 7 of the row's 32: units 2 part and 2 part + 1 of its eight
+        v4i v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = int(w.s[k] << (24 - 8 * i)) >> 24;
+        *reinterpret_cast<v4i *>(l.s[(2 * part + k) * 16 + row]) = v;
+    }
+    if (part == 0) l.d[row] = w.d;
+}
+
 // The launch as the kernel reads it: the members of a group (one, of a SwiGLU pair) by index, their 16-row tiles after
 // one another.
 struct GemmMember {
@@ -208,6 +296,13 @@ struct XStep {
     float bound;  // the largest over the token tiles
 };
 
+template <int T>
+struct XStep<T_Q6_K, T> {
+    v4u q[T][GS / 2];
+    float d[T][2];  // token r's scales of the step's super-blocks
+    float bound;
+};
+
 template <int TYPE, int T>
 __device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lane, int tile, int step, XStep<TYPE, T> & o) {
     float bd[T];
@@ -217,7 +312,12 @@ __device__ __forceinline__ void load_xstep(const GemmLaunch & a, int ns, int lan
         const v4u * p = reinterpret_cast<const v4u *>(a.q + at * 8192) + lane;
 #pragma unroll
         for (int k = 0; k < GS / 2; ++k) o.q[t][k] = p[k * WAVE];
-        o.d[t] = reinterpret_cast<const v2u *>(a.d + at * 256)[lane];
+        if constexpr (TYPE == T_Q6_K) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) o.d[t][k] = reinterpret_cast<const float *>(a.d)[at * 32 + k * 16 + (lane & 15)];
+        } else {
+            o.d[t] = reinterpret_cast<const v2u *>(a.d + at * 256)[lane];
+        }
         if constexpr (TYPE == T_Q4_1) o.s[t] = reinterpret_cast<const v2u *>(a.s + at * 256)[lane];
         bd[t] = a.bound[at * 16 + (lane & 15)];
     }
@@ -234,9 +334,50 @@ __device__ __forceinline__ v4h one_scale(const v2u & d, int c, bool mine) {
     return __builtin_bit_cast(v4h, o);
 }
 
-// 1.5 * 2^52 LSB: the FP64 accumulator's base. Q4_0 block sums carry a factor 16, so the LSB is 2^-36 there.
+// 1.5 * 2^52 LSB: the FP64 accumulator's base. Q4_0 block sums carry a factor 16 and Q6_K sums 4, so the LSB is 2^-36 and
+// 2^-38 there.
 template <int TYPE>
-constexpr double acc_base() { return TYPE == T_Q4_0 ? 98304.0 : 6144.0; }
+constexpr double acc_base() { return TYPE == T_Q4_0 ? 98304.0 : TYPE == T_Q6_K ? 24576.0 : 6144.0; }
+
+// The sums S = sum over the 16 sub-blocks of scale * (sum of quant products), times 4, of super-block sb of a Q6_K step:
+// S[t][i] of row 4g + i, token r. A quant byte is 4 (q - 32): the nibble in bits 2..5, its high bits in 6 and 7, the sign
+// bit flipped. Unit j's low nibbles are its quants A and the high nibbles its quants B (gq_runtime.hip's repack), 16 of each
+// per 16-byte piece and sub-block: an operand's low word belongs to the first sub-block, its high word to the second.
+template <int T>
+__device__ __forceinline__ void superblock_sums(const WLds<T_Q6_K> & l, const XStep<T_Q6_K, T> & x, int sb, int lane, int (*S)[4]) {
+    const int r = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[t][i] = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_sched_barrier(0);  // one unit in work at a time: its products must fit in registers
+        const int pc = sb * 8 + 4 * (j >> 1) + 2 * (j & 1);  // the unit's first low-bit piece
+        const auto slot = [&](int c) { return 4 * (4 * r + ((c + (r >> 2)) & 3)) + g; };
+        const uint32_t q0 = l.q[0][pc >> 2][slot(pc & 3)], q1 = l.q[0][pc >> 2][slot((pc & 3) + 1)], hw = l.h[sb][slot(j)];
+        constexpr uint32_t LO = 0x3C3C3C3Cu, HI = 0xC0C0C0C0u, SG = 0x80808080u;
+        const uint32_t w[4] = {(((q0 << 2) & LO) | ((hw << 6) & HI)) ^ SG, (((q1 << 2) & LO) | ((hw << 4) & HI)) ^ SG,
+                               (((q0 >> 2) & LO) | ((hw << 2) & HI)) ^ SG, (((q1 >> 2) & LO) | (hw & HI)) ^ SG};
+        v4i sc[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[i] = *reinterpret_cast<const v4i *>(l.s[(sb * 4 + j) * 16 + 4 * g + i]);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {  // sub-blocks: A's first and second 16, B's
+                const int blk = sb * 8 + 4 * (j >> 1) + 2 * (k >> 1) + (j & 1);
+                const v4u qv = x.q[t][blk >> 1];
+                const long bx = (blk & 1) ? long((uint64_t(qv[3]) << 32) | qv[2]) : long((uint64_t(qv[1]) << 32) | qv[0]);
+                const v4i zi = {0, 0, 0, 0};
+                const long aop = (k & 1) ? long(uint64_t(w[k]) << 32) : long(uint64_t(w[k]));
+                const v4i p = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) S[t][i] += __mul24(sc[i][k], p[i]);
+            }
+        }
+    }
+}
 
 // One step into the accumulators acc[t][i] (row 4g + i, token r of token tile t).
 template <int TYPE, int T>
@@ -281,6 +422,42 @@ __device__ __forceinline__ void step_terms(const WLds<TYPE> & l, const XStep<TYP
 
 __device__ __forceinline__ void add_total(long long * p, long long v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Q6_K's step: per super-block and output one fused multiply-add, or with `exact` (wave-uniform; as step_terms_exact) the single-token
+// kernel's integer term, added to the int64 totals.
+template <int T>
+__device__ __forceinline__ void step_terms_k(const WLds<T_Q6_K> & l, const XStep<T_Q6_K, T> & x, int lane, bool exact,
+                                             double (*acc)[4], long long (*tot)[4][WAVE]) {
+    const int g = lane >> 4;
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb) {
+        int S[T][4];
+        superblock_sums<T>(l, x, sb, lane, S);
+        if (!exact) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double dw = h2f(l.d[4 * g + i] >> (16 * sb) & 0xffffu);
+#pragma unroll
+                for (int t = 0; t < T; ++t) acc[t][i] = __builtin_fma(double(S[t][i]), dw * double(x.d[t][sb]), acc[t][i]);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                int m, e;
+                float_parts(x.d[t][sb], m, e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t dw = l.d[4 * g + i] >> (16 * sb) & 0xffffu;
+                    int md, ed;
+                    half_parts(dw, md, ed);
+                    const int v = S[t][i] >> 2;  // exact: a multiple of 4
+                    const bool neg = ((dw >> 15) ^ (__float_as_uint(x.d[t][sb]) >> 31)) & 1;
+                    add_total(&tot[t][i][lane], fixed_term((long long)(neg ? -v : v) * ((long long)md * (long long)m), ed + e));
+                }
+            }
+        }
+    }
 }
 
 // One step with every term formed alone and added to the int64 totals: for steps whose terms could pass the
@@ -328,6 +505,8 @@ __device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLd
 // blocks over the wave, as the host's weight_bound forms it.
 template <int TYPE>
 __device__ __forceinline__ float step_bound(const WLds<TYPE> & l, int lane) {
+    if constexpr (TYPE == T_Q6_K) return __builtin_inff();
+    else {
     uint32_t dm = 0, mm = 0;
     constexpr int N = TYPE == T_Q4_1 ? 4 : 2;
 #pragma unroll
@@ -343,6 +522,7 @@ __device__ __forceinline__ float step_bound(const WLds<TYPE> & l, int lane) {
     }
     constexpr float smax = TYPE == T_Q4_0 ? 32.0f * 8 * 127 : TYPE == T_Q4_1 ? 32.0f * 15 * 127 : 32.0f * 128 * 127;
     return h2f(dm) * smax + (TYPE == T_Q4_1 ? h2f(mm) * (32.0f * 127) : 0.0f);
+    }
 }
 
 // FP64 round mode (MODE bits 3:2; 0 nearest even, 2 toward minus infinity). FP32 arithmetic keeps its own. As asm: the
@@ -418,8 +598,9 @@ void gemm_kernel(GemmLaunch a) {
                     else if (m + 1 < NM) load_wstep<TYPE>(a.w2, first_block(b, mi) + size_t(wave) * GS, part, wn);
                     else if (bn < a.n_tiles) load_wstep<TYPE>(a.m[next].w, first_block(bn, next) + size_t(wave) * GS, part, wn);
                     const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
-                    if (__builtin_amdgcn_ballot_w64(!(wb * xs.bound < limit)) != 0)
-                        step_terms_exact<TYPE, T>(a, wl, ns, lane, 0, step, tot[set][m]);
+                    const bool exact = __builtin_amdgcn_ballot_w64(!(wb * xs.bound < limit)) != 0;
+                    if constexpr (TYPE == T_Q6_K) step_terms_k<T>(wl, xs, lane, exact, acc, tot[set][m]);
+                    else if (exact) step_terms_exact<TYPE, T>(a, wl, ns, lane, 0, step, tot[set][m]);
                     else step_terms<TYPE, T>(wl, xs, lane, acc);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -623,10 +804,14 @@ hipError_t launch_tiles(const GemmArgs & g, hipStream_t st) {
         a.n_tiles += (o.rows + GT - 1) / GT;
     }
     const int steps = a.cols / (32 * GS);
-    if (a.n_tok > 2 * GT) {
+    if constexpr (TYPE == T_Q6_K) {
+        if (a.n_tok > 2 * GT) return hipErrorInvalidValue;
+    } else if (a.n_tok > 2 * GT) {
         const int n_tg = (a.n_tok + WT * GT - 1) / (WT * GT);
         GQ_LAUNCH((gemm_wide_kernel<TYPE, PAIR>), dim3(std::min(n_tg * a.n_tiles, 256)), dim3(GNT), 0, st, a, n_tg);
-    } else if (a.n_tok <= GT) {
+        return hipGetLastError();
+    }
+    if (a.n_tok <= GT) {
         if (steps <= GNW) launch_one<TYPE, PAIR, 1, 1>(a, st);
         else if (steps <= 3 * GNW) launch_one<TYPE, PAIR, 1, 3>(a, st);
         else launch_one<TYPE, PAIR, 1, 0>(a, st);
@@ -649,7 +834,8 @@ hipError_t launch_gemm_quant(const GemmQuantArgs & a, hipStream_t s) {
     if (a.n_tok < 1 || a.n_pad != gemm_pad(a.n_tok) || a.n_tok > GEMM_WIDE_TOK || a.cols % 512 ||
         a.cols > GEMV_MAXK || a.x_stride < a.cols || a.x_stride % 16)
         return hipErrorInvalidValue;
-    GQ_LAUNCH(gemm_quant_kernel, dim3(a.n_pad), dim3(NT), 0, s, a);
+    if (a.kq) GQ_LAUNCH(gemm_quant_k_kernel, dim3(a.n_pad), dim3(NT), 0, s, a);
+    else GQ_LAUNCH(gemm_quant_kernel, dim3(a.n_pad), dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 
@@ -667,6 +853,7 @@ hipError_t launch_gemm(const GemmArgs & a, int type, hipStream_t s) {
     case T_Q4_0: return launch_type<T_Q4_0>(a, s);
     case T_Q4_1: return launch_type<T_Q4_1>(a, s);
     case T_Q8_0: return launch_type<T_Q8_0>(a, s);
+    case T_Q6_K: return a.epi == EPI_SWIGLU ? hipErrorInvalidValue : launch_tiles<T_Q6_K, false>(a, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -233,6 +233,7 @@ struct GemmQuantArgs {
     int n_tok, n_pad, cols, x_stride;
     int norm, norm_l2;
     float eps;
+    int kq;                // K-quant weights: Q8_K super-blocks (d holds their FP32 scales; s is not written)
 };
 
 constexpr int GEMM_MAX_MORE = 3;  // a GEMM group has at most four members
@@ -287,6 +288,9 @@ struct TokArgs {
 constexpr int GEMV_MAXK = 16384;  // GEMV columns at most
 constexpr int GEMM_MAX_TOK = 32;  // tokens of one GEMM command (two tiles of 16)
 constexpr int GEMM_WIDE_TOK = 512;  // tokens of a batched GEMV in the model driver's own lists (prompt chunks)
+// Q6_K GEMMs of at least this many tokens and weights take the matrix-core form, the others the small-token GEMV.
+constexpr unsigned GEMM_KQ_TOK = 3;
+constexpr unsigned long long GEMM_KQ_SIZE = 1ull << 24;
 // Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
 constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 : (n_tok + 15) / 16 * 16; }
 constexpr int ATTN_CHUNK = 64;

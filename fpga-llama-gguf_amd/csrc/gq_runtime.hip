@@ -31,7 +31,7 @@ namespace {
 struct Weight {
     int type, rows, cols;
     size_t bytes;
-    float wbound;  // Q4_0 / Q4_1 / Q8_0: the largest block term magnitude over |d_x| * 2^40 (see weight_bound)
+    float wbound;  // the largest block term magnitude over |d_x| * 2^40 (see weight_bound)
 };
 
 // IEEE binary16 to float (subnormals, infinities and NaN included).
@@ -43,8 +43,22 @@ float half_to_float_host(uint16_t h) {
 
 // The largest |block term| / (|d_x| 2^40) of a Q4_0 / Q4_1 / Q8_0 matrix: over its blocks, |d_w| times the largest
 // |sum of products| with Q8_0 quants (|q_x| <= 127: 32 * 8 * 127 for Q4_0, 32 * 15 * 127 for Q4_1, 32 * 128 * 127
-// for Q8_0), plus for Q4_1 |m_w| times the largest |s_x| / d_x (32 * 127); rounded up to FP32. 0 for other types.
+// for Q8_0), plus for Q4_1 |m_w| times the largest |s_x| / d_x (32 * 127); rounded up to FP32. For Q6_K the largest
+// |super-block term| / (|d_x| * (sum of |quants|)): |d_w| times its largest |sub-block scale| times 32. 0 for Q5_K.
 float weight_bound(int type, int rows, int cols, const uint8_t * gguf) {
+    if (type == T_Q6_K) {
+        double best = 0.0;
+        for (size_t i = 0, n = size_t(rows) * size_t(cols / 256); i < n; ++i) {
+            const uint8_t * blk = gguf + i * 210;
+            int sc = 0;
+            for (int j = 0; j < 16; ++j) sc = std::max(sc, std::abs(int(int8_t(blk[192 + j]))));
+            uint16_t u;
+            std::memcpy(&u, blk + 208, 2);
+            const double t = std::fabs(double(half_to_float_host(u))) * (32.0 * sc);
+            if (!(t <= best)) best = t;  // a NaN scale makes the bound NaN
+        }
+        return std::nextafter(float(best), INFINITY);
+    }
     if (type != T_Q4_0 && type != T_Q4_1 && type != T_Q8_0) return 0.0f;
     const size_t nb = size_t(rows) * size_t(cols / 32), bb = type == T_Q4_0 ? 18 : type == T_Q4_1 ? 20 : 34;
     const double smax = type == T_Q4_0 ? 32.0 * 8 * 127 : type == T_Q4_1 ? 32.0 * 15 * 127 : 32.0 * 128 * 127;
@@ -895,7 +909,7 @@ struct Compiler {
         const uint32_t * k = cmds + size_t(i) * GEMVQ_CMD_WORDS, * k2 = k + GEMVQ_CMD_WORDS;
         const int t = int(k[1] & 0xffu), rows = int(k[2]);
         const uint32_t flags = k[1] & ~0xffu, cols = k[3], ntok = k2[0], xs = k2[1], ys = k2[2], nflags = k2[7];
-        const bool kq = t == T_Q5_K || t == T_Q6_K;  // no MFMA form: launches of up to 4 tokens of the small-token GEMV
+        const bool kq = t == T_Q5_K || t == T_Q6_K;  // launches of up to 4 tokens of the small-token GEMV, or for Q6_K (k_mfma) MFMA
         if (t != T_Q4_0 && t != T_Q4_1 && t != T_Q8_0 && !kq) return reject(i, "GEMM format (Q4_0, Q4_1, Q8_0, Q5_K or Q6_K)");
         if (rows <= 0 || cols == 0 || cols % 512 || cols > GEMVQ_MAX_COLS) return reject(i, "GEMM shape (cols a multiple of 512)");
         if (flags & ~(GEMVQ_GEMV_SWIGLU | GEMVQ_GEMV_ADD | GEMVQ_GEMV_SILU) || __builtin_popcount(flags) > 1)
@@ -955,7 +969,8 @@ struct Compiler {
         const bool over = (y_off < k[6] + x_len && k[6] < y_off + y_len) || (normw && y_off < k2[5] + cols && k2[5] < y_off + y_len);
         if (kq && over && !ref()) return reject(i, "GEMM on K-quant weights: the output falls on the input rows or the norm weight");
         if (ref()) return gemm_ref(g, t, k, k2, over, normw, i, used);
-        if (kq || (!over && gemv_tok_ok(t, int(cols), int(ntok), g.epi == EPI_SWIGLU))) {
+        const bool k_mfma = t == T_Q6_K && ntok >= GEMM_KQ_TOK && uint64_t(rows) * cols >= GEMM_KQ_SIZE;
+        if ((kq && !k_mfma) || (!kq && !over && gemv_tok_ok(t, int(cols), int(ntok), g.epi == EPI_SWIGLU))) {
             const uint32_t cs = kq ? (gemv_tok_ok(t, int(cols), TOK_MAX, false) ? TOK_MAX : 2) : ntok;  // tokens a launch
             for (uint32_t c0 = 0; c0 < ntok; c0 += cs) {
                 const uint32_t nt = std::min(cs, ntok - c0);
@@ -1010,13 +1025,14 @@ struct Compiler {
         q.norm = norm ? 1 : 0;
         q.norm_l2 = (nflags & GEMVQ_NORM_L2) ? 1 : 0;
         q.eps = bits_f(k2[6]);
+        q.kq = kq ? 1 : 0;
         g.q = q.q;
         g.d = q.d;
         g.s = q.s;
         g.bound = q.bound;
         const bool same = lastq.on && lastq.x_off == k[6] && lastq.x_len == x_len && lastq.q.n_tok == q.n_tok &&
                           lastq.q.cols == q.cols && lastq.q.x_stride == q.x_stride && lastq.q.norm == q.norm &&
-                          lastq.q.norm_l2 == q.norm_l2 && lastq.q.norm_w == q.norm_w && lastq.q.eps == q.eps;
+                          lastq.q.norm_l2 == q.norm_l2 && lastq.q.norm_w == q.norm_w && lastq.q.eps == q.eps && lastq.q.kq == q.kq;
         if (!same) {
             out.push_back(LGemmQ{q});
             spans.push_back({int(i), int(used)});
