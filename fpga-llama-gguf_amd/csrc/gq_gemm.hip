@@ -147,10 +147,10 @@ __global__ __launch_bounds__(NT) void gemm_quant_k_kernel(GemmQuantArgs a) {
 }
 
 // ---- weights ----
-// One step of one 16-row tile as a wave loads it: lane l takes row l / 4; of its 16 blocks the quants of blocks 4c + l % 4
-// (instruction c: 64 contiguous bytes of a row by four neighbouring lanes; Q8_0 twice) and the scales of blocks
-// 4 (l % 4) .. + 3 as they lie in memory. Weight bytes are read once per launch: the non-temporal hint keeps them from
-// displacing the activations in L2.
+// One step of one 16-row tile as a wave loads it: of its 16 blocks' quants, instruction c reads blocks 8 (c / 2) + l % 8 of
+// rows 8 (c % 2) + l / 8, so that eight neighbouring lanes read a whole 128-byte line (Q8_0 twice), and the scales of blocks
+// 4 (l % 4) .. + 3 of row l / 4 as they lie in memory. Weight bytes are read once per launch: the non-temporal hint keeps
+// them from displacing the activations in L2.
 template <int TYPE>
 struct WStep {
     v4u q[4];
@@ -158,8 +158,8 @@ struct WStep {
     typename std::conditional<TYPE == T_Q4_1, v4u, v2u>::type s;  // Q4_1: four (d, m) pairs; others: four d
 };
 
-// Q6_K: of the row's two super-blocks the 16 low-bit pieces as the quants above, the high-bit pieces 4c + l % 4 (unit
-// l % 4 of super-block c), 8 of the 32 sub-block scales, and both d.
+// Q6_K: of the row's two super-blocks the 16 low-bit pieces as the quants above, the high-bit piece l % 8 (unit l % 4 of
+// super-block l % 8 / 4) of row 8 c + l / 8, 8 of the 32 sub-block scales, and both d.
 template <>
 struct WStep<T_Q6_K> {
     v4u q[4], h[2];
@@ -167,35 +167,38 @@ struct WStep<T_Q6_K> {
     uint32_t d;
 };
 
-// blk: the first block of the step in row l / 4
-template <int TYPE>
-__device__ __forceinline__ void load_wstep(const WeightView & w, size_t blk, int part, WStep<TYPE> & o) {
-    const v4u * p = reinterpret_cast<const v4u *>(w.a + (blk + part) * 16);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) o.q[c] = __builtin_nontemporal_load(p + 4 * c);
-    if constexpr (TYPE == T_Q8_0) {
-        const v4u * p2 = reinterpret_cast<const v4u *>(w.b + (blk + part) * 16);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) o.q2[c] = __builtin_nontemporal_load(p2 + 4 * c);
-    }
-    const size_t sb = blk + 4 * part;
-    if constexpr (TYPE == T_Q4_1) {
-        o.s = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(w.b + sb * 4));
-    } else {
-        o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>((TYPE == T_Q4_0 ? w.b : w.c) + sb * 2));
-    }
-}
+// Where a lane's part of a step starts: the step's first block in rows l / 8, 8 + l / 8 and l / 4.
+// (Block indices: a matrix has fewer than 2^32 blocks of 32, checked at launch.)
+struct WAt {
+    uint32_t lo, hi, sc;
+};
 
-template <>
-__device__ __forceinline__ void load_wstep<T_Q6_K>(const WeightView & w, size_t blk, int part, WStep<T_Q6_K> & o) {
-    const v4u * p = reinterpret_cast<const v4u *>(w.a + (blk + part) * 16);
+// A SwiGLU pair's tile is 8 rows of g over the same 8 rows of u: rows 8 .. 15 (at.hi and the upper half's at.sc) are u's.
+template <int TYPE, bool PAIR>
+__device__ __forceinline__ void load_wstep(const WeightView & w, const WeightView & w2, const WAt & at, int lane, WStep<TYPE> & o) {
+    const int col = lane & 7;
+    const auto piece = [&](const uint8_t * lo, const uint8_t * hi, int c) {
+        return __builtin_nontemporal_load(reinterpret_cast<const v4u *>(
+            (PAIR && (c & 1) ? hi : lo) + size_t((c & 1 ? at.hi : at.lo) + 8 * (c >> 1) + col) * 16));
+    };
 #pragma unroll
-    for (int c = 0; c < 4; ++c) o.q[c] = __builtin_nontemporal_load(p + 4 * c);
-    const v4u * h = reinterpret_cast<const v4u *>(w.b + blk * 8) + part;
+    for (int c = 0; c < 4; ++c) o.q[c] = piece(w.a, w2.a, c);
+    if constexpr (TYPE == T_Q8_0) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c) o.h[c] = __builtin_nontemporal_load(h + 4 * c);
-    o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(w.c + blk * 2) + part);
-    o.d = *reinterpret_cast<const uint32_t *>(w.d + blk / 4);
+        for (int c = 0; c < 4; ++c) o.q2[c] = piece(w.b, w2.b, c);
+    }
+    if constexpr (TYPE == T_Q6_K) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)  // the row's 8 high-bit pieces
+            o.h[c] = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(w.b + size_t(c & 1 ? at.hi : at.lo) * 8) + col);
+        o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(w.c + size_t(at.sc) * 2) + (lane & 3));
+        o.d = *reinterpret_cast<const uint32_t *>(w.d + (at.sc >> 2));
+    } else {
+        const uint8_t * sb = TYPE == T_Q8_0 ? (PAIR && lane >= 32 ? w2.c : w.c) : (PAIR && lane >= 32 ? w2.b : w.b);
+        const size_t at4 = at.sc + 4 * (lane & 3);
+        if constexpr (TYPE == T_Q4_1) o.s = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(sb + at4 * 4));
+        else o.s = __builtin_nontemporal_load(reinterpret_cast<const v2u *>(sb + at4 * 2));
+    }
 }
 
 // A wave's step in its part of LDS, which turns the load order into the operand order: the 16-byte quants of (row r,
@@ -208,14 +211,21 @@ struct WLds {
     uint32_t s[WAVE * (TYPE == T_Q4_1 ? 4 : 2)];
 };
 
+// The word slot of the piece that lane l loaded with instruction c (row 8 (c % 2) + l / 8, piece l % 4 of its KiB).
+__device__ __forceinline__ int stage_slot(int lane, int c) {
+    const int row = 8 * (c & 1) + (lane >> 3);
+    return 4 * (4 * row + (((lane & 3) + (row >> 2)) & 3));
+}
+
 template <int TYPE>
 __device__ __forceinline__ void stage(const WStep<TYPE> & w, int lane, WLds<TYPE> & l) {
-    const int row = lane >> 2, part = lane & 3, slot = 4 * (4 * row + ((part + (row >> 2)) & 3));
+    const int row = lane >> 2, part = lane & 3;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][c][slot]) = w.q[c];
+    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][2 * (c >> 1) + (lane >> 2 & 1)][stage_slot(lane, c)]) = w.q[c];
     if constexpr (TYPE == T_Q8_0) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[WLds<TYPE>::QH - 1][c][slot]) = w.q2[c];
+        for (int c = 0; c < 4; ++c)
+            *reinterpret_cast<v4u *>(&l.q[WLds<TYPE>::QH - 1][2 * (c >> 1) + (lane >> 2 & 1)][stage_slot(lane, c)]) = w.q2[c];
     }
     if constexpr (TYPE == T_Q4_1) *reinterpret_cast<v4u *>(&l.s[4 * (part * 16 + row)]) = w.s;
     else *reinterpret_cast<v2u *>(&l.s[2 * (part * 16 + row)]) = w.s;
@@ -247,11 +257,11 @@ struct WLds<T_Q6_K> {
 
 template <>
 __device__ __forceinline__ void stage<T_Q6_K>(const WStep<T_Q6_K> & w, int lane, WLds<T_Q6_K> & l) {
-    const int row = lane >> 2, part = lane & 3, slot = 4 * (4 * row + ((part + (row >> 2)) & 3));
+    const int row = lane >> 2, part = lane & 3;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][c][slot]) = w.q[c];
+    for (int c = 0; c < 4; ++c) *reinterpret_cast<v4u *>(&l.q[0][2 * (c >> 1) + (lane >> 2 & 1)][stage_slot(lane, c)]) = w.q[c];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) *reinterpret_cast<v4u *>(&l.h[c][slot]) = w.h[c];
+    for (int c = 0; c < 2; ++c) *reinterpret_cast<v4u *>(&l.h[lane >> 2 & 1][stage_slot(lane, c)]) = w.h[c];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {  // scales 8 part .. + 7 of the row's 32: units 2 part and 2 part + 1 of its eight
         v4i v;
@@ -352,7 +362,6 @@ __device__ __forceinline__ void superblock_sums(const WLds<T_Q6_K> & l, const XS
         for (int i = 0; i < 4; ++i) S[t][i] = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        __builtin_amdgcn_sched_barrier(0);  // one unit in work at a time: its products must fit in registers
         const int pc = sb * 8 + 4 * (j >> 1) + 2 * (j & 1);  // the unit's first low-bit piece
         const auto slot = [&](int c) { return 4 * (4 * r + ((c + (r >> 2)) & 3)) + g; };
         const uint32_t q0 = l.q[0][pc >> 2][slot(pc & 3)], q1 = l.q[0][pc >> 2][slot((pc & 3) + 1)], hw = l.h[sb][slot(j)];
@@ -393,7 +402,6 @@ __device__ __forceinline__ void step_terms(const WLds<TYPE> & l, const XStep<TYP
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        __builtin_amdgcn_sched_barrier(0);  // four blocks in work at a time: their products must fit in registers
 #pragma unroll
         for (int gb = 0; gb < 4; ++gb) {
             // block 4c + gb: its scales are lane group c's, at place gb
@@ -529,257 +537,183 @@ __device__ __forceinline__ float step_bound(const WLds<TYPE> & l, int lane) {
 // compiler, which takes the default mode for granted, sets it back ahead of FP64 instructions after a builtin's switch.
 #define GQ_ROUND_F64(mode) asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), " #mode "\n\ts_nop 3" ::: "memory")
 
-// A workgroup takes the tiles of 16 rows b, b + gridDim.x, .. of all members, each against T tiles of 16 tokens; of a
-// SwiGLU pair the same rows of both matrices in turn. Its wave w sums the steps of 16 blocks w, w + 8, .. of every tile.
-// The launch is a stream of weight bytes, so the weights move past activations that stay: with up to 8 steps (4096
-// columns; HOLD = 1) or, for one token tile, 24 (12288 columns; HOLD = 3) a wave holds the activation operands of its
-// steps in registers for the whole launch, and requests the weights of its next step, or of the next tile's first,
-// before it sums the current one. Every load instruction reads whole 64-byte (activation: 1 KiB) runs; the operand
-// order comes from the wave's own part of LDS, without a workgroup barrier. The waves' sums meet in int64 totals in LDS
-// (exact in any order; two sets in turn, so one barrier a tile).
-// Measured (events, Q4_0, MI355X) against four waves sharing one staged tile, two rounds of 16 blocks in flight, seven
-// vector instructions a term: gate/up pair 2 x 12288 x 4096 17.1 us at 16 tokens and 27 at 32 (57 MB: 3.3 and 2.1 TB/s),
-// 12352 x 4096 group 13.2 and 20, 4096 x 12288 12.0 and 16.5, 4096 x 4096 5.8 and 8.1; the average launch of a layer 12.0
-// instead of 17.9 and 17.7 instead of 29.8. Loads whose neighbouring lanes lay in different rows (the operand order read
-// straight from memory) took 20.5 and 30.5: the address unit then works a line per lane.
-template <int TYPE, bool PAIR, int T, int HOLD>
-__global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(T == 1 && HOLD == 1 ? 4 : 2)))
-void gemm_kernel(GemmLaunch a) {
-    constexpr int NM = PAIR ? 2 : 1;
-    __shared__ WLds<TYPE> ws[GNW];
-    __shared__ long long tot[2][NM][T][4][WAVE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lrow = lane >> 2, part = lane & 3;
-    const int nb = a.cols / 32, ns = nb / GS;
-    const int per_wave = (ns + GNW - 1) / GNW;
-    const float limit = 1125899906842624.0f / float(per_wave);  // 2^50 LSB over the wave's steps (half of what fits)
-    const bool mine = wave < ns;
-    WLds<TYPE> & wl = ws[wave];
-    int mi = member_of(a, blockIdx.x);
-    WStep<TYPE> wn;
-    XStep<TYPE, T> x[HOLD ? HOLD : 1];
-    const auto first_block = [&](int b, int mb) {  // of this lane's row of tile b
-        return size_t(min((b - a.m[mb].tile0) * GT + lrow, a.m[mb].rows - 1)) * nb;
-    };
-    if (mine) {
-        if constexpr (HOLD > 0) {
-#pragma unroll
-            for (int h = 0; h < HOLD; ++h)
-                if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, 0, wave + GNW * h, x[h]);
-        }
-        load_wstep<TYPE>(a.m[mi].w, first_block(blockIdx.x, mi) + size_t(wave) * GS, part, wn);
-    }
-    for (int i = tid; i < 2 * NM * T * 4 * WAVE; i += GNT) (&tot[0][0][0][0][0])[i] = 0;
-    __syncthreads();
-    GQ_ROUND_F64(2);
-    double acc[T][4];
-#pragma unroll
-    for (int k = 0; k < T; ++k)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[k][i] = acc_base<TYPE>();
-            asm volatile("" : "+v"(acc[k][i]));  // the sums stay behind the mode switch
-        }
-    int set = 0;
-    for (int b = blockIdx.x; b < a.n_tiles; b += gridDim.x, set ^= 1) {
-        const int bn = b + int(gridDim.x);
-        const int next = bn < a.n_tiles ? member_of(a, bn) : mi;
-        if (mine) {
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const WeightView & w = PAIR && m ? a.w2 : a.m[mi].w;
-                const auto one = [&](int step, XStep<TYPE, T> & xs) {
-                    if constexpr (HOLD == 0) load_xstep<TYPE, T>(a, ns, lane, 0, step, xs);
-                    stage<TYPE>(wn, lane, wl);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    if (step + GNW < ns) load_wstep<TYPE>(w, first_block(b, mi) + size_t(step + GNW) * GS, part, wn);
-                    else if (m + 1 < NM) load_wstep<TYPE>(a.w2, first_block(b, mi) + size_t(wave) * GS, part, wn);
-                    else if (bn < a.n_tiles) load_wstep<TYPE>(a.m[next].w, first_block(bn, next) + size_t(wave) * GS, part, wn);
-                    const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
-                    const bool exact = __builtin_amdgcn_ballot_w64(!(wb * xs.bound < limit)) != 0;
-                    if constexpr (TYPE == T_Q6_K) step_terms_k<T>(wl, xs, lane, exact, acc, tot[set][m]);
-                    else if (exact) step_terms_exact<TYPE, T>(a, wl, ns, lane, 0, step, tot[set][m]);
-                    else step_terms<TYPE, T>(wl, xs, lane, acc);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                };
-                if constexpr (HOLD > 0) {
-#pragma unroll
-                    for (int h = 0; h < HOLD; ++h)
-                        if (wave + GNW * h < ns) one(wave + GNW * h, x[h]);
-                } else {
-                    for (int step = wave; step < ns; step += GNW) one(step, x[0]);
-                }
-#pragma unroll
-                for (int k = 0; k < T; ++k)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        add_total(&tot[set][m][k][i][lane],
-                                  __builtin_bit_cast(long long, acc[k][i]) - __builtin_bit_cast(long long, acc_base<TYPE>()));
-                        acc[k][i] = acc_base<TYPE>();
-                    }
-            }
-        }
-        __syncthreads();
-        // thread e: row e % 16 of token e / 16 (consecutive rows are stored together); the total is cleared for the
-        // tile after next, whose sums start behind the next barrier
-        if (tid < T * GT * GT) {
-            const int tok = tid >> 4, rr = tid & 15, src = (rr >> 2) * 16 + (tok & 15);
-            long long sum[NM];
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                long long * p = &tot[set][m][tok >> 4][rr & 3][src];
-                sum[m] = *p;
-                *p = 0;
-            }
-            const GemmMember & t = a.m[mi];
-            const int row = (b - t.tile0) * GT + rr;
-            if (row < t.rows && tok < a.n_tok) {
-                const float v = fixed_to_float(sum[0]);
-                float out = v;
-                if (PAIR) {
-                    out = (v / (1.0f + expf_(-v))) * fixed_to_float(sum[NM - 1]);  // gemvqc_ops.h:88-92
-                } else if (t.epi == EPI_ADD) {
-                    out = v + t.res[size_t(tok) * t.res_stride + row];  // gemvqc16.cpp:282-301
-                } else if (t.epi == EPI_SILU) {
-                    out = silu_(v);
-                }
-                t.y[size_t(tok) * t.y_stride + row] = out;
-            }
-        }
-        mi = next;
-    }
-#pragma unroll
-    for (int k = 0; k < T; ++k)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[k][i]));
-    GQ_ROUND_F64(0);
+// Output rows of a tile: of a SwiGLU pair 8, each from a row of both matrices.
+template <bool PAIR>
+constexpr int tile_rows() { return PAIR ? GT / 2 : GT; }
+
+// The output of row rr of a tile for one token (lane `src` of the totals tt holds the token in lane group 0).
+template <bool PAIR>
+__device__ __forceinline__ float tile_output(int epi, const long long (*tt)[WAVE], int rr, int src, float res) {
+    const float v = fixed_to_float(tt[rr & 3][(rr >> 2) * 16 + src]);
+    if (PAIR) return (v / (1.0f + expf_(-v))) * fixed_to_float(tt[rr & 3][((rr >> 2) + 2) * 16 + src]);  // gemvqc_ops.h:88-92
+    if (epi == EPI_ADD) return v + res;  // gemvqc16.cpp:282-301
+    return epi == EPI_SILU ? silu_(v) : v;
 }
 
-// ---- more than 32 tokens: bound by the vector instructions of the terms, no longer by the weight bytes ----
-// The (token group of 64, tile of 16 rows) pairs of the launch, in this order, are dealt to the workgroups in equal
-// contiguous runs, each summed in batches of up to WTB tile products whose int64 totals lie in LDS. A batch goes through the
-// columns in chunks of 4096 (128 blocks): wave w holds the activation operands of the chunk's blocks 16 w .. 16 w + 15 for
-// all 64 tokens in registers while the batch's weights stream past, four token tiles to every weight operand formed, and
-// adds its part of each tile to the totals. (Held operands: read per tile instead, 64 tokens' would need four times the
-// weights' bandwidth from L2.)
-// Measured (trace, Q4_0, 511 tokens, MI355X): gate/up pair 2 x 12288 x 4096 290 us, 12352 x 4096 group 140 us, 4096 x 12288
-// 140-190 us; a layer's launches 0.66 ms, where 16 chunks of 32 tokens took 1.1 ms. At 16.4 cycles per 64 terms (the
-// matrix product, two conversions and the multiply-add in a loop of their own) the pair's terms alone are 172 us.
-constexpr int WT = 4;   // token tiles
-constexpr int WTB = 8;  // tile products per batch (64 KiB of totals)
+// The launch is a stream of weight bytes past activations that stay. The (token group of T tiles, tile of 16 rows) pairs,
+// in this order, are dealt to the workgroups in equal contiguous runs (a SwiGLU pair's tile: 8 rows of both matrices), each
+// summed in batches of up to 8 tiles whose int64 totals lie in LDS. A batch goes through the columns in chunks of 4096
+// (128 blocks): wave w holds the activation operands of the chunk's blocks 16 w .. 16 w + 15 in registers while the
+// batch's weights stream past, and adds its part of each tile to the totals (exact in any order). The waves meet at
+// barriers only around a batch, so that one wave's staging and waits run beside another's sums. With HOLD chunks of
+// operands in registers a launch of up to that many chunks reads its activations once per token group; HOLD = 0 reads a
+// chunk's operands once per batch. The weights of the next product, or of the next two where one workgroup per CU leaves
+// the registers, are requested before the current one is summed. Every load instruction reads whole 128-byte
+// (activation: 1 KiB) runs; the operand order comes from the wave's own part of LDS, without a workgroup barrier.
+// Up to 16 tokens the weight bytes bound the launch, past that more and more the vector instructions of the terms (405 a
+// wave and product of 16 blocks at one token tile, 662 at two, of which the terms are 192 and 384); past 32 tokens four
+// token tiles share every weight operand formed.
+// Measured (events, Q4_0, MI355X): gate/up pair 2 x 12288 x 4096 15.4 us at 16 tokens (57 MB: 3.7 TB/s) and 24 at 32, 12352 x
+// 4096 group 12.5 and 19, 4096 x 12288 12.5 and 17, 4096 x 4096 6.1 and 8.3. Four waves sharing one staged tile, two rounds of
+// 16 blocks in flight and seven vector instructions a term took 17.9 and 29.8 us for the average of these launches (now 11.6
+// and 17.0). Loads whose neighbouring lanes lay in different rows (the operand order read straight from memory): 20.5 and
+// 30.5; the address unit then works a line per lane. 511 tokens (trace): pair 290 us, group 140 us, a layer's launches 0.66
+// ms, where 16 chunks of 32 tokens took 1.1 ms; at 16.4 cycles per 64 terms (the matrix product, two conversions and the
+// multiply-add in a loop of their own) the pair's terms alone are 172 us.
+template <int T>
+constexpr int batch_tiles() { return T == 1 ? 4 : 8; }  // (two workgroups' LDS per CU for one token tile)
 
-template <int TYPE, bool PAIR>
-__global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_wide_kernel(GemmLaunch a, int n_tg) {
-    constexpr int NM = PAIR ? 2 : 1, TB = WTB / NM;  // row tiles per batch
+// Two workgroups per CU for the variants that 128 registers hold (Q4_0, 16 tokens: the gate/up pair 15.4 us, with one
+// workgroup and two products ahead 17.0), else one (Q8_0, where 128 registers spill: a layer's launches 254 us, 322 with two).
+template <int TYPE, int T, int HOLD>
+constexpr int groups_per_cu() { return T == 1 && HOLD == 1 && (TYPE == T_Q4_0 || TYPE == T_Q4_1) ? 2 : 1; }
+
+template <int TYPE, bool PAIR, int T, int HOLD>
+__global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2 * groups_per_cu<TYPE, T, HOLD>())))
+void gemm_kernel(GemmLaunch a, int n_tg) {
+    constexpr int AHEAD = T <= 2 && groups_per_cu<TYPE, T, HOLD>() == 1 ? 2 : 1, R = tile_rows<PAIR>(), GTB = batch_tiles<T>();
     __shared__ WLds<TYPE> ws[GNW];
-    __shared__ long long tot[WTB][WT][4][WAVE];
+    __shared__ long long tot[GTB][T][4][WAVE];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lrow = lane >> 2, part = lane & 3;
-    const int nb = a.cols / 32, ns = nb / GS, chunks = (ns + GNW - 1) / GNW;
+    const int nb = a.cols / 32, ns = nb / GS;
     WLds<TYPE> & wl = ws[wave];
     const int total = n_tg * a.n_tiles;
     const int begin = int((long long)(blockIdx.x) * total / gridDim.x), end = int((long long)(blockIdx.x + 1) * total / gridDim.x);
-    const auto first_block = [&](int b, int mb) {  // of this lane's row of tile b
-        return size_t(min((b - a.m[mb].tile0) * GT + lrow, a.m[mb].rows - 1)) * nb;
+    const auto batch = [&](int at) { return min(min(GTB, end - at), a.n_tiles - at % a.n_tiles); };  // tiles of the batch at `at`
+    // the products still to request, in the order they are summed: batch, step, tile; the member of the last one requested
+    int r_at = begin, r_n = begin < end ? batch(begin) : 0, r_step = wave, r_j = 0, r_lo = 0, r_hi = 0;
+    GemmMember rm{};
+    WStep<TYPE> wn[AHEAD];
+    float wb[AHEAD];  // their members' term bounds
+    const auto request = [&](WStep<TYPE> & o, float & bound) {
+        if (r_at >= end) return;
+        const int t = r_at % a.n_tiles + r_j;
+        if (t < r_lo || t >= r_hi) {
+            const int mi = member_of(a, t);
+            rm = a.m[mi];
+            r_lo = rm.tile0;
+            r_hi = mi + 1 < a.n_members ? a.m[mi + 1].tile0 : a.n_tiles;
+        }
+        const int r0 = (t - r_lo) * R, top = rm.rows - 1;
+        const uint32_t s0 = r_step * GS;
+        const WAt at{uint32_t(min(r0 + (lane >> 3), top)) * nb + s0, uint32_t(min(r0 + (PAIR ? 0 : 8) + (lane >> 3), top)) * nb + s0,
+                     uint32_t(min(r0 + (lane >> 2 & (R - 1)), top)) * nb + s0};
+        load_wstep<TYPE, PAIR>(rm.w, a.w2, at, lane, o);
+        bound = rm.wbound;
+        if (++r_j < r_n) return;
+        r_j = 0;
+        r_step += GNW;
+        if (r_step < ns) return;
+        r_step = wave;
+        r_at += r_n;
+        if (r_at < end) r_n = batch(r_at);
     };
-    WStep<TYPE> wn;
-    XStep<TYPE, WT> x;
-    int held = -1;  // the token group whose only chunk x holds
-    if (begin < end && wave < ns) {
-        const int b = begin % a.n_tiles, mi = member_of(a, b);
-        load_wstep<TYPE>(a.m[mi].w, first_block(b, mi) + size_t(wave) * GS, part, wn);
+    XStep<TYPE, T> x[HOLD ? HOLD : 1];
+    int held = -1;  // the token group whose operands x holds (HOLD > 0)
+    if (wave < ns) {
+        if (HOLD > 0 && begin < end) {
+            held = begin / a.n_tiles;
+#pragma unroll
+            for (int h = 0; h < HOLD; ++h)
+                if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, held * T, wave + GNW * h, x[h]);
+        }
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) request(wn[k], wb[k]);
     }
     for (int at = begin; at < end;) {
-        const int tg = at / a.n_tiles, t0 = at % a.n_tiles, n = min(min(TB, end - at), a.n_tiles - t0);
-        for (int i = tid; i < n * NM * WT * 4 * WAVE; i += GNT) (&tot[0][0][0][0])[i] = 0;
+        const int tg = at / a.n_tiles, t0 = at % a.n_tiles, n = batch(at);
+        for (int i = tid; i < n * T * 4 * WAVE; i += GNT) (&tot[0][0][0][0])[i] = 0;
         __syncthreads();
         GQ_ROUND_F64(2);
-        for (int kc = 0; kc < chunks; ++kc) {
-            const int step = kc * GNW + wave;
-            if (step >= ns) break;
-            if (chunks > 1 || held != tg) load_xstep<TYPE, WT>(a, ns, lane, tg * WT, step, x);
-            held = tg;
+        const auto chunk = [&](int step, XStep<TYPE, T> & xs) {
             for (int j = 0; j < n; ++j) {
-                const int mi = member_of(a, t0 + j);
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    stage<TYPE>(wn, lane, wl);
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    // the next product's weights: u of the pair, the next tile, the batch's first of the next chunk, or
-                    // the next batch's first
-                    if (m + 1 < NM) {
-                        load_wstep<TYPE>(a.w2, first_block(t0 + j, mi) + size_t(step) * GS, part, wn);
-                    } else {
-                        int b = t0 + j + 1, st = step;
-                        bool more = true;
-                        if (j + 1 == n) {
-                            if (step + GNW < ns) {
-                                b = t0;
-                                st = step + GNW;
-                            } else {
-                                more = at + n < end;
-                                b = (at + n) % a.n_tiles;
-                                st = wave;
-                            }
-                        }
-                        if (more) {
-                            const int mb = member_of(a, b);
-                            load_wstep<TYPE>(a.m[mb].w, first_block(b, mb) + size_t(st) * GS, part, wn);
-                        }
-                    }
-                    const float wb = a.m[mi].wbound < __builtin_inff() ? a.m[mi].wbound : step_bound<TYPE>(wl, lane);
-                    long long (*tt)[4][WAVE] = tot[j * NM + m];
-                    if (__builtin_amdgcn_ballot_w64(!(wb * x.bound < 1125899906842624.0f)) != 0) {  // 2^50 LSB
-                        step_terms_exact<TYPE, WT>(a, wl, ns, lane, tg * WT, step, tt);
-                    } else {
-                        double acc[WT][4];
-#pragma unroll
-                        for (int k = 0; k < WT; ++k)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                acc[k][i] = acc_base<TYPE>();
-                                asm volatile("" : "+v"(acc[k][i]));  // the sums stay between the mode switches
-                            }
-                        step_terms<TYPE, WT>(wl, x, lane, acc);
-#pragma unroll
-                        for (int k = 0; k < WT; ++k)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                asm volatile("" : "+v"(acc[k][i]));
-                                add_total(&tt[k][i][lane], __builtin_bit_cast(long long, acc[k][i]) -
-                                                               __builtin_bit_cast(long long, acc_base<TYPE>()));
-                            }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
+                stage<TYPE>(wn[0], lane, wl);
+                const float wbd = wb[0];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if constexpr (AHEAD == 2) {
+                    wn[0] = wn[1];
+                    wb[0] = wb[1];
                 }
+                request(wn[AHEAD - 1], wb[AHEAD - 1]);
+                const float bound = (wbd < __builtin_inff() ? wbd : step_bound<TYPE>(wl, lane)) * xs.bound;
+                const bool exact = __builtin_amdgcn_ballot_w64(!(bound < 1125899906842624.0f)) != 0;  // 2^50 LSB
+                if (TYPE != T_Q6_K && exact) {
+                    if constexpr (TYPE != T_Q6_K) step_terms_exact<TYPE, T>(a, wl, ns, lane, tg * T, step, tot[j]);
+                } else {
+                    double acc[T][4];
+#pragma unroll
+                    for (int k = 0; k < T; ++k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            acc[k][i] = acc_base<TYPE>();
+                            asm volatile("" : "+v"(acc[k][i]));  // the sums stay between the mode switches
+                        }
+                    if constexpr (TYPE == T_Q6_K) step_terms_k<T>(wl, xs, lane, exact, acc, tot[j]);
+                    else step_terms<TYPE, T>(wl, xs, lane, acc);
+#pragma unroll
+                    for (int k = 0; k < T; ++k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            asm volatile("" : "+v"(acc[k][i]));
+                            add_total(&tot[j][k][i][lane], __builtin_bit_cast(long long, acc[k][i]) -
+                                                               __builtin_bit_cast(long long, acc_base<TYPE>()));
+                        }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        };
+        if constexpr (HOLD > 0) {
+            if (held != tg && wave < ns) {
+                held = tg;
+#pragma unroll
+                for (int h = 0; h < HOLD; ++h)
+                    if (wave + GNW * h < ns) load_xstep<TYPE, T>(a, ns, lane, tg * T, wave + GNW * h, x[h]);
+            }
+#pragma unroll
+            for (int h = 0; h < HOLD; ++h)
+                if (wave + GNW * h < ns) chunk(wave + GNW * h, x[h]);
+        } else {
+            for (int step = wave; step < ns; step += GNW) {
+                load_xstep<TYPE, T>(a, ns, lane, tg * T, step, x[0]);
+                chunk(step, x[0]);
             }
         }
         GQ_ROUND_F64(0);
         __syncthreads();
-        // element e: row e % (16 TB) of the batch, token e / (16 TB) of the group: consecutive rows are stored together
-        for (int e = tid; e < TB * GT * WT * GT; e += GNT) {
-            const int q = e % (TB * GT), tk = e / (TB * GT), j = q / GT, rr = q % GT;
-            const int tok = tg * WT * GT + tk, src = (rr >> 2) * 16 + (tk & 15);
-            if (j >= n || tok >= a.n_tok) continue;
-            const GemmMember & t = a.m[member_of(a, t0 + j)];
-            const int row = (t0 + j - t.tile0) * GT + rr;
-            if (row >= t.rows) continue;
-            const float v = fixed_to_float(tot[j * NM][tk >> 4][rr & 3][src]);
-            float out = v;
-            if (PAIR) {
-                out = (v / (1.0f + expf_(-v))) * fixed_to_float(tot[j * NM + NM - 1][tk >> 4][rr & 3][src]);
-            } else if (t.epi == EPI_ADD) {
-                out = v + t.res[size_t(tok) * t.res_stride + row];
-            } else if (t.epi == EPI_SILU) {
-                out = silu_(v);
+        // element e: row e % R of tile e / (R tokens), its token in between (consecutive rows are stored together); four
+        // elements a thread at a time, their residuals requested together
+        for (int e0 = tid; e0 < n * R * T * GT; e0 += 4 * GNT) {
+            float res[4];
+            float * y[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = e0 + k * GNT, rr = e % R, tk = e / R % (T * GT), b = t0 + e / (R * T * GT), tok = tg * T * GT + tk;
+                const GemmMember & t = a.m[member_of(a, min(b, a.n_tiles - 1))];
+                const int row = (b - t.tile0) * R + rr;
+                const bool on = e < n * R * T * GT && tok < a.n_tok && row < t.rows;
+                y[k] = on ? t.y + size_t(tok) * t.y_stride + row : nullptr;
+                res[k] = on && !PAIR && t.epi == EPI_ADD ? t.res[size_t(tok) * t.res_stride + row] : 0.0f;
             }
-            t.y[size_t(tok) * t.y_stride + row] = out;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (!y[k]) continue;
+                const int e = e0 + k * GNT, rr = e % R, tk = e / R % (T * GT), j = e / (R * T * GT);
+                const int epi = PAIR ? int(EPI_SWIGLU) : a.m[member_of(a, t0 + j)].epi;
+                *y[k] = tile_output<PAIR>(epi, tot[j][tk >> 4], rr, tk & 15, res[k]);
+            }
         }
         __syncthreads();
         at += n;
@@ -788,9 +722,10 @@ __global__ __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) void g
 
 template <int TYPE, bool PAIR, int T, int HOLD>
 void launch_one(const GemmLaunch & a, hipStream_t st) {
-    // as many workgroups as the 256 CUs hold at once (two of 8 waves each where the registers allow)
-    const int grid = std::min(a.n_tiles, T == 1 && HOLD == 1 ? 512 : 256);
-    GQ_LAUNCH((gemm_kernel<TYPE, PAIR, T, HOLD>), dim3(grid), dim3(GNT), 0, st, a);
+    // as many workgroups as the 256 CUs hold at once
+    const int n_tg = (a.n_tok + T * GT - 1) / (T * GT);
+    const int grid = std::min(n_tg * a.n_tiles, 256 * groups_per_cu<TYPE, T, HOLD>());
+    GQ_LAUNCH((gemm_kernel<TYPE, PAIR, T, HOLD>), dim3(grid), dim3(GNT), 0, st, a, n_tg);
 }
 
 template <int TYPE, bool PAIR>
@@ -799,26 +734,23 @@ hipError_t launch_tiles(const GemmArgs & g, hipStream_t st) {
     for (int i = 0; i <= g.n_more; ++i) {  // members follow each other, every one at least a tile
         const GemmMore f{g.w, g.y, g.res, g.rows, g.y_stride, g.res_stride, g.epi};
         const GemmMore & o = i ? g.more[i - 1] : f;
-        if (o.rows < 1) return hipErrorInvalidValue;
+        if (o.rows < 1 || (uint64_t(o.rows) * unsigned(g.cols / 32)) >> 32) return hipErrorInvalidValue;
         a.m[i] = GemmMember{o.w, o.y, o.res, o.rows, o.y_stride, o.res_stride, o.epi, a.n_tiles, g.wbound[i]};
-        a.n_tiles += (o.rows + GT - 1) / GT;
+        a.n_tiles += (o.rows + tile_rows<PAIR>() - 1) / tile_rows<PAIR>();
     }
-    const int steps = a.cols / (32 * GS);
-    if constexpr (TYPE == T_Q6_K) {
-        if (a.n_tok > 2 * GT) return hipErrorInvalidValue;
-    } else if (a.n_tok > 2 * GT) {
-        const int n_tg = (a.n_tok + WT * GT - 1) / (WT * GT);
-        GQ_LAUNCH((gemm_wide_kernel<TYPE, PAIR>), dim3(std::min(n_tg * a.n_tiles, 256)), dim3(GNT), 0, st, a, n_tg);
-        return hipGetLastError();
-    }
+    const int chunks = (a.cols / (32 * GS) + GNW - 1) / GNW;
     if (a.n_tok <= GT) {
-        if (steps <= GNW) launch_one<TYPE, PAIR, 1, 1>(a, st);
-        else if (steps <= 3 * GNW) launch_one<TYPE, PAIR, 1, 3>(a, st);
+        if (chunks == 1) launch_one<TYPE, PAIR, 1, 1>(a, st);
+        else if (chunks <= 3) launch_one<TYPE, PAIR, 1, 3>(a, st);
         else launch_one<TYPE, PAIR, 1, 0>(a, st);
-    } else if (steps <= GNW) {
-        launch_one<TYPE, PAIR, 2, 1>(a, st);
+    } else if (a.n_tok <= 2 * GT) {
+        if (chunks == 1) launch_one<TYPE, PAIR, 2, 1>(a, st);
+        else launch_one<TYPE, PAIR, 2, 0>(a, st);
+    } else if constexpr (TYPE == T_Q6_K) {
+        return hipErrorInvalidValue;
     } else {
-        launch_one<TYPE, PAIR, 2, 0>(a, st);
+        if (chunks == 1) launch_one<TYPE, PAIR, 4, 1>(a, st);
+        else launch_one<TYPE, PAIR, 4, 0>(a, st);
     }
     return hipGetLastError();
 }
