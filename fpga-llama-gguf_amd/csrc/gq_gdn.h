@@ -7,21 +7,19 @@
 
 namespace gq {
 
-// L2 norm of q and k of the key head (ggml_l2_norm: x / max(sqrt(sum x^2), eps)), each lane holding 8 elements.
+// L2 norm of one row of a key head (ggml_l2_norm: x / max(sqrt(sum x^2), eps)), each lane holding 8 elements.
+__device__ __forceinline__ void gdn_l2(float (&v)[8], float eps) {
+    float sq[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sq[i] = v[i] * v[i];
+    const float f = 1.0f / fmaxf(sqrtf(pair_sum_lanes<16>(tree<8>(sq))), eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * f;
+}
+
 __device__ __forceinline__ void gdn_l2_qk(float (&q)[8], float (&k)[8], float eps) {
-    float sq[8], sk[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        sq[i] = q[i] * q[i];
-        sk[i] = k[i] * k[i];
-    }
-    const float tq = pair_sum_lanes<16>(tree<8>(sq)), tk = pair_sum_lanes<16>(tree<8>(sk));
-    const float fq = 1.0f / fmaxf(sqrtf(tq), eps), fk = 1.0f / fmaxf(sqrtf(tk), eps);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        q[i] = q[i] * fq;
-        k[i] = k[i] * fk;
-    }
+    gdn_l2(q, eps);
+    gdn_l2(k, eps);
 }
 
 // The step's gates: with `raw` (GDN gates flag) beta = sigmoid(b) and the log decay g = softplus(a_raw + dt) * a

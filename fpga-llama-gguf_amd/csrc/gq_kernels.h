@@ -125,6 +125,8 @@ struct GdnArgs {
     int s_qkv, s_gb, s_y;  // row strides (floats) between tokens of q / k / v, of g / beta, of y
     int seqs;              // nonzero: the tokens belong to n_tok sequences, token t on its own state rows (src and
                            // dst + t * hv * 128 rows), all in one launch
+    float * prep;          // many tokens of one sequence: where their L2 norms and gates are formed ahead (n_tok rows of 2
+                           // hk 128 + 2 hv floats), NULL: in the step
     // reference arithmetic with the gated output norm (GEMVQ_GDN_GATED): the step's launch also applies the norm to
     // its token's heads (z rows hv * 128 apart per token, the norm weight [128], the RMS eps); NULL gz: not applied
     const float * gz;
@@ -296,6 +298,9 @@ constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 :
 constexpr int ATTN_CHUNK = 64;
 constexpr int ATTN_MAXG = 8;  // q heads per KV head
 constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command
+// GDN commands of at least this many tokens form norms and gates in a launch of their own (a launch costs what about
+// three tokens do in the step).
+constexpr unsigned GDN_PREP_TOK = 8;
 
 // Profiling: when set (by gemvq_profile on the calling thread), launchers start kernels through
 // hipExtLaunchKernelGGL with these events, which record the kernel's own start and end on the device.

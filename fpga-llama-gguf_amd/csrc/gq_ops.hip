@@ -280,6 +280,83 @@ __global__ __launch_bounds__(128) void gdn_kernel(const float * src, const float
     }
 }
 
+// ---- the step over many tokens of one sequence, in two launches ----
+// A token's state update needs the one before it, but its L2 norms and gates do not, and gdn_kernel computes them again in
+// every row's lanes inside that chain (1.23 us a token at C5's heads, of which the chain itself is a sixth). So a first
+// launch forms them for all tokens at once, with the same operations on the same lanes: workgroup (token, 8 of the 2 hk
+// rows of q and k), 16 lanes a row as in gdn_kernel; the first one of a token also its decays and betas. prep: per token 2
+// hk 128 floats (q, then k), then the hv (decay, beta) pairs.
+constexpr int GDN_PREP_ROWS = 8;
+__global__ __launch_bounds__(128) void gdn_prep_kernel(GdnArgs a) {
+    const int tk = blockIdx.y, l16 = threadIdx.x & 15, r = blockIdx.x * GDN_PREP_ROWS + int(threadIdx.x >> 4);
+    float * out = a.prep + size_t(tk) * (2 * a.hk * 128 + 2 * a.hv);
+    if (blockIdx.x == 0)
+        for (int h = threadIdx.x; h < a.hv; h += 128) {
+            float bt;
+            const float decay = gdn_gates(a.flags & 8, a.g[size_t(tk) * a.s_gb + h], a.beta[size_t(tk) * a.s_gb + h],
+                                          a.flags & 8 ? a.dt[h] : 0.0f, a.flags & 8 ? a.a[h] : 0.0f, bt);
+            out[2 * a.hk * 128 + 2 * h] = decay;
+            out[2 * a.hk * 128 + 2 * h + 1] = bt;
+        }
+    if (r >= 2 * a.hk) return;  // whole groups of 16 lanes
+    const float * row = (r < a.hk ? a.q + r * 128 : a.k + (r - a.hk) * 128) + size_t(tk) * a.s_qkv + 8 * l16;
+    const float4 v0 = *reinterpret_cast<const float4 *>(row), v1 = *reinterpret_cast<const float4 *>(row + 4);
+    float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    if (a.flags & 2) gdn_l2(v, a.l2_eps);
+    float * o = out + r * 128 + 8 * l16;
+    *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4 *>(o + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+
+// The second runs the tokens in order: workgroup (value head, 8 state rows) as gdn_kernel, the state in registers, the
+// inputs of GDN_AHEAD tokens requested ahead (an update takes less time than a load).
+constexpr int GDN_AHEAD = 4;
+struct GdnPrepped {
+    float4 q0, q1, k0, k1;
+    float2 db;  // decay, beta
+    float v;
+};
+
+__global__ __launch_bounds__(128) void gdn_tokens_kernel(GdnArgs a) {
+    const int chunks = 128 / GDN_ROWS, h = blockIdx.x / chunks, chunk = blockIdx.x % chunks, kh = h % a.hk;
+    const int l16 = threadIdx.x & 15, j = chunk * GDN_ROWS + int(threadIdx.x >> 4);
+    const size_t row = (size_t(h) * 128 + j) * 128 + 8 * l16, ps = 2 * a.hk * 128 + 2 * a.hv;
+    const float * qp = a.prep + kh * 128 + 8 * l16, * kp = qp + a.hk * 128, * dp = a.prep + 2 * a.hk * 128 + 2 * h;
+    const float * vp = a.v + h * 128 + j;
+    float * yp = a.y + h * 128 + j;
+    const float4 s0 = *reinterpret_cast<const float4 *>(a.src + row), s1 = *reinterpret_cast<const float4 *>(a.src + row + 4);
+    float x[1][8] = {{s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w}};
+    GdnPrepped in[GDN_AHEAD];
+    const int n = a.n_tok;
+    const auto load = [&](int tk, GdnPrepped & o) {  // past the last token: the last one's again, not used
+        const size_t t = min(tk, n - 1);
+        o.q0 = *reinterpret_cast<const float4 *>(qp + t * ps);
+        o.q1 = *reinterpret_cast<const float4 *>(qp + t * ps + 4);
+        o.k0 = *reinterpret_cast<const float4 *>(kp + t * ps);
+        o.k1 = *reinterpret_cast<const float4 *>(kp + t * ps + 4);
+        o.db = *reinterpret_cast<const float2 *>(dp + t * ps);
+        o.v = vp[t * a.s_qkv];
+    };
+#pragma unroll
+    for (int i = 0; i < GDN_AHEAD; ++i) load(i, in[i]);
+    for (int tk = 0; tk < n; tk += GDN_AHEAD) {
+#pragma unroll
+        for (int i = 0; i < GDN_AHEAD; ++i) {
+            if (tk + i < n) {  // uniform over the workgroup
+                const GdnPrepped c = in[i];
+                load(tk + i + GDN_AHEAD, in[i]);
+                const float q[8] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, c.q1.x, c.q1.y, c.q1.z, c.q1.w};
+                const float k[8] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w};
+                float out[1];
+                gdn_step_rows<1>(q, k, &c.v, c.db.x, c.db.y, x, out);
+                if (l16 == 0) yp[size_t(tk + i) * a.s_y] = out[0] * a.scale;
+            }
+        }
+    }
+    *reinterpret_cast<float4 *>(a.dst + row) = make_float4(x[0][0], x[0][1], x[0][2], x[0][3]);
+    *reinterpret_cast<float4 *>(a.dst + row + 4) = make_float4(x[0][4], x[0][5], x[0][6], x[0][7]);
+}
+
 // ---- gated output norm (gemvqc_gdn.h:284-346): one wave per head, lane l holds elements 2l, 2l + 1 ----
 __global__ __launch_bounds__(64) void gated_norm_kernel(GatedNormArgs a) {
     const int h = blockIdx.x, l = threadIdx.x;
@@ -753,6 +830,11 @@ hipError_t launch_rope(const RopeArgs & a, hipStream_t s) {
 }
 
 hipError_t launch_gdn(const GdnArgs & a, hipStream_t s) {
+    if (!a.seqs && a.prep) {
+        GQ_LAUNCH(gdn_prep_kernel, dim3((2 * a.hk + GDN_PREP_ROWS - 1) / GDN_PREP_ROWS, a.n_tok), dim3(128), 0, s, a);
+        GQ_LAUNCH(gdn_tokens_kernel, dim3(a.hv * (128 / GDN_ROWS)), dim3(128), 0, s, a);
+        return hipGetLastError();
+    }
     if (a.seqs)
         GQ_LAUNCH(gdn_kernel<true>, dim3(a.hv * (128 / GDN_ROWS), a.n_tok), dim3(128), 0, s, a.src, a.q, a.k, a.v, a.g,
                   a.beta, a.hk, a);

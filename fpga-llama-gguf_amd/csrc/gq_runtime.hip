@@ -136,6 +136,9 @@ struct gemvq_ctx {
     uint16_t * gemm_s = nullptr;  // and their Q8_1 block sums (for Q4_1 weights)
     float * gemm_b = nullptr;     // and their parts of the term bounds
     uint8_t * wide = nullptr;     // the same for a list of the model driver's prompt chunks (up to GEMM_WIDE_TOK rows)
+    float * gdn_prep = nullptr;   // norms and gates of a GDN command's tokens, and the floats it holds; the smaller
+    size_t gdn_prep_n = 0;        // buffers before it, which captured graphs may still use
+    std::vector<float *> gdn_prep_old;
     int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
     int arith = GEMVQ_ARITH_CANONICAL;  // the arithmetic lists are compiled in (gemvq_set_arith)
@@ -698,6 +701,14 @@ struct Compiler {
                     i = next + 2;
                     return true;
                 }
+                // many tokens: norms and gates ahead of the step, unless an output row falls on what later tokens read
+                const std::vector<Rng> reads = {{k[2], uint64_t(k[2]) + uint64_t(sq) * (ntok - 1) + hk * 128},
+                                                {k[3], uint64_t(k[3]) + uint64_t(sq) * (ntok - 1) + hk * 128},
+                                                {k[4], uint64_t(k[4]) + uint64_t(sq) * (ntok - 1) + hv * 128},
+                                                {k[5], uint64_t(k[5]) + uint64_t(sg) * (ntok - 1) + hv},
+                                                {k[6], uint64_t(k[6]) + uint64_t(sg) * (ntok - 1) + hv}};
+                if (ntok >= GDN_PREP_TOK && !seqs && !meet_any({{k[7], uint64_t(k[7]) + yz + hv * 128}}, reads))
+                    a.prep = gdn_prep(size_t(ntok) * (2 * hk * 128 + 2 * hv));
                 if ((flags & GEMVQ_GDN_GATED) && ntok == 1 && fold_gated(cmds, n, next, k[7], hv * 128, k2[7], k2[6])) {
                     // the gated norm runs in the next GEMV's activation prologue: the step writes its raw output
                     // to scratch, and that GEMV writes the gated values to y as the norm would have
@@ -890,6 +901,21 @@ struct Compiler {
             ++i;
         }
         return true;
+    }
+
+    // A buffer of n floats for the norms and gates of a GDN command's tokens; NULL (they are formed in the step) without
+    // memory for it. Commands run in order, so they share one.
+    float * gdn_prep(size_t n) const {
+        if (c->gdn_prep_n >= n) return c->gdn_prep;
+        float * p = nullptr;
+        if (hipMalloc(&p, n * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (c->gdn_prep) c->gdn_prep_old.push_back(c->gdn_prep);
+        c->gdn_prep = p;
+        c->gdn_prep_n = n;
+        return p;
     }
 
     // The activation scratch of a launch with more than GEMM_MAX_TOK tokens, one allocation (WIDE_BYTES).
@@ -1528,6 +1554,8 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->gemm_s);
     hipFree(c->gemm_b);
     hipFree(c->wide);
+    hipFree(c->gdn_prep);
+    for (float * p : c->gdn_prep_old) hipFree(p);
     hipFree(c->ref_x);
     hipFree(c->dbg);
     if (c->stream) hipStreamDestroy(c->stream);
