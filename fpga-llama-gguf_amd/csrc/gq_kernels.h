@@ -327,6 +327,8 @@ hipError_t launch_attn(const AttnArgs & a, hipStream_t s);
 hipError_t launch_get_rows(const GetRowsArgs & a, hipStream_t s);
 hipError_t launch_argmax(const float * x, int n, unsigned long long * key, int rows, int stride, hipStream_t s);
 hipError_t launch_next_token(const NextTokenArgs & a, hipStream_t s);
+hipError_t launch_stage_copy(const void * src, void * dst, int n_words, hipStream_t s);
+hipError_t launch_done(uint32_t * flag, uint32_t v, hipStream_t s);
 hipError_t launch_gemm_quant(const GemmQuantArgs & a, hipStream_t s);
 hipError_t launch_gemm(const GemmArgs & a, int type, hipStream_t s);
 // Whether launch_gemv_tok has an instance for this weight type, width, token count and member kind (a SwiGLU pair).

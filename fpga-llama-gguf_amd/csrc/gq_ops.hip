@@ -952,6 +952,29 @@ hipError_t launch_argmax(const float * x, int n, unsigned long long * key, int r
     return hipGetLastError();
 }
 
+// ---- host copies and completion through pinned host memory ----
+// Words between the activation buffer and a staging area in host memory, on the launches' own queue (a copy by the runtime
+// goes to another engine and is waited for there). Stores to host memory are complete before the kernel ends.
+__global__ __launch_bounds__(256) void stage_copy_kernel(const uint32_t * src, uint32_t * dst, int n) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+    __threadfence_system();
+}
+__global__ void done_kernel(uint32_t * flag, uint32_t v) {
+    __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_stage_copy(const void * src, void * dst, int n_words, hipStream_t s) {
+    const int grid = (n_words + 1023) / 1024;
+    hipLaunchKernelGGL(stage_copy_kernel, dim3(grid < 256 ? grid : 256), dim3(256), 0, s, static_cast<const uint32_t *>(src),
+                       static_cast<uint32_t *>(dst), n_words);
+    return hipGetLastError();
+}
+
+hipError_t launch_done(uint32_t * flag, uint32_t v, hipStream_t s) {
+    hipLaunchKernelGGL(done_kernel, dim3(1), dim3(1), 0, s, flag, v);
+    return hipGetLastError();
+}
+
 hipError_t launch_next_token(const NextTokenArgs & a, hipStream_t s) {
     GQ_LAUNCH(next_token_kernel, dim3(1), dim3(a.n_seq > 1 ? ((a.n_seq + 63) / 64) * 64 : 1), 0, s, a);
     return hipGetLastError();
