@@ -261,7 +261,7 @@ struct GemmArgs {
     int n_more;         // members after the first (not with a SwiGLU pair); tiles of member i + 1 follow member i's
     GemmMore more[GEMM_MAX_MORE];
     float wbound[GEMM_MAX_MORE + 1];  // per member: the largest block term magnitude over |d_x| * 2^40 (INFINITY:
-                                      // unknown, every round's terms are summed in int64)
+                                      // unknown, each step's is formed from its scales)
 };
 
 // The GEMM command for 2-4 tokens on the single-token GEMV's structure: each lane keeps its activation blocks of

@@ -44,35 +44,31 @@ float half_to_float_host(uint16_t h) {
 // The largest |block term| / (|d_x| 2^40) of a Q4_0 / Q4_1 / Q8_0 matrix: over its blocks, |d_w| times the largest
 // |sum of products| with Q8_0 quants (|q_x| <= 127: 32 * 8 * 127 for Q4_0, 32 * 15 * 127 for Q4_1, 32 * 128 * 127
 // for Q8_0), plus for Q4_1 |m_w| times the largest |s_x| / d_x (32 * 127); rounded up to FP32. For Q6_K the largest
-// |super-block term| / (|d_x| * (sum of |quants|)): |d_w| times its largest |sub-block scale| times 32. 0 for Q5_K.
+// |super-block term| / (|d_x| * (sum of |quants|)): |d_w| times a sub-block scale of at most 128 times 32. 0 for Q5_K.
+// NaN if a scale is one: every launch on the matrix then sums in int64.
 float weight_bound(int type, int rows, int cols, const uint8_t * gguf) {
-    if (type == T_Q6_K) {
-        double best = 0.0;
-        for (size_t i = 0, n = size_t(rows) * size_t(cols / 256); i < n; ++i) {
-            const uint8_t * blk = gguf + i * 210;
-            int sc = 0;
-            for (int j = 0; j < 16; ++j) sc = std::max(sc, std::abs(int(int8_t(blk[192 + j]))));
-            uint16_t u;
-            std::memcpy(&u, blk + 208, 2);
-            const double t = std::fabs(double(half_to_float_host(u))) * (32.0 * sc);
-            if (!(t <= best)) best = t;  // a NaN scale makes the bound NaN
-        }
-        return std::nextafter(float(best), INFINITY);
-    }
-    if (type != T_Q4_0 && type != T_Q4_1 && type != T_Q8_0) return 0.0f;
-    const size_t nb = size_t(rows) * size_t(cols / 32), bb = type == T_Q4_0 ? 18 : type == T_Q4_1 ? 20 : 34;
-    const double smax = type == T_Q4_0 ? 32.0 * 8 * 127 : type == T_Q4_1 ? 32.0 * 15 * 127 : 32.0 * 128 * 127;
-    const auto h = [](const uint8_t * p) {
+    const auto bits = [](const uint8_t * p) {
         uint16_t u;
         std::memcpy(&u, p, 2);
-        return std::fabs(double(half_to_float_host(u)));
+        return u & 0x7fff;
     };
     double best = 0.0;
-    for (size_t i = 0; i < nb; ++i) {
-        const uint8_t * blk = gguf + i * bb;
-        double t = h(blk) * smax;
-        if (type == T_Q4_1) t += h(blk + 2) * (32.0 * 127);
-        if (!(t <= best)) best = t;  // a NaN scale makes the bound NaN: every launch on it sums in int64
+    if (type == T_Q4_1) {
+        for (size_t i = 0, n = size_t(rows) * size_t(cols / 32); i < n; ++i) {
+            const uint8_t * p = gguf + i * 20;
+            const double t = half_to_float_host(uint16_t(bits(p))) * (32.0 * 15 * 127) +
+                             half_to_float_host(uint16_t(bits(p + 2))) * (32.0 * 127);
+            if (!(t <= best)) best = t;
+        }
+    } else if (type == T_Q4_0 || type == T_Q8_0 || type == T_Q6_K) {  // the largest magnitude by its bits
+        const size_t bb = type == T_Q4_0 ? 18 : type == T_Q8_0 ? 34 : 210, at = type == T_Q6_K ? 208 : 0;
+        int m = 0;
+        for (size_t i = 0, n = size_t(rows) * size_t(cols / (type == T_Q6_K ? 256 : 32)); i < n; ++i)
+            m = std::max(m, bits(gguf + i * bb + at));
+        best = half_to_float_host(uint16_t(m)) *
+               (type == T_Q4_0 ? 32.0 * 8 * 127 : type == T_Q8_0 ? 32.0 * 128 * 127 : 32.0 * 128);
+    } else {
+        return 0.0f;
     }
     return std::nextafter(float(best), INFINITY);
 }
