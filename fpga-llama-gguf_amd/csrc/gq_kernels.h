@@ -296,6 +296,10 @@ constexpr unsigned long long GEMM_KQ_SIZE = 1ull << 24;
 // Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
 constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 : (n_tok + 15) / 16 * 16; }
 constexpr int ATTN_CHUNK = 64;
+// attn_tile_kernel's smallest head_dim (lanes are elements of the values) and token count: it and the combine after it cost
+// a launch more than attn_group_kernel, which is the faster for few tokens at short positions (head_dim 256, position 100:
+// 8 tokens 25 us against 29, 16 tokens 33 against 32, 32 tokens 47 against 38; 128: 28 / 24, 40 / 28, 64 / 34).
+constexpr int ATTN_TILE_HD = 64, ATTN_TILE_TOK = 16;
 constexpr int ATTN_MAXG = 8;  // q heads per KV head
 constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command
 // GDN commands of at least this many tokens form norms and gates in a launch of their own (a launch costs what about

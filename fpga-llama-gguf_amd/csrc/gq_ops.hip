@@ -511,6 +511,81 @@ __device__ __forceinline__ void attn_chunk(const AttnArgs & a, const kv16 (&kr)[
     }
 }
 
+template <bool COH>
+__device__ __forceinline__ float part_get(const float * p) {
+    if constexpr (COH) return part_load(p);
+    else return *p;
+}
+
+// The combine of set th's nc chunks into its output row: M over every chunk, then L and O in chunk order, MAXCH chunks a
+// round (wave 0 forms a round's f_c and l_c in LDS). COH: the partials were stored by other workgroups of this launch.
+template <int HD, bool COH>
+__device__ __forceinline__ void attn_combine(const AttnArgs & a, float & mx, float * fcs, float * lcs, int th, int nc, int nchmax,
+                                             float gt) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, pstride = 2 + HD;
+    const bool el = tid < HD;
+    const int e = el ? tid : 0;
+    const float * pk = a.part + size_t(th) * nchmax * pstride;
+    const int nr0 = min(nc, MAXCH);  // chunks of the first round
+    float ov[CMB];
+    float mc = -__builtin_inff(), lc = 0.0f;
+    if (wave == 0 && lane < nr0) {
+        mc = part_get<COH>(pk + size_t(lane) * pstride);
+        lc = part_get<COH>(pk + size_t(lane) * pstride + 1);
+    }
+#pragma unroll
+    for (int c = 0; c < CMB; ++c) ov[c] = c < nc ? part_get<COH>(pk + size_t(c) * pstride + 2 + e) : 0.0f;
+    if (wave == 0) {
+        float M = mc;
+        for (int r0 = MAXCH; r0 < nc; r0 += MAXCH)  // contexts past MAXCH chunks: the later rounds' maxima
+            M = fmaxf(M, r0 + lane < nc ? part_get<COH>(pk + size_t(r0 + lane) * pstride) : -__builtin_inff());
+#pragma unroll
+        for (int st = 32; st >= 1; st >>= 1) M = fmaxf(M, __shfl_xor(M, st, WAVE));
+        if (lane < nr0) {
+            fcs[lane] = expf_(mc - M);
+            lcs[lane] = lc;
+        }
+        if (lane == 0) mx = M;
+    }
+    __syncthreads();
+    float O = 0.0f, L = 0.0f;
+    for (int r0 = 0;;) {
+        const int rn = min(MAXCH, nc - r0);
+        for (int c0 = 0;;) {  // the round's chunks, CMB value rows a dependent load
+#pragma unroll
+            for (int c = 0; c < CMB; ++c) {
+                if (c0 + c >= rn) break;
+                const float f = fcs[c0 + c];
+                L += lcs[c0 + c] * f;
+                O += ov[c] * f;
+            }
+            c0 += CMB;
+            if (c0 >= rn) break;
+#pragma unroll
+            for (int c = 0; c < CMB; ++c)
+                ov[c] = c0 + c < rn ? part_get<COH>(pk + size_t(r0 + c0 + c) * pstride + 2 + e) : 0.0f;
+        }
+        r0 += MAXCH;
+        if (r0 >= nc) break;
+        const int rn2 = min(MAXCH, nc - r0);
+        __syncthreads();  // every thread has read this round's f_c and l_c
+        if (wave == 0 && lane < rn2) {
+            const float m2 = part_get<COH>(pk + size_t(r0 + lane) * pstride);
+            fcs[lane] = expf_(m2 - mx);
+            lcs[lane] = part_get<COH>(pk + size_t(r0 + lane) * pstride + 1);
+        }
+#pragma unroll
+        for (int c = 0; c < CMB; ++c)
+            ov[c] = c < rn2 ? part_get<COH>(pk + size_t(r0 + c) * pstride + 2 + e) : 0.0f;
+        __syncthreads();
+    }
+    if (el) {
+        float out = O / L;
+        if (a.gate) out = (1.0f / (1.0f + expf_(-gt))) * out;
+        a.y[size_t(th) * HD + e] = out;
+    }
+}
+
 // Steps 3-5 of one token on a loaded chunk (as attn_chunk); the partials go to set th, and the workgroup that
 // completes the set's nc chunks combines them into the output row (and clears the set's counter).
 template <int HD, bool NEW>
@@ -542,67 +617,8 @@ __device__ __forceinline__ void attn_token(const AttnArgs & a, const kv16 (&kr)[
         last = __hip_atomic_fetch_add(a.counter + th, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == unsigned(nc - 1);
     __syncthreads();
     if (!last) return;
-    // ---- 5. combine (last workgroup of the q head): M over every chunk, then L and O in chunk order, MAXCH
-    //      chunks a round (wave 0 forms a round's f_c and l_c in LDS) ----
-    const float * pk = a.part + size_t(th) * nchmax * pstride;
-    const int nr0 = min(nc, MAXCH);  // chunks of the first round
-    float ov[CMB];
-    float mc = -__builtin_inff(), lc = 0.0f;
-    if (wave == 0 && lane < nr0) {
-        mc = part_load(pk + size_t(lane) * pstride);
-        lc = part_load(pk + size_t(lane) * pstride + 1);
-    }
-#pragma unroll
-    for (int c = 0; c < CMB; ++c) ov[c] = c < nc ? part_load(pk + size_t(c) * pstride + 2 + e) : 0.0f;
-    if (wave == 0) {
-        float M = mc;
-        for (int r0 = MAXCH; r0 < nc; r0 += MAXCH)  // contexts past MAXCH chunks: the later rounds' maxima
-            M = fmaxf(M, r0 + lane < nc ? part_load(pk + size_t(r0 + lane) * pstride) : -__builtin_inff());
-#pragma unroll
-        for (int st = 32; st >= 1; st >>= 1) M = fmaxf(M, __shfl_xor(M, st, WAVE));
-        if (lane < nr0) {
-            fcs[lane] = expf_(mc - M);
-            lcs[lane] = lc;
-        }
-        if (lane == 0) mx = M;
-    }
-    __syncthreads();
-    float O = 0.0f, L = 0.0f;
-    for (int r0 = 0;;) {
-        const int rn = min(MAXCH, nc - r0);
-        for (int c0 = 0;;) {  // the round's chunks, CMB value rows a dependent load
-#pragma unroll
-            for (int c = 0; c < CMB; ++c) {
-                if (c0 + c >= rn) break;
-                const float f = fcs[c0 + c];
-                L += lcs[c0 + c] * f;
-                O += ov[c] * f;
-            }
-            c0 += CMB;
-            if (c0 >= rn) break;
-#pragma unroll
-            for (int c = 0; c < CMB; ++c)
-                ov[c] = c0 + c < rn ? part_load(pk + size_t(r0 + c0 + c) * pstride + 2 + e) : 0.0f;
-        }
-        r0 += MAXCH;
-        if (r0 >= nc) break;
-        const int rn2 = min(MAXCH, nc - r0);
-        __syncthreads();  // every thread has read this round's f_c and l_c
-        if (wave == 0 && lane < rn2) {
-            const float m2 = part_load(pk + size_t(r0 + lane) * pstride);
-            fcs[lane] = expf_(m2 - mx);
-            lcs[lane] = part_load(pk + size_t(r0 + lane) * pstride + 1);
-        }
-#pragma unroll
-        for (int c = 0; c < CMB; ++c)
-            ov[c] = c < rn2 ? part_load(pk + size_t(r0 + c) * pstride + 2 + e) : 0.0f;
-        __syncthreads();
-    }
-    if (el) {
-        float out = O / L;
-        if (a.gate) out = (1.0f / (1.0f + expf_(-gt))) * out;
-        a.y[size_t(th) * HD + e] = out;
-    }
+    // ---- 5. combine (last workgroup of the q head) ----
+    attn_combine<HD, true>(a, mx, fcs, lcs, th, nc, nchmax, gt);
     if (tid == 0) a.counter[th] = 0u;
 }
 
@@ -906,8 +922,205 @@ __global__ __launch_bounds__(ATT_T) void attn_group_kernel(AttnArgs a) {
     }
 }
 
+// ---- attention of many tokens of one sequence (after attn_append_kernel) ----
+// A query is a (token, q head) pair, token-major; workgroup (unit, group of NW x QW queries of the unit's KV head), a wave
+// QW queries. Lane i holds key i's score: its products with a query (whose elements are wave-uniform scalars) are
+// added in the pairwise order of the one-token form, so a score costs head_dim products and sums and a 1/QW of the
+// key's conversion, with no exchange between lanes, and a query's chunk maximum and numerators are a wave's own. Then lane
+// e takes over the elements of the values: o in position order for all of the wave's queries, each converted value used
+// QW times. The partials go to their sets; attn_combine_kernel follows. Bound by the FP32 instructions of the products
+// and sums (1024 a query and chunk at head_dim 256, about 1200 executed), where attn_group_kernel spends as many again on
+// conversions and exchanges and idles three of four waves in the softmax: 32 tokens of 16 heads of 256 at positions 100 /
+// 2000 / 8000 take 38 / 63 / 164 us (with append and combine) against its 47 / 139 / 444, a prompt of 1983 tokens 1.3 ms
+// against 4.1.
+constexpr int ATTN_PS = ATTN_CHUNK + 4;  // (+ 4: rows of the numerators on different banks)
+
+template <int HD, int QW, int NW>
+__global__ __launch_bounds__(NW * 64, 4) void attn_tile_kernel(AttnArgs a) {
+    constexpr int TT = NW * 64, QT = NW * QW;
+    constexpr int KP = HD + 8, PER = HD / 8, NP = ATTN_CHUNK * PER / TT, E = HD / 64;
+    __shared__ __align__(16) uint16_t kv[ATTN_CHUNK * KP];  // the keys, then (rows HD long) the values
+    __shared__ __align__(16) float pr[QT * ATTN_PS];
+    const int G = a.n_head / a.n_head_kv, u = blockIdx.x, kvh = u % a.n_head_kv, chunk = u / a.n_head_kv;
+    const int nq = a.n_tok * G, q0 = int(blockIdx.y) * QT, q1 = min(q0 + QT, nq);
+    const int pos0 = *a.pos, t0 = chunk * ATTN_CHUNK;
+    const int first = max(pos0 + q0 / G, 0), plast = min(pos0 + (q1 - 1) / G, a.n_ctx - 1);  // the group's stored positions
+    if (first > plast || t0 > plast) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ntmax = min(ATTN_CHUNK, plast + 1 - t0);
+    kv16 vr[NP];  // rows past ntmax re-read row ntmax - 1 (stored memory); they are not used
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+        const int i = (tid + j * TT) / PER, pc = tid % PER;
+        const size_t off = (size_t(t0 + min(i, ntmax - 1)) * a.n_head_kv + kvh) * HD + pc * 8;
+        *reinterpret_cast<kv16 *>(kv + i * KP + pc * 8) = *reinterpret_cast<const kv16 *>(a.kc + off);
+        vr[j] = *reinterpret_cast<const kv16 *>(a.vc + off);
+    }
+    __syncthreads();
+    // the wave's queries: their rows and the number of this chunk's positions that each attends to (0: none of its own)
+    const int qw = q0 + wave * QW;
+    const __attribute__((address_space(4))) float * qp[QW];  // written by the launch before
+    int nt[QW], th[QW], lo = ATTN_CHUNK, hi = 0;
+#pragma unroll
+    for (int j = 0; j < QW; ++j) {
+        const int qi = min(qw + j, nq - 1), t = qi / G, pos = pos0 + t;
+        th[j] = t * a.n_head + kvh * G + qi % G;
+        qp[j] = (const __attribute__((address_space(4))) float *)(a.qr + size_t(th[j]) * HD);
+        nt[j] = qw + j >= q1 || pos < 0 || pos >= a.n_ctx ? 0 : max(0, min(ATTN_CHUNK, pos + 1 - t0));
+        lo = min(lo, nt[j]);
+        hi = max(hi, nt[j]);
+    }
+    float m[QW];
+    if (hi > 0) {
+        float s[QW], st0[QW], st1[QW];
+#pragma unroll 1
+        for (int it = 0; it < E; ++it) {  // 64 elements, then pairwise over the rounds
+            float lv[3][QW];
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const kv16 kw = *reinterpret_cast<const kv16 *>(kv + lane * KP + it * 64 + b * 8);
+                const uint32_t w[4] = {kw.x, kw.y, kw.z, kw.w};
+                float kf[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) kf[i] = h2f((w[i / 2] >> (16 * (i % 2))) & 0xffffu);
+#pragma unroll
+                for (int j = 0; j < QW; ++j) {
+                    float t[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) t[i] = qp[j][it * 64 + b * 8 + i] * kf[i];
+                    float v = tree<8>(t);
+                    if (b & 1) {
+                        v = lv[0][j] + v;
+                        if (b & 2) {
+                            v = lv[1][j] + v;
+                            if (b & 4) s[j] = lv[2][j] + v;
+                            else lv[2][j] = v;
+                        } else lv[1][j] = v;
+                    } else lv[0][j] = v;
+                }
+            }
+            if (it & 1) {
+#pragma unroll
+                for (int j = 0; j < QW; ++j) s[j] = st0[j] + s[j];
+                if (it & 2) {
+#pragma unroll
+                    for (int j = 0; j < QW; ++j) s[j] = st1[j] + s[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < QW; ++j) st1[j] = s[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < QW; ++j) st0[j] = s[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < QW; ++j) {
+            s[j] = lane < nt[j] ? s[j] * a.scale : -__builtin_inff();
+            m[j] = s[j];
+        }
+#pragma unroll
+        for (int st = 32; st >= 1; st >>= 1)
+#pragma unroll
+            for (int j = 0; j < QW; ++j) m[j] = fmaxf(m[j], __shfl_xor(m[j], st, WAVE));
+#pragma unroll
+        for (int j = 0; j < QW; ++j)
+            pr[(wave * QW + j) * ATTN_PS + lane] = lane < nt[j] ? expf_(s[j] - m[j]) : 0.0f;
+    }
+    __syncthreads();  // every wave has read the keys
+#pragma unroll
+    for (int j = 0; j < NP; ++j) *reinterpret_cast<kv16 *>(kv + (tid + j * TT) * 8) = vr[j];
+    __syncthreads();
+    if (hi == 0) return;
+    const float * pw = pr + wave * QW * ATTN_PS;
+    float o[QW][E];
+#pragma unroll
+    for (int j = 0; j < QW; ++j)
+#pragma unroll
+        for (int k = 0; k < E; ++k) o[j][k] = 0.0f;
+    const auto values = [&](int i, float * v) {
+        const uint16_t * p = kv + i * HD + lane * E;
+        if constexpr (E == 4) {
+            const uint2 w = *reinterpret_cast<const uint2 *>(p);
+            v[0] = h2f(w.x & 0xffffu);
+            v[1] = h2f(w.x >> 16);
+            v[2] = h2f(w.y & 0xffffu);
+            v[3] = h2f(w.y >> 16);
+        } else if constexpr (E == 2) {
+            const uint32_t w = *reinterpret_cast<const uint32_t *>(p);
+            v[0] = h2f(w & 0xffffu);
+            v[1] = h2f(w >> 16);
+        } else {
+            v[0] = h2f(*p);
+        }
+    };
+    if (lo == ATTN_CHUNK) {
+#pragma unroll 1
+        for (int i0 = 0; i0 < ATTN_CHUNK; i0 += 4) {
+            float4 p[QW];
+#pragma unroll
+            for (int j = 0; j < QW; ++j) p[j] = *reinterpret_cast<const float4 *>(pw + j * ATTN_PS + i0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v[E];
+                values(i0 + i, v);
+#pragma unroll
+                for (int j = 0; j < QW; ++j) {
+                    const float pj = i == 0 ? p[j].x : i == 1 ? p[j].y : i == 2 ? p[j].z : p[j].w;
+#pragma unroll
+                    for (int k = 0; k < E; ++k) o[j][k] += pj * v[k];
+                }
+            }
+        }
+    } else {  // the queries' own ends (a value past one, infinite or not, does not enter its sum)
+#pragma unroll 1
+        for (int i = 0; i < hi; ++i) {
+            float v[E];
+            values(i, v);
+#pragma unroll
+            for (int j = 0; j < QW; ++j) {
+                const float pj = pw[j * ATTN_PS + i];
+#pragma unroll
+                for (int k = 0; k < E; ++k) o[j][k] = i < nt[j] ? o[j][k] + pj * v[k] : o[j][k];
+            }
+        }
+    }
+    float l = 0.0f;  // of query lane % QW, in position order (zeros past its end)
+    for (int i = 0; i < ATTN_CHUNK; i += 4) {
+        const float4 p = *reinterpret_cast<const float4 *>(pw + (lane % QW) * ATTN_PS + i);
+        l += p.x;
+        l += p.y;
+        l += p.z;
+        l += p.w;
+    }
+    const int nchmax = (a.n_ctx + ATTN_CHUNK - 1) / ATTN_CHUNK;
+#pragma unroll
+    for (int j = 0; j < QW; ++j) {
+        if (nt[j] == 0) continue;
+        float * pp = a.part + (size_t(th[j]) * nchmax + chunk) * (2 + HD);
+        if (lane == j) *reinterpret_cast<float2 *>(pp) = make_float2(m[j], l);
+        if constexpr (E == 1) {
+            pp[2 + lane] = o[j][0];
+        } else {
+#pragma unroll
+            for (int k = 0; k < E; k += 2) *reinterpret_cast<float2 *>(pp + 2 + lane * E + k) = make_float2(o[j][k], o[j][k + 1]);
+        }
+    }
+}
+
+// Workgroup: one set (token, q head).
+template <int HD>
+__global__ __launch_bounds__(ATT_T) void attn_combine_kernel(AttnArgs a) {
+    __shared__ float mx, fcs[MAXCH], lcs[MAXCH];
+    const int th = blockIdx.x, t = th / a.n_head, hq = th % a.n_head, pos = *a.pos + t;
+    if (pos < 0 || pos >= a.n_ctx) return;
+    const int e = threadIdx.x < HD ? threadIdx.x : 0;
+    const float gt = a.gate ? a.gate[size_t(t) * a.n_head * a.q_stride + size_t(hq) * 2 * HD + e] : 0.0f;
+    attn_combine<HD, false>(a, mx, fcs, lcs, th, (pos + ATTN_CHUNK) / ATTN_CHUNK, (a.n_ctx + ATTN_CHUNK - 1) / ATTN_CHUNK, gt);
+}
+
 // One token: the attention kernel alone. Several: their new keys, values and queries first (one launch), then the
-// attention of every (token, q head, chunk).
+// attention of every (token, q head, chunk): for one sequence's tokens from ATTN_TILE_TOK on as tiles.
 template <int HD>
 hipError_t launch_attn_hd(const AttnArgs & a, dim3 grid, hipStream_t s) {
     if (grid.y == 1) {
@@ -916,6 +1129,22 @@ hipError_t launch_attn_hd(const AttnArgs & a, dim3 grid, hipStream_t s) {
         return hipGetLastError();
     }
     GQ_LAUNCH(attn_append_kernel<HD>, dim3(a.n_head + a.n_head_kv, grid.y), dim3(ATT_T), 0, s, a);
+    const int G = a.n_head / a.n_head_kv;
+    if constexpr (HD >= ATTN_TILE_HD)
+        if (!a.seq_ctx && int(grid.y) >= ATTN_TILE_TOK) {
+            // A prompt chunk's batch: 4 waves of work a SIMD and more at once, so the queries a wave holds pay (7 batches up
+            // to 1983 positions of 16 heads, 256 wide: 1.10 ms at 4 queries x 8 waves, 1.16 at 8 x 8, 1.21 at 8 x 4). A
+            // command's 16 to 32 tokens leave the chip idle at short positions: fewer queries a wave (32 tokens at position
+            // 500: 39 us at 2 x 4, 46 at 4 x 4, 71 at 8 x 8; at 8000 164, 150, 159).
+            const int nq = int(grid.y) * a.n_head / a.n_head_kv, units = int(grid.x) / (a.n_head / a.n_head_kv);
+            if (grid.y > GEMM_MAX_TOK)
+                GQ_LAUNCH((attn_tile_kernel<HD, 4, 8>), dim3(units, (nq + 31) / 32), dim3(512), 0, s, a);
+            else
+                GQ_LAUNCH((attn_tile_kernel<HD, 2, 4>), dim3(units, (nq + 7) / 8), dim3(256), 0, s, a);
+            GQ_LAUNCH(attn_combine_kernel<HD>, dim3(grid.y * a.n_head), dim3(ATT_T), 0, s, a);
+            return hipGetLastError();
+        }
+    if (int(grid.y) * a.n_head > ATTN_MAXG * a.n_head_kv * GEMM_MAX_TOK) return hipErrorInvalidValue;  // the counters
     const int tg = a.seq_ctx ? 1 : ATTN_TG;
     GQ_LAUNCH(attn_group_kernel<HD>, dim3(grid.x, (grid.y + tg - 1) / tg), dim3(ATT_T), 0, s, a);
     return hipGetLastError();
@@ -928,7 +1157,7 @@ hipError_t launch_attn(const AttnArgs & a, hipStream_t s) {
     // (b / (8 G)) 8 + b % 8 (units past the last are idle) and q head (b / 8) % G of its KV head
     const int units = a.n_head_kv * ((a.n_ctx + ATTN_CHUNK - 1) / ATTN_CHUNK);
     const int n_tok = a.n_tok > 1 ? a.n_tok : 1;
-    if (n_tok > GEMM_MAX_TOK || (n_tok > 1 && !a.qr)) return hipErrorInvalidValue;
+    if (n_tok > GEMM_WIDE_TOK || (n_tok > 1 && !a.qr)) return hipErrorInvalidValue;
     const dim3 grid(((units + 7) / 8) * 8 * (a.n_head / a.n_head_kv), n_tok);
     switch (a.head_dim) {
     case 16: return launch_attn_hd<16>(a, grid, s);

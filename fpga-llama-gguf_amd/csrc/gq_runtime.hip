@@ -143,6 +143,9 @@ struct gemvq_ctx {
     float * gdn_prep = nullptr;   // norms and gates of a GDN command's tokens, and the floats it holds; the smaller
     size_t gdn_prep_n = 0;        // buffers before it, which captured graphs may still use
     std::vector<float *> gdn_prep_old;
+    float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens), likewise
+    size_t attn_wide_n = 0;
+    std::vector<float *> attn_wide_old;
     int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
     int arith = GEMVQ_ARITH_CANONICAL;  // the arithmetic lists are compiled in (gemvq_set_arith)
@@ -397,6 +400,12 @@ struct Compiler {
         }
     }
 
+    // The token count in a word's bits from 16 on (8 bits; 16 in the model driver's lists). 0 means 1.
+    uint32_t tokens16(uint32_t word) const {
+        const uint32_t n = (word >> 16) & (c->max_tok > GEMM_MAX_TOK ? 0xffffu : 0xffu);
+        return n ? n : 1;
+    }
+
     // Act ranges the commands i .. i + used - 1 write (a superset is fine: it only costs a snapshot).
     void cmd_writes(const uint32_t * cmds, unsigned n, unsigned i, unsigned used, std::vector<Rng> & wr) const {
         for (unsigned j = i; j < i + used && j < n;) {
@@ -428,13 +437,13 @@ struct Compiler {
                 break;
             }
             case GEMVQ_OP_ATTN: {
-                const uint64_t nt = (k[7] >> 16) & 0xffu ? (k[7] >> 16) & 0xffu : 1;
+                const uint64_t nt = tokens16(k[7]);
                 wr.push_back({k[4], k[4] + uint64_t(k[1] & 0xffffu) * (k[5] & 0xffffu) * nt});
                 step = 2;
                 break;
             }
             case GEMVQ_OP_GET_ROWS: {
-                const uint64_t nt = (k[1] >> 16) & 0xffu ? (k[1] >> 16) & 0xffu : 1;
+                const uint64_t nt = tokens16(k[1]);
                 wr.push_back({k[7], k[7] + uint64_t(k[3]) * nt});
                 break;
             }
@@ -801,8 +810,15 @@ struct Compiler {
                 if (nkv == 0 || nh % nkv || nh / nkv > ATTN_MAXG || int(nkv) != b.n_head_kv || int(hd) != b.head_dim || hd > 256 ||
                     hd < 16 || (hd & (hd - 1)) || nrot > hd || nrot % 2)
                     return reject(i, "ATTN shape");
-                const uint32_t qstride = (flags & 1) ? 2 * hd : hd, ntok = (flags >> 16) & 0xffu ? (flags >> 16) & 0xffu : 1;
-                if (ntok > GEMVQ_GEMM_MAX_TOK) return reject(i, "ATTN tokens");
+                const uint32_t qstride = (flags & 1) ? 2 * hd : hd, ntok = tokens16(flags);
+                // the cache's sets of partials and rotated queries serve GEMM_MAX_TOK tokens of ATTN_MAXG q heads per KV head;
+                // the model driver's lists use them for more tokens of fewer heads, or the context's (gq_attn_tokens)
+                const bool wide = c->max_tok > GEMM_MAX_TOK;
+                const uint32_t tok_sets = ATTN_MAXG * nkv * GEMM_MAX_TOK / std::max(nh, 1u);
+                const bool own = wide && ntok > tok_sets && ntok <= uint32_t(c->max_tok) &&
+                                 attn_wide_floats(b, int(nh), int(ntok)) <= c->attn_wide_n;
+                const uint32_t tok_max = own ? ntok : wide ? tok_sets : GEMVQ_GEMM_MAX_TOK;
+                if (ntok > tok_max) return reject(i, "ATTN tokens");
                 // token t of sequence t: position at pos + 16 t, the cache split into ntok equal regions
                 const bool seqs = (flags & GEMVQ_ATTN_SEQS) && ntok > 1;
                 if (seqs && (b.n_ctx % int(ntok) || !range(k[6], 16ull * (ntok - 1) + 1))) return reject(i, "ATTN sequences");
@@ -824,7 +840,7 @@ struct Compiler {
                 a.y = A(k[4]);
                 a.kc = b.k;
                 a.vc = b.v;
-                a.part = b.part;
+                a.part = own ? c->attn_wide : b.part;
                 a.counter = b.counter;
                 a.n_head = int(nh);
                 a.n_head_kv = int(nkv);
@@ -836,7 +852,7 @@ struct Compiler {
                 a.scale = bits_f(k2[2]);
                 a.eps = bits_f(k2[3]);
                 a.n_tok = int(ntok);
-                a.qr = b.qr;
+                a.qr = own ? c->attn_wide + attn_wide_part(b, int(nh), int(ntok)) : b.qr;
                 if (ref()) {  // the tokens one launch pair each, in order
                     for (uint32_t t = 0; t < ntok; ++t) {
                         out.push_back(LAttn{a, 1, int(t)});
@@ -857,8 +873,7 @@ struct Compiler {
             }
             case GEMVQ_OP_GET_ROWS: {
                 const int type = int(k[1] & 0xffu), rows = int(k[2]), cols = int(k[3]);
-                const uint32_t tw = (k[1] >> 16) & (c->max_tok > GEMM_MAX_TOK ? 0xffffu : 0xffu);
-                const uint32_t ntok = tw ? tw : 1;  // ids 16 floats apart
+                const uint32_t ntok = tokens16(k[1]);  // ids 16 floats apart
                 const uint64_t woff = uint64_t(k[4]) | (uint64_t(k[5]) << 32);
                 if (type != T_Q6_K && type != T_Q4_0 && type != T_Q8_0) return reject(i, "GET_ROWS type");
                 if (ntok > uint32_t(c->max_tok)) return reject(i, "GET_ROWS tokens");
@@ -929,6 +944,15 @@ struct Compiler {
             ++i;
         }
         return true;
+    }
+
+    // Floats of the partials of n_tok tokens, and with their rotated queries behind them.
+    static size_t attn_wide_part(const KvBuf & b, int n_head, int n_tok) {
+        const size_t nch = size_t(b.n_ctx + ATTN_CHUNK - 1) / ATTN_CHUNK;
+        return (size_t(n_tok) * n_head * nch * (2 + b.head_dim) + 63) & ~size_t(63);
+    }
+    static size_t attn_wide_floats(const KvBuf & b, int n_head, int n_tok) {
+        return attn_wide_part(b, n_head, n_tok) + size_t(n_tok) * n_head * b.head_dim;
     }
 
     // A buffer of n floats for the norms and gates of a GDN command's tokens; NULL (they are formed in the step) without
@@ -1589,6 +1613,8 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->wide);
     hipFree(c->gdn_prep);
     for (float * p : c->gdn_prep_old) hipFree(p);
+    hipFree(c->attn_wide);
+    for (float * p : c->attn_wide_old) hipFree(p);
     hipFree(c->ref_x);
     hipFree(c->dbg);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -1814,7 +1840,7 @@ int gemvq_run(gemvq_ctx * c, const uint32_t * cmds, unsigned n) {
     return e == hipSuccess ? 0 : fail(c, e, "run");
 }
 
-// Whether the lists compiled from now on may hold commands of up to GEMM_WIDE_TOK tokens (GEMM, CONV, GDN, GET_ROWS): for
+// Whether the lists compiled from now on may hold commands of up to GEMM_WIDE_TOK tokens (GEMM, CONV, GDN, GET_ROWS; ATTN: gq_attn_tokens): for
 // the prompt chunks of the model driver, which switches it on around its own lists. A caller's lists keep the limits of
 // the header.
 __attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int on) {
@@ -1830,6 +1856,33 @@ __attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int on) {
     }
     c->max_tok = on ? GEMM_WIDE_TOK : GEMM_MAX_TOK;
     return 0;
+}
+
+// Tokens (a multiple of 32, at most `most`) that one ATTN command of such a list may hold on cache kv: what 256 MiB of
+// partials serve, the memory-side cache's size, so that the combine reads them back from there; without memory for that,
+// or where that is no more, what the cache's own sets serve. Attention runs in order, so the layers share one buffer.
+__attribute__((visibility("hidden"))) int gq_attn_tokens(gemvq_ctx * c, int kv, int n_head, int most) {
+    if (!c || kv < 0 || size_t(kv) >= c->kvs.size() || n_head < 1) return GEMVQ_EINVAL;
+    const KvBuf & b = c->kvs[size_t(kv)];
+    most = std::min(most, GEMM_WIDE_TOK) & ~31;
+    const int sets = std::min(most, (ATTN_MAXG * b.n_head_kv * GEMM_MAX_TOK / n_head) & ~31);
+    if (b.head_dim < ATTN_TILE_HD || !c->usable) return std::max(sets, 32);
+    int tok = most;
+    while (tok > sets && Compiler::attn_wide_floats(b, n_head, tok) > (size_t(64) << 20)) tok -= 32;
+    if (tok <= sets) return std::max(sets, 32);
+    const size_t n = Compiler::attn_wide_floats(b, n_head, tok);
+    if (c->attn_wide_n < n) {
+        hipSetDevice(c->device);
+        float * p = nullptr;
+        if (hipMalloc(&p, n * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            return std::max(sets, 32);
+        }
+        if (c->attn_wide) c->attn_wide_old.push_back(c->attn_wide);
+        c->attn_wide = p;
+        c->attn_wide_n = n;
+    }
+    return tok;
 }
 
 int gemvq_graph_create(gemvq_ctx * c, const uint32_t * cmds, unsigned n, int * graph) {

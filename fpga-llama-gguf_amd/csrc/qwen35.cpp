@@ -48,7 +48,9 @@ struct gemvq_qwen35 {
     std::map<std::string, T> t;
     std::vector<uint32_t> cmds;
     int graph = -1;
+    uint32_t attn_batch = GEMVQ_GEMM_MAX_TOK;  // tokens of a prompt chunk's ATTN commands
     int chunk_graph = -1;  // the prefill's full-chunk command list (positions and ids come from the act slots)
+    int chunk_graph_tok = 0;
     std::vector<int> kv;  // per layer (attention layers only)
     // activation layout
     uint32_t tok = 16, pos = 32, key = 48;
@@ -218,10 +220,12 @@ bool build_chunk(const gemvq_qwen35 & m, uint32_t ntok, std::vector<uint32_t> & 
             e.gemm(*W(p + "attn_q.weight"), m.bh, E, m.bqg, qrow, ntok, 0, 0, 0, an, eps);
             e.gemm(*W(p + "attn_k.weight"), m.bh, E, m.bk, kvrow, ntok, 0, 0, 0, an, eps);
             e.gemm(*W(p + "attn_v.weight"), m.bh, E, m.bv, kvrow, ntok, 0, 0, 0, an, eps);
-            // batches of up to GEMVQ_GEMM_MAX_TOK of the chunk's tokens, batch b's at positions act[bpos + 16 b] + i, packed
-            // rows (q + gate, k, v, output)
-            for (uint32_t t0 = 0; t0 < ntok; t0 += GEMVQ_GEMM_MAX_TOK) {
-                const uint32_t nt = std::min(GEMVQ_GEMM_MAX_TOK, ntok - t0);
+            // batches of the chunk's tokens, as many as the attention's scratch serves: a longer batch fills the chip and starts
+            // launches less often. The batch from token t0 is at positions act[bpos + 16 (t0 / 32)] + i, packed rows (q +
+            // gate, k, v, output).
+            const uint32_t batch = m.attn_batch;
+            for (uint32_t t0 = 0; t0 < ntok; t0 += batch) {
+                const uint32_t nt = std::min(batch, ntok - t0);
                 e.cmd({GEMVQ_OP_ATTN, uint32_t(c.n_head) | (uint32_t(c.n_head_kv) << 16), m.bqg + t0 * qrow, uint32_t(m.kv[il]),
                        m.batt + t0 * arow, hd | (uint32_t(c.n_rot) << 16), m.bpos + t0 / GEMVQ_GEMM_MAX_TOK * 16, 1u | (nt << 16)});
                 e.cmd({m.bk + t0 * kvrow, m.bv + t0 * kvrow, fb(1.0f / std::sqrt(float(c.head_dim))), fb(eps),
@@ -396,6 +400,7 @@ bool build_commands(gemvq_qwen35 & m, std::string & err) {
 
 extern "C" void gq_set_error(gemvq_ctx * ctx, const char * what);  // gq_runtime.hip
 extern "C" int gq_wide_lists(gemvq_ctx * ctx, int on);
+extern "C" int gq_attn_tokens(gemvq_ctx * ctx, int kv, int n_head, int most);
 
 namespace {
 int set_err(gemvq_ctx * ctx, const std::string & what) {
@@ -554,7 +559,15 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
     if (pos < 0 || pos + n > np - 1) return set_err(ctx, "gemvq_qwen35_prefill: positions past the last prompt token but one");
     // chunks of the layout's rows; the reference arithmetic runs its commands token by token and keeps their limit
     const int most = gemvq_arith(ctx) == GEMVQ_ARITH_REFERENCE ? int(GEMVQ_GEMM_MAX_TOK) : int(m->chunk);
-    if (most > int(GEMVQ_GEMM_MAX_TOK)) st = gq_wide_lists(ctx, 1);
+    m->attn_batch = GEMVQ_GEMM_MAX_TOK;
+    if (most > int(GEMVQ_GEMM_MAX_TOK)) {
+        st = gq_wide_lists(ctx, 1);
+        for (int il = 0; il < m->c.n_layer; ++il)  // (the layers' caches are alike)
+            if (is_attn(m->c, il)) {
+                m->attn_batch = uint32_t(std::max(gq_attn_tokens(ctx, m->kv[il], m->c.n_head, most), int(GEMVQ_GEMM_MAX_TOK)));
+                break;
+            }
+    }
     std::vector<uint32_t> w;
     for (int p0 = pos; p0 < pos + n && !st;) {
         const int nt = std::min<int>(most, pos + n - p0);
@@ -566,8 +579,13 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
         if (!st) st = gemvq_act_write(ctx, m->bpos, first.data(), first.size());
         if (!st && nt == most) {
             // full chunks replay one captured list: it reads the chunk's ids and positions from the slots just written
-            // (the write waits for the previous replay; the replay follows it on the same stream)
+            // (the writes, the previous replay before them and this one run in order on the same stream)
+            if (m->chunk_graph >= 0 && m->chunk_graph_tok != most) {  // the arithmetic was switched: other chunks
+                gemvq_graph_destroy(ctx, m->chunk_graph);
+                m->chunk_graph = -1;
+            }
             if (m->chunk_graph < 0) {
+                m->chunk_graph_tok = most;
                 w.clear();
                 build_chunk(*m, uint32_t(most), w);
                 st = gemvq_graph_create(ctx, w.data(), unsigned(w.size() / GEMVQ_CMD_WORDS), &m->chunk_graph);

@@ -234,6 +234,55 @@ def test_gdn_tokens_gated_norm_then_gemm(gq, orc, hv, hk, wtype, z_silu, ntok, s
         ctx.close()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,n_ctx,p0,ntok", [
+    (16, 4, 256, 192, 64, 16),   # the first token count of the tiles; the chunk's start to its middle
+    (16, 4, 256, 192, 48, 17),   # up to the chunk's last position and one more
+    (3, 1, 64, 130, 100, 31),    # queries past the last full tile, a position past the capacity
+    (8, 8, 128, 300, 120, 32),   # one q head per KV head
+    (6, 2, 64, 4200, 4160, 20),  # 66 chunks: two rounds in the combine
+])
+def test_attention_tiles_at_infinite_values(gq, ctx, nh, nkv, hd, n_ctx, p0, ntok):
+    """Token counts of the tiled attention against one-token commands on a second cache, bit for bit, with values of a late
+    token beyond FP16's range: they are stored as infinities and enter no earlier token's sums."""
+    kvs = ctx.kv_create(n_ctx, nkv, hd), ctx.kv_create(n_ctx, nkv, hd)
+    qrow, kvrow, arow, nrot = 2 * nh * hd, nkv * hd, nh * hd, hd // 4
+    O, at = {}, 0
+    for name, size in dict(q=ntok * qrow, k=ntok * kvrow, v=ntok * kvrow, qn=hd, kn=hd, pos=16 * ntok, y=ntok * arow,
+                           y2=ntok * arow, cs=n_ctx * nrot).items():
+        O[name], at = at, at + up16_(size)
+    ctx.write(O["qn"], gq.uniform(2, 1, hd, 0.5, 1.5))
+    ctx.write(O["kn"], gq.uniform(2, 2, hd, 0.5, 1.5))
+    ctx.write(O["cs"], gq.uniform(2, 3, n_ctx * nrot, -1.0, 1.0))
+
+    def attn(kv, t, n, y):
+        return gq.attn(nh, nkv, O["q"] + t * qrow, kv, y, hd, nrot, O["pos"] + 16 * t, O["k"] + t * kvrow,
+                       O["v"] + t * kvrow, 1 / 16, 1e-6, O["qn"], O["kn"], O["cs"], gate=O["q"] + t * qrow + hd, n_tok=n)
+
+    def tokens(first, n):
+        v = gq.normal(4, first + 2, n * kvrow)
+        v[(n - 3) * kvrow:(n - 2) * kvrow:7] = 1e6
+        ctx.write(O["q"], gq.normal(4, first, n * qrow))
+        ctx.write(O["k"], gq.normal(4, first + 1, n * kvrow) * 3)
+        ctx.write(O["v"], v if first == p0 else gq.normal(4, first + 3, n * kvrow))
+        slots = np.zeros(16 * ntok, np.int32)
+        slots[0:16 * n:16] = np.arange(first, first + n)
+        ctx.write(O["pos"], slots)
+
+    for b0 in range(0, p0, 15):  # the same history in both caches
+        n = min(15, p0 - b0)
+        tokens(b0, n)
+        assert ctx.run(sum((attn(kv, 0, n, O["y"]) for kv in kvs), [])) == 0, ctx.error()
+    tokens(p0, ntok)
+    sentinel = np.full(ntok * arow, -7.25, np.float32)
+    ctx.write(O["y"], sentinel)
+    ctx.write(O["y2"], sentinel)
+    assert ctx.run(sum((attn(kvs[0], t, 1, O["y"] + t * arow) for t in range(ntok)), [])) == 0, ctx.error()
+    assert ctx.run(attn(kvs[1], 0, ntok, O["y2"])) == 0, ctx.error()
+    one, tiled = ctx.read(O["y"], ntok * arow), ctx.read(O["y2"], ntok * arow)
+    assert_bits(tiled, one, "tiled vs one-token outputs")
+    assert np.isfinite(one[:(ntok - 3) * arow]).all()
+
+
 def up16_(n: int) -> int:
     return (n + 15) // 16 * 16
 
