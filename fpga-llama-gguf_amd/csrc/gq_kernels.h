@@ -290,7 +290,10 @@ struct TokArgs {
 constexpr int GEMV_MAXK = 16384;  // GEMV columns at most
 constexpr int GEMM_MAX_TOK = 32;  // tokens of one GEMM command (two tiles of 16)
 constexpr int GEMM_WIDE_TOK = 512;  // tokens of a batched GEMV in the model driver's own lists (prompt chunks)
-// Q6_K GEMMs of at least this many tokens and weights take the matrix-core form, the others the small-token GEMV.
+// Q6_K GEMMs of at least this many tokens and weights take the matrix-core form, the others the small-token GEMV in launches
+// of up to 4 tokens (4096 x 4096, us at 2 / 3 / 4 / 8 / 32 tokens, quantization included: 17.6 / 17.5 / 17.3 / 17.4 / 19.7
+// against 18.5 / 23.4 / 25.8 / 46.3 / 169; 8192 x 4096 at 2 tokens 21.9 against 20.3). Below 2^24 weights, less than an
+// output head has, the difference at 3 and 4 tokens is 1 to 5 us, and the small-token form's launch counts are kept.
 constexpr unsigned GEMM_KQ_TOK = 3;
 constexpr unsigned long long GEMM_KQ_SIZE = 1ull << 24;
 // Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
@@ -302,8 +305,8 @@ constexpr int ATTN_CHUNK = 64;
 constexpr int ATTN_TILE_HD = 64, ATTN_TILE_TOK = 16;
 constexpr int ATTN_MAXG = 8;  // q heads per KV head
 constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command
-// GDN commands of at least this many tokens form norms and gates in a launch of their own (a launch costs what about
-// three tokens do in the step).
+// GDN commands of at least this many tokens form norms and gates in a launch of their own (32 value heads, us in a graph at
+// 6 / 8 / 10 / 16 / 32 tokens: 15.8 / 16.0 / 16.0 / 17.5 / 23.8 against 15.3 / 16.3 / 18.5 / 25.4 / 43.6 in the step).
 constexpr unsigned GDN_PREP_TOK = 8;
 
 // Profiling: when set (by gemvq_profile on the calling thread), launchers start kernels through

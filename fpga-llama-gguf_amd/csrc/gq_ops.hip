@@ -106,7 +106,8 @@ __global__ void conv_kernel(ConvArgs a) {
 // The same for the tokens of one sequence, x and y apart: the outputs do not wait for each other (a window holds inputs
 // only), so grid y takes CONV_SEG tokens each instead of one thread walking through all of a channel's. The threads of
 // the first segment, which alone read the old state, store the new one (it may be the same memory); n_tok >= CONV_SEG.
-// 31 tokens of 8192 channels took 8.6 us in one thread per channel.
+// 31 tokens of 8192 channels took 8.6 us in one thread per channel, 512 take 10.2 us here; up to 32 tokens alone in a graph
+// the two forms are even (15 us, the graph's own).
 constexpr int CONV_SEG = 8;
 __global__ __launch_bounds__(256) void conv_tokens_kernel(ConvArgs a) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, t0 = blockIdx.y * CONV_SEG;

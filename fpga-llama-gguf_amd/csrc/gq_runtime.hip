@@ -987,7 +987,7 @@ struct Compiler {
         const uint32_t * k = cmds + size_t(i) * GEMVQ_CMD_WORDS, * k2 = k + GEMVQ_CMD_WORDS;
         const int t = int(k[1] & 0xffu), rows = int(k[2]);
         const uint32_t flags = k[1] & ~0xffu, cols = k[3], ntok = k2[0], xs = k2[1], ys = k2[2], nflags = k2[7];
-        const bool kq = t == T_Q5_K || t == T_Q6_K;  // launches of up to 4 tokens of the small-token GEMV, or for Q6_K (k_mfma) MFMA
+        const bool kq = t == T_Q5_K || t == T_Q6_K;  // the small-token GEMV, or for Q6_K (k_mfma) MFMA
         if (t != T_Q4_0 && t != T_Q4_1 && t != T_Q8_0 && !kq) return reject(i, "GEMM format (Q4_0, Q4_1, Q8_0, Q5_K or Q6_K)");
         if (rows <= 0 || cols == 0 || cols % 512 || cols > GEMVQ_MAX_COLS) return reject(i, "GEMM shape (cols a multiple of 512)");
         if (flags & ~(GEMVQ_GEMV_SWIGLU | GEMVQ_GEMV_ADD | GEMVQ_GEMV_SILU) || __builtin_popcount(flags) > 1)

@@ -91,7 +91,7 @@
  *             x_off + t * x_stride and its output row at y_off + t * y_stride; each output row equals, bit for bit,
  *             what a GEMV command on that token row writes. Format 2 Q4_0, 3 Q4_1 or 8 Q8_0, cols a multiple of
  *             512; or 13 Q5_K or 14 Q6_K with cols a multiple of 512 up to 12288, no SwiGLU pair, and y not over x
- *             or the norm weight (these run in launches of up to 4 tokens, each reading the weights once).
+ *             or the norm weight (Q5_K, and Q6_K of up to 2 tokens or below 2^24 weights, in launches of up to 4 tokens).
  *             flags: GEMVQ_GEMV_SWIGLU (the next command is the u GEMM with the same format, rows, cols, x_off,
  *             n_tok, x_stride and norm words and no flags; y = silu(g) * u goes to the u command's y_off /
  *             y_stride), GEMVQ_GEMV_ADD (y = W x + res, token t's residual at res_off + t * res_stride) or
@@ -193,6 +193,7 @@ int gemvq_repack(int type, int rows, int cols, const void * gguf_rows, void * ds
 int gemvq_unpack(int type, int rows, int cols, const void * packed, void * gguf_rows);
 
 /* Activation buffer I/O (offsets and counts in floats; int32 data may be written through the same calls). */
+/* A write has taken src over when it returns; the device sees it before any work of a later call. */
 int gemvq_act_write(gemvq_ctx * ctx, size_t off, const void * src, size_t n);
 int gemvq_act_read(gemvq_ctx * ctx, size_t off, void * dst, size_t n);
 /* GDN state rows (128 floats each). */

@@ -374,3 +374,28 @@ def test_gemm_tiles_and_held_steps(gq, orc, ctx, fmt, rows, cols, ntok):
     for t in sorted({0, ntok // 2, ntok - 1}):
         want = orc.fx_gemv(fmt, w[:min(rows, 512) * gq.row_bytes(fmt, cols)], x[t * cols:(t + 1) * cols], min(rows, 512), cols)
         assert_bits(y[t], np.resize(want, rows), f"token {t}")
+
+
+@pytest.mark.parametrize("rows,cols,ntok,scale", [
+    (4096, 4096, 2, 1.0), (4095, 4096, 3, 1.0), (4096, 4096, 3, 1.0),  # both sides of the rule on tokens and on weights
+    (8209, 4096, 17, 1.0), (2064, 8192, 16, 1.0),  # a partial row tile, two token tiles; one full token tile
+    (1400, 12288, 32, 1.0), (33000, 512, 7, 1.0),  # the widest held steps, waves without a step
+    (4099, 4096, 5, 3e4), (4099, 4096, 20, 1e-7),  # terms summed in int64; terms that floor to 0 and -1
+])
+def test_q6_k_gemm_on_the_matrix_cores(gq, orc, rows, cols, ntok, scale):
+    """Q6_K rows of many weights and tokens, one activation far above the others: every token row bit for bit."""
+    w = gq.matrix(14, min(rows, 512), cols, 5, 30)
+    x = gq.normal(5, 31, ntok * cols) * np.float32(scale)
+    x[5] *= 300
+    ys = up16(rows)
+    X, Y = 0, ntok * cols
+    packed = np.resize(w, rows * gq.row_bytes(14, cols))
+    with gq.Context(act_floats=up16(Y + ntok * ys), weight_bytes=packed.size + 4096) as ctx:
+        off = ctx.upload(14, rows, cols, packed)
+        ctx.write(X, x)
+        print(f"[gemm] Q6_K rows {rows} cols {cols} tokens {ntok}", flush=True)
+        assert ctx.run(gq.gemm(14, rows, cols, off, X, Y, ntok, cols, ys)) == 0, ctx.error()
+        y = ctx.read(Y, ntok * ys).reshape(ntok, ys)[:, :rows]
+    for t in range(ntok):
+        want = orc.fx_gemv(14, w, x[t * cols:(t + 1) * cols], min(rows, 512), cols)
+        assert_bits(y[t], np.resize(want, rows), f"token {t}")

@@ -234,6 +234,62 @@ def test_gdn_tokens_gated_norm_then_gemm(gq, orc, hv, hk, wtype, z_silu, ntok, s
         ctx.close()
 
 
+@pytest.mark.parametrize("ch,ntok,apart", [(272, 7, True), (272, 8, True), (8192, 9, True), (528, 32, True), (272, 16, False)])
+def test_conv_tokens(gq, orc, ctx, ch, ntok, apart):
+    """A CONV of several tokens of one sequence around the token-parallel form's first count and segment edges, into rows
+    of its own and (apart False) in place: outputs and the new state (stored over the old) are the oracle's."""
+    st, x, w = gq.normal(3, 1, 3 * ch), gq.normal(3, 2, ntok * ch), gq.normal(3, 3, 4 * ch) * 0.5
+    X, W, S = 0, up16_(ntok * ch), up16_(ntok * ch) + 4 * ch
+    Y = S + 4 * ch if apart else X
+    for off, arr in ((X, x), (W, w), (S, st)):
+        ctx.write(off, arr)
+    c = gq.conv(ch, X, W, Y, S, S, silu=True)
+    c[7] |= ntok << 16
+    assert ctx.run(c) == 0, ctx.error()
+    want = []
+    for t in range(ntok):
+        y, st = orc.conv(st, x[t * ch:(t + 1) * ch], w, silu=True)
+        want.append(y)
+    assert_bits(ctx.read(Y, ntok * ch), np.concatenate(want), "conv rows")
+    assert_bits(ctx.read(S, 3 * ch), st, "conv state")
+
+
+@pytest.mark.parametrize("hv,hk,ntok,l2,gated", [(4, 2, 7, True, True), (4, 2, 8, True, True), (32, 16, 32, True, False),
+                                                 (2, 1, 9, False, True), (6, 3, 31, False, False)])
+def test_gdn_tokens_norms_ahead(gq, orc, hv, hk, ntok, l2, gated):
+    """A GDN of several tokens of one sequence on both sides of the count from which L2 norms and gates are formed ahead of
+    the recurrence, with and without L2 norms and output norm: rows and state equal the oracle's tokens in order."""
+    S = 128
+    flags = gq.GDN_GATES | (gq.GDN_L2_QK if l2 else 0) | (gq.GDN_GATED if gated else 0)
+    cols, sg = hv * S, up16_(hv)
+    q, k, v, z = (gq.normal(8, i, ntok * cols) for i in range(1, 5))
+    if not l2:  # as the model's, so that the state stays bounded
+        q, k = ((u.reshape(-1, S) / np.linalg.norm(u.reshape(-1, S), axis=1, keepdims=True)).ravel() for u in (q, k))
+    g, beta = gq.normal(8, 5, ntok * sg), gq.normal(8, 6, ntok * sg)
+    dt, a, w = gq.normal(8, 7, hv), -np.abs(gq.normal(8, 8, hv)), gq.uniform(8, 9, S, 0.5, 1.5)
+    st = gq.normal(8, 10, hv * S * S) * 0.1
+    O, at = {}, 0
+    for name, size in dict(q=ntok * cols, k=ntok * cols, v=ntok * cols, z=ntok * cols, g=ntok * sg, beta=ntok * sg, dt=hv,
+                           a=hv, w=S, y=ntok * cols).items():
+        O[name], at = at, at + up16_(size)
+    with gq.Context(act_floats=at, weight_bytes=1 << 16, state_rows=hv * S) as ctx:
+        for name, arr in dict(q=q, k=k, v=v, z=z, g=g, beta=beta, dt=dt, a=a, w=w).items():
+            ctx.write(O[name], arr)
+        ctx.state_write(0, st)
+        c = gq.gdn(hv, hk, O["q"], O["k"], O["v"], O["g"], O["beta"], O["y"], 0, 0, 1 / np.sqrt(S), flags, 1e-6, 1e-6, O["w"],
+                   O["z"], O["dt"], O["a"])
+        c[16 + 2:16 + 5] = [ntok, cols, sg]
+        assert ctx.run(c) == 0, ctx.error()
+        want = []
+        for t in range(ntok):
+            n, row, gb = hk * S, slice(t * cols, (t + 1) * cols), slice(t * sg, t * sg + hv)
+            y, st = orc.gdn(st, q[t * cols:t * cols + n], k[t * cols:t * cols + n], v[row], g[gb], beta[gb], hv, hk,
+                            float(1 / np.sqrt(S)), flags, dt, a, z[row], w)
+            want.append(y)
+        assert_bits(ctx.read(O["y"], ntok * cols), np.concatenate(want), "rows")
+        assert_bits(ctx.state_read(0, hv * S), st, "state")
+
+
 @pytest.mark.parametrize("nh,nkv,hd,n_ctx,p0,ntok", [
     (16, 4, 256, 192, 64, 16),   # the first token count of the tiles; the chunk's start to its middle
     (16, 4, 256, 192, 48, 17),   # up to the chunk's last position and one more
