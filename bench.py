@@ -508,7 +508,7 @@ def main() -> int:
             t_pre = time.perf_counter() - t
             prefill = {"positions": args.prompt - 1, "batched_tokens_per_s": round((args.prompt - 1) / t_pre, 1),
                        "decode_step_tokens_per_s": round((args.prompt - 1) / t_steps, 1),
-                       "method": "chunks of 32 tokens: GEMM projections, conv and DeltaNet over the tokens in order, "
+                       "method": "chunks of up to 512 tokens: GEMM projections, conv and DeltaNet over the tokens in order, "
                                  "attention over the chunk's tokens in one launch pair; full chunks replay one "
                                  "captured graph (captured by an untimed first prefill); wall time of the whole "
                                  "prefill call"}
