@@ -296,6 +296,11 @@ constexpr int GEMM_WIDE_TOK = 512;  // tokens of a batched GEMV in the model dri
 // output head has, the difference at 3 and 4 tokens is 1 to 5 us, and the small-token form's launch counts are kept.
 constexpr unsigned GEMM_KQ_TOK = 3;
 constexpr unsigned long long GEMM_KQ_SIZE = 1ull << 24;
+// Q4_0 SwiGLU pairs of 3 and 4 tokens: from this many weights a matrix on the matrix cores with their quantization launch (us
+// at 3 / 4 tokens: 9728 x 2560 15.1 / 15.1 against 16.6 / 18.0, 12288 x 4096 19.8 / 19.6 against 20.6 / 22.3, 4096 x 4096
+// 11.7 / 11.8 against 12.0 / 12.8). Q8_0 stays on the small-token GEMV (9728 x 2560 19.9 / 19.9 against 18.0 / 19.8).
+constexpr unsigned GEMM_PAIR_TOK = 3;
+constexpr unsigned long long GEMM_PAIR_SIZE = 1ull << 24;
 // Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
 constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 : (n_tok + 15) / 16 * 16; }
 constexpr int ATTN_CHUNK = 64;

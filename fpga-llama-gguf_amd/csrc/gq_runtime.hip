@@ -1048,7 +1048,8 @@ struct Compiler {
         if (kq && over && !ref()) return reject(i, "GEMM on K-quant weights: the output falls on the input rows or the norm weight");
         if (ref()) return gemm_ref(g, t, k, k2, over, normw, i, used);
         const bool k_mfma = t == T_Q6_K && ntok >= GEMM_KQ_TOK && uint64_t(rows) * cols >= GEMM_KQ_SIZE;
-        if ((kq && !k_mfma) || (!kq && !over && gemv_tok_ok(t, int(cols), int(ntok), g.epi == EPI_SWIGLU))) {
+        const bool pair_mfma = t == T_Q4_0 && g.epi == EPI_SWIGLU && ntok >= GEMM_PAIR_TOK && uint64_t(rows) * cols >= GEMM_PAIR_SIZE;
+        if ((kq && !k_mfma) || (!kq && !over && !pair_mfma && gemv_tok_ok(t, int(cols), int(ntok), g.epi == EPI_SWIGLU))) {
             const uint32_t cs = kq ? (gemv_tok_ok(t, int(cols), TOK_MAX, false) ? TOK_MAX : 2) : ntok;  // tokens a launch
             for (uint32_t c0 = 0; c0 < ntok; c0 += cs) {
                 const uint32_t nt = std::min(cs, ntok - c0);

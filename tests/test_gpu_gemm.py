@@ -399,3 +399,22 @@ def test_q6_k_gemm_on_the_matrix_cores(gq, orc, rows, cols, ntok, scale):
     for t in range(ntok):
         want = orc.fx_gemv(14, w, x[t * cols:(t + 1) * cols], min(rows, 512), cols)
         assert_bits(y[t], np.resize(want, rows), f"token {t}")
+
+
+@pytest.mark.parametrize("fmt", [2, 8])
+@pytest.mark.parametrize("rows,ntok", [(4096, 2), (4095, 4), (4096, 3), (4096, 4)])
+def test_small_token_pair_of_many_weights(gq, orc, ctx, fmt, rows, ntok):
+    """SwiGLU pairs on both sides of the rule that hands few tokens and many weights to the matrix cores: bit for bit."""
+    cols, pool, ys = 4096, 256, up16(rows)
+    wg, wu = (gq.matrix(fmt, pool, cols, 5, 80 + i, std=0.02) for i in (0, 1))
+    off = [ctx.upload(fmt, rows, cols, np.resize(w, rows * gq.row_bytes(fmt, cols))) for w in (wg, wu)]
+    x = gq.normal(5, 82, ntok * cols)
+    Y, YG = ntok * cols, ntok * (cols + ys)
+    ctx.write(0, x)
+    cmd = (gq.gemm(fmt, rows, cols, off[0], 0, YG, ntok, cols, ys, gq.GEMV_SWIGLU) +
+           gq.gemm(fmt, rows, cols, off[1], 0, Y, ntok, cols, ys))
+    assert ctx.run(cmd) == 0, ctx.error()
+    y = ctx.read(Y, ntok * ys).reshape(ntok, ys)[:, :rows]
+    for t in range(ntok):
+        g, u = (orc.fx_gemv(fmt, w, x[t * cols:(t + 1) * cols], pool, cols) for w in (wg, wu))
+        assert_bits(y[t], np.resize(orc.silu_mul(g, u), rows), f"token {t}")
