@@ -13,6 +13,10 @@ constexpr int WAVE = 64;
 // conversion; fp16 denormals are preserved in the default mode), NaN stays NaN.
 __device__ __forceinline__ float h2f(uint32_t h) { return float(__builtin_bit_cast(_Float16, uint16_t(h))); }
 
+// An fp16 sum as the fixed-point terms take it: an infinity is 2^16, its exponent field taken as any other
+// (gemvqw_engine.h:373-383).
+__device__ __forceinline__ float h2f_fixed(uint32_t h) { return __builtin_amdgcn_fmed3f(h2f(h), -65536.0f, 65536.0f); }
+
 // binary32 -> binary16, round to nearest even, subnormal results rounded, overflow to infinity (gemvq_ref.h:32-52):
 // the hardware conversion in the default rounding mode, of the binary32 value. The empty asm makes that value exist:
 // without it the compiler may fold a product into the conversion (v_fma_mixlo_f16, one rounding of the exact

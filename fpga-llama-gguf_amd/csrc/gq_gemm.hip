@@ -61,7 +61,9 @@ __device__ __forceinline__ size_t act_bound(int tok, int ns, int step) {
 // Workgroup t quantizes token t exactly as the single-token prologue: thread i holds the 16-float items i, i + NT,
 // ... (the two halves of a block in adjacent lanes), the norm scale is the canonical pairwise tree over the row, and
 // v = (x * scale) * w. Beside each step of 16 blocks goes its part of the term bound: the sum over the blocks of
-// d_x * 2^40 * (sum of |quants|) / (32 * 127), which times a matrix's wbound bounds the step's terms.
+// d_x * 2^40 * (sum of |quants|) / (32 * 127), which times a matrix's wbound bounds the step's terms; infinite where a block's
+// Q8_1 sum is (its values together past the largest fp16, its scale finite): in the FP16 product the zeros beside such a sum
+// would become NaNs, so that these steps go to step_terms_exact, whatever the format.
 __global__ __launch_bounds__(NT) void gemm_quant_kernel(GemmQuantArgs a) {
     __shared__ Lds s;
     const int tok = blockIdx.x, nb = a.cols / 32, ns = nb / GS, n16 = a.cols / 16;
@@ -98,12 +100,13 @@ __global__ __launch_bounds__(NT) void gemm_quant_kernel(GemmQuantArgs a) {
             *reinterpret_cast<uint32_t *>(q + act_group(tok, g, ns, b) + 4 * h) = packed[g];
             mag = __builtin_amdgcn_sad_u8(packed[g] ^ 0x80808080u, 0x80808080u, mag);  // |q + 128 - 128| per byte
         }
-        const uint32_t dh = f2h(d);
+        const uint32_t dh = f2h(d), sh = f2h(float(sum) * d);
         if (h == 0) {
             a.d[act_scale(tok, ns, b)] = uint16_t(dh);
-            a.s[act_scale(tok, ns, b)] = uint16_t(f2h(float(sum) * d));  // ggml quantize_row_q8_1: fp16(sum * d)
+            a.s[act_scale(tok, ns, b)] = uint16_t(sh);  // ggml quantize_row_q8_1: fp16(sum * d)
         }
         float bs = h2f(dh) * (1099511627776.0f / 4064.0f) * float(mag);
+        if ((sh & 0x7c00u) == 0x7c00u) bs = __builtin_inff();
         bs = pair_sum_lanes<32>(bs);  // the 32 halves of the step's 16 blocks
         if ((i & 31) == 0) a.bound[act_bound(tok, ns, i >> 5)] = bs;
     }
@@ -469,7 +472,7 @@ __device__ __forceinline__ void step_terms_k(const WLds<T_Q6_K> & l, const XStep
 }
 
 // One step with every term formed alone and added to the int64 totals: for steps whose terms could pass the
-// accumulators' 2^51 LSB (activation outliers in the thousands) or whose scales are not finite. Block by block in a
+// accumulators' 2^51 LSB (activation outliers in the thousands) or whose scales or Q8_1 sums are not finite. Block by block in a
 // rolled loop that reads its activation operands again where they lie, so that it takes no registers from step_terms.
 // tot[t][i][lane]: row 4g + i, token r of token tile t.
 template <int TYPE, int T>
@@ -497,7 +500,7 @@ __device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLd
             const v4i zi = {0, 0, 0, 0};
             const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bx, zi, 0, 0, 0);
             const float d40 = h2f(a.d[act_scale(tok, ns, blk)]) * 1099511627776.0f;  // * 2^40, exact
-            const float s40 = TYPE == T_Q4_1 ? h2f(a.s[act_scale(tok, ns, blk)]) * 1099511627776.0f : 0.0f;
+            const float s40 = TYPE == T_Q4_1 ? h2f_fixed(a.s[act_scale(tok, ns, blk)]) * 1099511627776.0f : 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const double sum = TYPE == T_Q4_0 ? double(sm[i]) * 0.0625 : double(sm[i]);

@@ -358,7 +358,7 @@ __device__ __forceinline__ void load_xb(const int8_t * xq, const uint32_t * info
     const uint32_t inf = in ? info[b] : 0u;
     x.dx40 = h2f(inf & 0xffffu) * 1099511627776.0f;  // * 2^40
     x.sum = int(int16_t(inf >> 16));
-    x.sx40 = TYPE == T_Q4_1 && in ? h2f(s1[b]) * 1099511627776.0f : 0.0f;
+    x.sx40 = TYPE == T_Q4_1 && in ? h2f_fixed(s1[b]) * 1099511627776.0f : 0.0f;
 }
 template <int TYPE>
 __device__ __forceinline__ void load_xb(const Lds & s, int b, int nb, XB & x) {

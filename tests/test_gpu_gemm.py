@@ -418,3 +418,28 @@ def test_small_token_pair_of_many_weights(gq, orc, ctx, fmt, rows, ntok):
     for t in range(ntok):
         g, u = (orc.fx_gemv(fmt, w, x[t * cols:(t + 1) * cols], pool, cols) for w in (wg, wu))
         assert_bits(y[t], np.resize(orc.silu_mul(g, u), rows), f"token {t}")
+
+
+@pytest.mark.parametrize("std", [5e-4, 0.02])
+@pytest.mark.parametrize("ntok", [5, 20])
+def test_q4_1_infinite_block_sums(gq, orc, ctx, ntok, std):
+    """Activation blocks whose Q8_1 sum passes the largest fp16 (32 values of 3000: the scale is 23.6, the sum 96000): the
+    canonical arithmetic takes the infinite fp16's bits as 2^16. Small weights keep the step's bound below the FP64
+    accumulators' range, larger ones do not. Every token row of the GEMM and of the GEMV command bit for bit."""
+    rows, cols = 40, 1024
+    w = gq.matrix(3, rows, cols, 6, 90, std=std)
+    off = ctx.upload(3, rows, cols, w)
+    x = gq.normal(6, 91, ntok * cols).reshape(ntok, cols)
+    x[1, 32 * 7:32 * 8] = 3000.0
+    x[3, 32 * 20:32 * 21] = -3000.0
+    x[ntok - 1, [0, 1, 32 * 31]] = 70000.0  # one block past the largest fp16 by two values, one by a single value
+    X, Y, Y1 = 0, ntok * cols, ntok * (cols + 48)
+    ctx.write(X, x.ravel())
+    print(f"[gemm] infinite Q8_1 sums, tokens {ntok} std {std}", flush=True)
+    assert ctx.run(gq.gemm(3, rows, cols, off, X, Y, ntok, cols, 48)) == 0, ctx.error()
+    y = ctx.read(Y, ntok * 48).reshape(ntok, 48)[:, :rows]
+    for t in range(ntok):
+        want = orc.fx_gemv(3, w, x[t], rows, cols)
+        assert ctx.run(gq.gemv(3, rows, cols, off, X + t * cols, Y1)) == 0, ctx.error()
+        assert_bits(ctx.read(Y1, rows), want, f"GEMV token {t}")
+        assert_bits(y[t], want, f"GEMM token {t}")
