@@ -512,7 +512,7 @@ __device__ __forceinline__ void step_terms_exact(const GemmLaunch & a, const WLd
     }
 }
 
-// A matrix whose bound is not known (the caller's own memory, never scanned): the largest |scale| of the step's
+// A matrix whose bound is not known (a scale that is not finite; the caller's own memory, never scanned): the largest |scale| of the step's
 // blocks over the wave, as the host's weight_bound forms it.
 template <int TYPE>
 __device__ __forceinline__ float step_bound(const WLds<TYPE> & l, int lane) {

@@ -45,7 +45,8 @@ float half_to_float_host(uint16_t h) {
 // |sum of products| with Q8_0 quants (|q_x| <= 127: 32 * 8 * 127 for Q4_0, 32 * 15 * 127 for Q4_1, 32 * 128 * 127
 // for Q8_0), plus for Q4_1 |m_w| times the largest |s_x| / d_x (32 * 127); rounded up to FP32. For Q6_K the largest
 // |super-block term| / (|d_x| * (sum of |quants|)): |d_w| times a sub-block scale of at most 128 times 32. 0 for Q5_K.
-// NaN if a scale is one: every launch on the matrix then sums in int64.
+// Infinite if a scale is infinite or NaN, and so is the bound of a pair with such a matrix: the single-token kernels then sum
+// in int64, the batched GEMV forms each step's bound from its own scales (Q6_K: sums in int64).
 float weight_bound(int type, int rows, int cols, const uint8_t * gguf) {
     const auto bits = [](const uint8_t * p) {
         uint16_t u;
@@ -58,7 +59,7 @@ float weight_bound(int type, int rows, int cols, const uint8_t * gguf) {
             const uint8_t * p = gguf + i * 20;
             const double t = half_to_float_host(uint16_t(bits(p))) * (32.0 * 15 * 127) +
                              half_to_float_host(uint16_t(bits(p + 2))) * (32.0 * 127);
-            if (!(t <= best)) best = t;
+            if (!(t <= best)) best = t == t ? t : INFINITY;
         }
     } else if (type == T_Q4_0 || type == T_Q8_0 || type == T_Q6_K) {  // the largest magnitude by its bits
         const size_t bb = type == T_Q4_0 ? 18 : type == T_Q8_0 ? 34 : 210, at = type == T_Q6_K ? 208 : 0;
@@ -70,7 +71,7 @@ float weight_bound(int type, int rows, int cols, const uint8_t * gguf) {
     } else {
         return 0.0f;
     }
-    return std::nextafter(float(best), INFINITY);
+    return best == best ? std::nextafter(float(best), INFINITY) : INFINITY;
 }
 
 struct KvBuf {
@@ -1024,7 +1025,7 @@ struct Compiler {
             const Weight * uw = weight(uoff, t, rows, int(cols));
             if (u2[2] % 16 || u2[2] < uint32_t(rows) || !uw || !range(u[7], uint64_t(u2[2]) * (ntok - 1) + rows))
                 return reject(i + 2, "SwiGLU u GEMM weight, stride or range");
-            if (!(uw->wbound <= g.wbound[0])) g.wbound[0] = uw->wbound;
+            g.wbound[0] = std::max(g.wbound[0], uw->wbound);
             g.epi = EPI_SWIGLU;
             g.w2 = weight_view(c->warena + uoff, t, rows, int(cols));
             g.y = A(u[7]);
@@ -1298,7 +1299,7 @@ struct Compiler {
                     return reject(i + 1, "SwiGLU u GEMV must match its g GEMV");
                 const Weight * uw = weight(uoff, t, rows, int(cols));
                 if (!uw || !range(u[7], uint64_t(rows))) return reject(i + 1, "SwiGLU u weight or range");
-                if (!(uw->wbound <= wb)) wb = uw->wbound;
+                wb = std::max(wb, uw->wbound);
                 m.epi = EPI_SWIGLU;
                 m.w2 = weight_view(c->warena + uoff, t, rows, int(cols));
                 m.y = A(u[7]);

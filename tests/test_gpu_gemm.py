@@ -443,3 +443,42 @@ def test_q4_1_infinite_block_sums(gq, orc, ctx, ntok, std):
         assert ctx.run(gq.gemv(3, rows, cols, off, X + t * cols, Y1)) == 0, ctx.error()
         assert_bits(ctx.read(Y1, rows), want, f"GEMV token {t}")
         assert_bits(y[t], want, f"GEMM token {t}")
+
+
+@pytest.mark.parametrize("fmt", [2, 3, 8, 14])
+def test_nan_scale_ahead_of_small_rows(gq, orc, fmt):
+    """A matrix with rows of large scales, then a row with a NaN scale, then small rows: the other rows' terms pass the
+    FP64 accumulators' range and are summed in int64, whatever follows the NaN in the matrix or (SwiGLU pair, where the
+    format has one) in its second matrix. The rows without the NaN bit for bit, by the GEMM and the GEMV command."""
+    rows, cols, ntok = 4096 if fmt == 14 else 64, 4096 if fmt == 14 else 1024, 6  # (Q6_K: the matrix-core form's size)
+    rb, ys = gq.row_bytes(fmt, cols), up16(rows)
+    small = np.resize(gq.matrix(fmt, 64, cols, 6, 93, std=1e-3), rows * rb).reshape(rows, rb)
+    w = small.copy()
+    w[:4] = gq.matrix(fmt, 4, cols, 6, 92, std=20.0).reshape(4, rb)
+    at = 208 if fmt == 14 else 3 * {2: 18, 3: 20, 8: 34}[fmt]
+    w[7, at:at + 2] = [0x00, 0x7e]
+    ok = np.array([0, 1, 2, 3, 4, 5, 6, 8, 9, 40, 63])
+    x = gq.normal(6, 94, ntok * cols) * 30.0
+    with gq.Context(act_floats=1 << 17, weight_bytes=2 * w.size + 8192) as ctx:
+        og, ou = ctx.upload(fmt, rows, cols, w.ravel()), ctx.upload(fmt, rows, cols, small.ravel())
+        X, Y = 0, ntok * cols
+        YG, Y1 = Y + ntok * ys, Y + 2 * ntok * ys
+        ctx.write(X, x)
+        print(f"[gemm] NaN scale, fmt {fmt}", flush=True)
+        assert ctx.run(gq.gemm(fmt, rows, cols, og, X, Y, ntok, cols, ys)) == 0, ctx.error()
+        y = ctx.read(Y, ntok * ys).reshape(ntok, ys)[:, ok]
+        pair = None
+        if fmt != 14:
+            cmd = (gq.gemm(fmt, rows, cols, og, X, YG, ntok, cols, ys, gq.GEMV_SWIGLU) +
+                   gq.gemm(fmt, rows, cols, ou, X, Y, ntok, cols, ys))
+            assert ctx.run(cmd) == 0, ctx.error()
+            pair = ctx.read(Y, ntok * ys).reshape(ntok, ys)[:, ok]
+        for t in range(ntok):
+            xt = x[t * cols:(t + 1) * cols]
+            g, u = (orc.fx_gemv(fmt, m[ok].ravel(), xt, len(ok), cols) for m in (w, small))
+            assert np.abs(g[:4]).max() > 4096.0  # past the accumulators' 2^51 LSB of 2^-40
+            assert ctx.run(gq.gemv(fmt, rows, cols, og, X + t * cols, Y1)) == 0, ctx.error()
+            assert_bits(ctx.read(Y1, rows)[ok], g, f"GEMV token {t}")
+            assert_bits(y[t], g, f"GEMM token {t}")
+            if pair is not None:
+                assert_bits(pair[t], orc.silu_mul(g, u), f"SwiGLU GEMM token {t}")
