@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <string>
+#include <vector>
+
 namespace gq {
 
 enum : int { T_Q4_0 = 2, T_Q4_1 = 3, T_Q8_0 = 8, T_Q5_K = 13, T_Q6_K = 14 };
@@ -308,22 +311,38 @@ constexpr int ATTN_CHUNK = 64;
 // a launch more than attn_group_kernel, which is the faster for few tokens at short positions (head_dim 256, position 100:
 // 8 tokens 25 us against 29, 16 tokens 33 against 32, 32 tokens 47 against 38; 128: 28 / 24, 40 / 28, 64 / 34).
 constexpr int ATTN_TILE_HD = 64, ATTN_TILE_TOK = 16;
+inline bool attn_tiled(const AttnArgs & a) { return a.head_dim >= ATTN_TILE_HD && !a.seq_ctx && a.n_tok >= ATTN_TILE_TOK; }
 constexpr int ATTN_MAXG = 8;  // q heads per KV head
 constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command
 // GDN commands of at least this many tokens form norms and gates in a launch of their own (32 value heads, us in a graph at
 // 6 / 8 / 10 / 16 / 32 tokens: 15.8 / 16.0 / 16.0 / 17.5 / 23.8 against 15.3 / 16.3 / 18.5 / 25.4 / 43.6 in the step).
 constexpr unsigned GDN_PREP_TOK = 8;
+inline bool gdn_ahead(const GdnArgs & a) { return !a.seqs && a.prep; }
 
-// Profiling: when set (by gemvq_profile on the calling thread), launchers start kernels through
-// hipExtLaunchKernelGGL with these events, which record the kernel's own start and end on the device.
-extern thread_local hipEvent_t g_prof_start, g_prof_stop;
+// Profiling: while g_prof points to one (set by gemvq_profile on the calling thread, per launch of a list), launchers start
+// kernels through hipExtLaunchKernelGGL with an event pair of it each, which record the kernel's own start and end on the
+// device.
+struct LaunchTimer {
+    struct Kernel {
+        hipEvent_t start = nullptr, stop = nullptr;
+        std::string name;  // without template arguments
+    };
+    std::vector<Kernel> kernels;  // the events are kept over repetitions
+    size_t n = 0;                 // kernels started since it was set to 0
+    hipError_t error = hipSuccess;  // of an event's creation
 
+    const Kernel & next(const char * kernel);
+    LaunchTimer() = default;
+    LaunchTimer(const LaunchTimer &) = delete;
+    ~LaunchTimer();
+};
+extern thread_local LaunchTimer * g_prof;
 #define GQ_LAUNCH(kernel, grid, block, shmem, stream, ...)                                                         \
     do {                                                                                                            \
-        if (::gq::g_prof_start)                                                                                     \
-            hipExtLaunchKernelGGL(kernel, grid, block, shmem, stream, ::gq::g_prof_start, ::gq::g_prof_stop, 0,     \
-                                  __VA_ARGS__);                                                                     \
-        else                                                                                                        \
+        if (::gq::g_prof) {                                                                                         \
+            const ::gq::LaunchTimer::Kernel & k_ = ::gq::g_prof->next(#kernel);                                     \
+            hipExtLaunchKernelGGL(kernel, grid, block, shmem, stream, k_.start, k_.stop, 0, __VA_ARGS__);           \
+        } else                                                                                                      \
             hipLaunchKernelGGL(kernel, grid, block, shmem, stream, __VA_ARGS__);                                    \
     } while (0)
 

@@ -847,7 +847,7 @@ hipError_t launch_rope(const RopeArgs & a, hipStream_t s) {
 }
 
 hipError_t launch_gdn(const GdnArgs & a, hipStream_t s) {
-    if (!a.seqs && a.prep) {
+    if (gdn_ahead(a)) {
         GQ_LAUNCH(gdn_prep_kernel, dim3((2 * a.hk + GDN_PREP_ROWS - 1) / GDN_PREP_ROWS, a.n_tok), dim3(128), 0, s, a);
         GQ_LAUNCH(gdn_tokens_kernel, dim3(a.hv * (128 / GDN_ROWS)), dim3(128), 0, s, a);
         return hipGetLastError();
@@ -1132,7 +1132,7 @@ hipError_t launch_attn_hd(const AttnArgs & a, dim3 grid, hipStream_t s) {
     GQ_LAUNCH(attn_append_kernel<HD>, dim3(a.n_head + a.n_head_kv, grid.y), dim3(ATT_T), 0, s, a);
     const int G = a.n_head / a.n_head_kv;
     if constexpr (HD >= ATTN_TILE_HD)
-        if (!a.seq_ctx && int(grid.y) >= ATTN_TILE_TOK) {
+        if (attn_tiled(a)) {
             // A prompt chunk's batch: 4 waves of work a SIMD and more at once, so the queries a wave holds pay (7 batches up
             // to 1983 positions of 16 heads, 256 wide: 1.10 ms at 4 queries x 8 waves, 1.16 at 8 x 8, 1.21 at 8 x 4). A
             // command's 16 to 32 tokens leave the chip idle at short positions: fewer queries a wave (32 tokens at position

@@ -23,8 +23,28 @@
 using namespace gq;
 
 namespace gq {
-thread_local hipEvent_t g_prof_start = nullptr, g_prof_stop = nullptr;
+thread_local LaunchTimer * g_prof = nullptr;
+
+const LaunchTimer::Kernel & LaunchTimer::next(const char * kernel) {
+    if (n == kernels.size()) {
+        kernels.emplace_back();
+        Kernel & k = kernels.back();
+        hipError_t e = hipEventCreate(&k.start);
+        if (e == hipSuccess) e = hipEventCreate(&k.stop);
+        if (e != hipSuccess && error == hipSuccess) error = e;
+        k.name = kernel + (*kernel == '(');
+        k.name.resize(std::min(k.name.find_first_of("<)"), k.name.size()));
+    }
+    return kernels[n++];
 }
+
+LaunchTimer::~LaunchTimer() {
+    for (const Kernel & k : kernels) {
+        if (k.start) (void)hipEventDestroy(k.start);
+        if (k.stop) (void)hipEventDestroy(k.stop);
+    }
+}
+}  // namespace gq
 
 namespace {
 
@@ -1478,6 +1498,29 @@ std::pair<std::string, uint64_t> describe(const Launch & l, int pos) {
     return {"next_token_kernel", 32};
 }
 
+// The kernels a launch starts.
+int kernels_of(const Launch & l) {
+    if (auto * x = std::get_if<LAttn>(&l)) return x->ref ? 2 : x->a.n_tok <= 1 ? 1 : attn_tiled(x->a) ? 3 : 2;
+    if (auto * x = std::get_if<LGdn>(&l)) return !x->ref && gdn_ahead(x->a) ? 2 : 1;
+    return 1;
+}
+
+// The name a profiled launch is reported by: one kernel's own (with the template arguments that describe gives it), several
+// joined by + without their ending.
+std::string launch_name(const std::string & described, const LaunchTimer & t) {
+    if (t.kernels.size() == 1) {
+        const std::string & k = t.kernels[0].name;
+        return described.compare(0, described.find('<'), k) == 0 ? described : k;
+    }
+    std::string name;
+    for (const LaunchTimer::Kernel & k : t.kernels) {
+        const std::string ending = "_kernel";
+        const bool ends = k.name.size() > ending.size() && k.name.compare(k.name.size() - ending.size(), ending.size(), ending) == 0;
+        name += (name.empty() ? "" : "+") + k.name.substr(0, k.name.size() - (ends ? ending.size() : 0));
+    }
+    return name;
+}
+
 hipError_t issue(const std::vector<Launch> & ls, hipStream_t s) {
     for (const Launch & l : ls) {
         hipError_t e = hipSuccess;
@@ -1514,7 +1557,8 @@ int compile_list(gemvq_ctx * c, const uint32_t * cmds, unsigned n, std::vector<L
     }
     out = std::move(cp.out);
     if (spans) *spans = std::move(cp.spans);
-    c->last_launches = int(out.size());
+    c->last_launches = 0;
+    for (const Launch & l : out) c->last_launches += kernels_of(l);
     return 0;
 }
 
@@ -2047,43 +2091,40 @@ int gemvq_profile(gemvq_ctx * c, const uint32_t * cmds, unsigned n, int reps, ge
             break;
         }
     const size_t L = ls.size();
-    std::vector<hipEvent_t> e0(L), e1(L);
-    std::vector<std::vector<float>> ms_of(L);  // per launch, one duration per repetition
+    std::vector<LaunchTimer> timers(L);
+    std::vector<std::vector<float>> ms_of(L);  // per launch, one duration (the sum over its kernels) per repetition
     hipError_t e = hipSuccess;
     int ws = 0;
-    for (size_t i = 0; i < L && e == hipSuccess; ++i) {
-        e = hipEventCreate(&e0[i]);
-        if (e == hipSuccess) e = hipEventCreate(&e1[i]);
-    }
     for (int r = 0; r < reps && e == hipSuccess && ws == 0; ++r) {
-        for (size_t i = 0; i < L && e == hipSuccess; ++i) {
-            g_prof_start = e0[i];
-            g_prof_stop = e1[i];
-            e = issue({ls[i]}, c->stream);
-        }
-        g_prof_start = g_prof_stop = nullptr;
         c->busy = true;
+        for (size_t i = 0; i < L && e == hipSuccess; ++i) {
+            g_prof = &timers[i];
+            g_prof->n = 0;
+            e = issue({ls[i]}, c->stream);
+            if (e == hipSuccess) e = g_prof->error;
+        }
+        g_prof = nullptr;
         if (e == hipSuccess) ws = wait_stream(c, "profile");
         if (ws) break;
         for (size_t i = 0; i < L && e == hipSuccess; ++i) {
-            float ms = 0.0f;
-            e = hipEventSynchronize(e1[i]);
-            if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0[i], e1[i]);
-            ms_of[i].push_back(ms);
+            float sum = 0.0f;
+            for (size_t k = 0; k < timers[i].n && e == hipSuccess; ++k) {
+                float ms = 0.0f;
+                e = hipEventSynchronize(timers[i].kernels[k].stop);
+                if (e == hipSuccess) e = hipEventElapsedTime(&ms, timers[i].kernels[k].start, timers[i].kernels[k].stop);
+                sum += ms;
+            }
+            ms_of[i].push_back(sum);
         }
-    }
-    g_prof_start = g_prof_stop = nullptr;
-    for (size_t i = 0; i < L; ++i) {
-        if (e0[i]) hipEventDestroy(e0[i]);
-        if (e1[i]) hipEventDestroy(e1[i]);
     }
     if (ws) return ws;
     if (e != hipSuccess) return fail(c, e, "profile");
     for (size_t i = 0; i < L && int(i) < max_out; ++i) {
         const auto d = describe(ls[i], pos);
+        const std::string name = launch_name(d.first, timers[i]);
         gemvq_launch_stat & o = out[i];
         std::memset(&o, 0, sizeof(o));
-        std::strncpy(o.name, d.first.c_str(), sizeof(o.name) - 1);
+        std::strncpy(o.name, name.c_str(), sizeof(o.name) - 1);
         o.first_cmd = spans[i].first;
         o.n_cmds = spans[i].second;
         o.bytes = d.second;

@@ -221,7 +221,7 @@ int gemvq_usable(const gemvq_ctx * ctx);
 /* Free and total HBM of a device (hipMemGetInfo); 0 or a negative HIP error. */
 int gemvq_device_memory(int device, size_t * free_bytes, size_t * total_bytes);
 
-/* Number of kernel launches the last validated list compiled to (after fusion). */
+/* Number of kernels the last validated list starts (after fusion). */
 int gemvq_last_launch_count(const gemvq_ctx * ctx);
 
 /* Debug: the integer block sums of the next GEMV pass's first matrix are written to dst (int32 per 32-block for
@@ -236,7 +236,9 @@ int gemvq_graph_time(gemvq_ctx * ctx, int graph, int times, double * us_per_repl
  * ggml-xrt.cpp:285-314, 1302-1397): runs a command list `reps` times, each kernel launched with device start/stop
  * events (hipExtLaunchKernelGGL), and reports per launch the kernel, the commands it executes, its algorithmic
  * bytes (GGUF-sized weights, fp32 vectors read and written once, state and KV cache traffic) and its median
- * duration over the repetitions. The list's side effects happen `reps` times. Returns the number of launches (>= 0) or a status. */
+ * duration over the repetitions. A command that starts several kernels (ATTN and GDN of several tokens) is one entry, named
+ * after all of them ("attn_append+attn_tile+attn_combine"), with the sum of their durations. The list's side effects happen
+ * `reps` times. Returns the number of entries (>= 0) or a status. */
 typedef struct {
     char name[40];
     int32_t first_cmd, n_cmds;

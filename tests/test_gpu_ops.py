@@ -653,3 +653,55 @@ def test_c4_gated_deltanet_layer(gq, orc):
     assert_bits(ctx.read(O["y"], Hv * S), y, "gated output")
     assert_bits(ctx.read(O["x"], E), orc.fx_gemv(2, Wo, y, E, Hv * S) + x, "layer output")
     ctx.close()
+
+
+def _attn_of(gq, ctx, ntok):
+    """An ATTN command of ntok tokens (16 heads of 256 on a cache of 2048 positions, zeros for inputs) and its cache."""
+    nh, nkv, hd, n_ctx = 16, 4, 256, 2048
+    kv = ctx.kv_create(n_ctx, nkv, hd)
+    O = dict(q=0, k=262144, v=294912, qn=327680, kn=327936, pos=328192, y=328704, cs=460800)
+    slots = np.zeros(16 * 32, np.int32)
+    slots[::16] = 2000
+    ctx.write(O["pos"], slots)
+    return gq.attn(nh, nkv, O["q"], kv, O["y"], hd, 64, O["pos"], O["k"], O["v"], 1 / 16, 1e-6, O["qn"], O["kn"], O["cs"],
+                   gate=O["q"] + hd, n_tok=ntok)
+
+
+@pytest.mark.parametrize("ntok,kernels", [(1, ["attn_kernel"]), (8, ["attn_append", "attn_group"]),
+                                          (32, ["attn_append", "attn_tile", "attn_combine"])])
+def test_profile_reports_every_kernel_of_a_launch(gq, ctx, ntok, kernels):
+    """A launch that starts several kernels: the profile names them all and gives the sum of their durations (compared with
+    the device time of its captured replays, which has the gaps between kernels too); the launch count counts them."""
+    cmd = _attn_of(gq, ctx, ntok)
+    ctx.run(cmd)
+    assert ctx.launch_count() == len(kernels)
+    stats = ctx.profile(np.array(cmd, np.uint32), 9)
+    assert len(stats) == 1
+    assert stats[0]["name"] == "+".join(kernels), stats[0]["name"]
+    g = ctx.graph(cmd)
+    ctx.replay(g, 5)
+    us = ctx.graph_time_us(g, 50)
+    print(f"[profile] {stats[0]['name']}: {stats[0]['us']:.1f} us, replay {us:.1f} us", flush=True)
+    if ntok == 32:  # the append and the combine are a small part
+        assert 0.5 * us < stats[0]["us"] < 1.5 * us
+
+
+def test_profile_of_many_token_deltanet(gq):
+    """The same for a DeltaNet step with its norms and gates ahead, and the token-parallel conv's own name."""
+    hv, hk, S = 32, 16, 128
+
+    def step(ntok):
+        c = gq.gdn(hv, hk, 0, 131072, 262144, 524288, 528384, 540672, 0, 0, 1 / np.sqrt(S), gq.GDN_GATES | gq.GDN_L2_QK, 1e-6,
+                   1e-6, 0, 0, 532480, 532544)
+        c[16 + 2:16 + 5] = [ntok, hv * S, hv]
+        return c
+    with gq.Context(act_floats=1 << 20, weight_bytes=1 << 16, state_rows=hv * S) as c2:
+        for ntok, name in ((7, "gdn_kernel"), (32, "gdn_prep+gdn_tokens")):
+            assert c2.run(step(ntok)) == 0, c2.error()
+            assert c2.launch_count() == len(name.split("+"))
+            stats = c2.profile(np.array(step(ntok), np.uint32), 3)
+            assert [s_["name"] for s_ in stats] == [name]
+        x, w, st = 0, 700000, 710000
+        conv = gq.conv(272, x, w, 8192, st, st, silu=True)
+        conv[7] |= 8 << 16
+        assert [s_["name"] for s_ in c2.profile(np.array(conv, np.uint32), 3)] == ["conv_tokens_kernel"]
