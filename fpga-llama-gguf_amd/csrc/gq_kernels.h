@@ -128,8 +128,8 @@ struct GdnArgs {
     int s_qkv, s_gb, s_y;  // row strides (floats) between tokens of q / k / v, of g / beta, of y
     int seqs;              // nonzero: the tokens belong to n_tok sequences, token t on its own state rows (src and
                            // dst + t * hv * 128 rows), all in one launch
-    float * prep;          // many tokens of one sequence: where their L2 norms and gates are formed ahead (n_tok rows of 2
-                           // hk 128 + 2 hv floats), NULL: in the step
+    float * prep;          // many tokens of one sequence: where their L2 norms and gates are formed ahead (n_tok rows of
+                           // gdn_prep_row floats), NULL: in the step
     // reference arithmetic with the gated output norm (GEMVQ_GDN_GATED): the step's launch also applies the norm to
     // its token's heads (z rows hv * 128 apart per token, the norm weight [128], the RMS eps); NULL gz: not applied
     const float * gz;
@@ -317,6 +317,8 @@ constexpr int GDN_MAX_HEADS = 64;  // value heads of one GDN command
 // GDN commands of at least this many tokens form norms and gates in a launch of their own (32 value heads, us in a graph at
 // 6 / 8 / 10 / 16 / 32 tokens: 15.8 / 16.0 / 16.0 / 17.5 / 23.8 against 15.3 / 16.3 / 18.5 / 25.4 / 43.6 in the step).
 constexpr unsigned GDN_PREP_TOK = 8;
+// Floats of a token there: 2 hk rows of 128 (q, then k), then hv (decay, beta) pairs, in whole 16 bytes.
+__host__ __device__ constexpr int gdn_prep_row(int hk, int hv) { return 2 * hk * 128 + (2 * hv + 3) / 4 * 4; }
 inline bool gdn_ahead(const GdnArgs & a) { return !a.seqs && a.prep; }
 
 // Profiling: while g_prof points to one (set by gemvq_profile on the calling thread, per launch of a list), launchers start

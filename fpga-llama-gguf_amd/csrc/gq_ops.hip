@@ -285,12 +285,11 @@ __global__ __launch_bounds__(128) void gdn_kernel(const float * src, const float
 // A token's state update needs the one before it, but its L2 norms and gates do not, and gdn_kernel computes them again in
 // every row's lanes inside that chain (1.23 us a token at C5's heads, of which the chain itself is a sixth). So a first
 // launch forms them for all tokens at once, with the same operations on the same lanes: workgroup (token, 8 of the 2 hk
-// rows of q and k), 16 lanes a row as in gdn_kernel; the first one of a token also its decays and betas. prep: per token 2
-// hk 128 floats (q, then k), then the hv (decay, beta) pairs.
+// rows of q and k), 16 lanes a row as in gdn_kernel; the first one of a token also its decays and betas.
 constexpr int GDN_PREP_ROWS = 8;
 __global__ __launch_bounds__(128) void gdn_prep_kernel(GdnArgs a) {
     const int tk = blockIdx.y, l16 = threadIdx.x & 15, r = blockIdx.x * GDN_PREP_ROWS + int(threadIdx.x >> 4);
-    float * out = a.prep + size_t(tk) * (2 * a.hk * 128 + 2 * a.hv);
+    float * out = a.prep + size_t(tk) * gdn_prep_row(a.hk, a.hv);
     if (blockIdx.x == 0)
         for (int h = threadIdx.x; h < a.hv; h += 128) {
             float bt;
@@ -321,7 +320,7 @@ struct GdnPrepped {
 __global__ __launch_bounds__(128) void gdn_tokens_kernel(GdnArgs a) {
     const int chunks = 128 / GDN_ROWS, h = blockIdx.x / chunks, chunk = blockIdx.x % chunks, kh = h % a.hk;
     const int l16 = threadIdx.x & 15, j = chunk * GDN_ROWS + int(threadIdx.x >> 4);
-    const size_t row = (size_t(h) * 128 + j) * 128 + 8 * l16, ps = 2 * a.hk * 128 + 2 * a.hv;
+    const size_t row = (size_t(h) * 128 + j) * 128 + 8 * l16, ps = gdn_prep_row(a.hk, a.hv);
     const float * qp = a.prep + kh * 128 + 8 * l16, * kp = qp + a.hk * 128, * dp = a.prep + 2 * a.hk * 128 + 2 * h;
     const float * vp = a.v + h * 128 + j;
     float * yp = a.y + h * 128 + j;

@@ -161,11 +161,9 @@ struct gemvq_ctx {
     uint16_t * gemm_s = nullptr;  // and their Q8_1 block sums (for Q4_1 weights)
     float * gemm_b = nullptr;     // and their parts of the term bounds
     uint8_t * wide = nullptr;     // the same for a list of the model driver's prompt chunks (up to GEMM_WIDE_TOK rows)
-    float * gdn_prep = nullptr;   // norms and gates of a GDN command's tokens, and the floats it holds; the smaller
-    size_t gdn_prep_n = 0;        // buffers before it, which captured graphs may still use
-    std::vector<float *> gdn_prep_old;
-    float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens), likewise
-    size_t attn_wide_n = 0;
+    float * gdn_prep[2] = {};     // norms and gates of a GDN command's tokens: of a caller's list, of a prompt chunk's
+    float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens); the
+    size_t attn_wide_n = 0;       // smaller ones before it, which captured graphs may still use
     std::vector<float *> attn_wide_old;
     int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
@@ -766,7 +764,7 @@ struct Compiler {
                                                 {k[5], uint64_t(k[5]) + uint64_t(sg) * (ntok - 1) + hv},
                                                 {k[6], uint64_t(k[6]) + uint64_t(sg) * (ntok - 1) + hv}};
                 if (ntok >= GDN_PREP_TOK && !seqs && !meet_any({{k[7], uint64_t(k[7]) + yz + hv * 128}}, reads))
-                    a.prep = gdn_prep(size_t(ntok) * (2 * hk * 128 + 2 * hv));
+                    a.prep = gdn_prep();
                 if ((flags & GEMVQ_GDN_GATED) && ntok == 1 && fold_gated(cmds, n, next, k[7], hv * 128, k2[7], k2[6])) {
                     // the gated norm runs in the next GEMV's activation prologue: the step writes its raw output
                     // to scratch, and that GEMV writes the gated values to y as the norm would have
@@ -976,18 +974,15 @@ struct Compiler {
         return attn_wide_part(b, n_head, n_tok) + size_t(n_tok) * n_head * b.head_dim;
     }
 
-    // A buffer of n floats for the norms and gates of a GDN command's tokens; NULL (they are formed in the step) without
-    // memory for it. Commands run in order, so they share one.
-    float * gdn_prep(size_t n) const {
-        if (c->gdn_prep_n >= n) return c->gdn_prep;
-        float * p = nullptr;
-        if (hipMalloc(&p, n * sizeof(float)) != hipSuccess) {
+    // The buffer for the norms and gates of a GDN command's tokens, allocated once for the most tokens and heads that a command
+    // of the list may have (2 MiB; 32 MiB in the model driver's lists): commands run in order and share it, and its size does
+    // not depend on the commands seen. NULL (they are formed in the step) without memory for it.
+    float * gdn_prep() const {
+        float *& p = c->gdn_prep[c->max_tok > GEMM_MAX_TOK];
+        if (!p && hipMalloc(&p, size_t(c->max_tok) * gdn_prep_row(GDN_MAX_HEADS, GDN_MAX_HEADS) * sizeof(float)) != hipSuccess) {
             (void)hipGetLastError();
-            return nullptr;
+            p = nullptr;
         }
-        if (c->gdn_prep) c->gdn_prep_old.push_back(c->gdn_prep);
-        c->gdn_prep = p;
-        c->gdn_prep_n = n;
         return p;
     }
 
@@ -1657,8 +1652,7 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->gemm_s);
     hipFree(c->gemm_b);
     hipFree(c->wide);
-    hipFree(c->gdn_prep);
-    for (float * p : c->gdn_prep_old) hipFree(p);
+    for (float * p : c->gdn_prep) hipFree(p);
     hipFree(c->attn_wide);
     for (float * p : c->attn_wide_old) hipFree(p);
     hipFree(c->ref_x);

@@ -705,3 +705,27 @@ def test_profile_of_many_token_deltanet(gq):
         conv = gq.conv(272, x, w, 8192, st, st, silu=True)
         conv[7] |= 8 << 16
         assert [s_["name"] for s_ in c2.profile(np.array(conv, np.uint32), 3)] == ["conv_tokens_kernel"]
+
+
+def _free_memory(gq):
+    free = gq.C.c_size_t()
+    assert gq.hip_lib().gemvq_device_memory(0, gq.C.byref(free), None) == 0
+    return free.value
+
+
+def test_gdn_token_scratch_is_bounded(gq):
+    """DeltaNet commands of ascending token counts leave the device's free memory where the first left it (one scratch for
+    norms and gates serves every count of a command)."""
+    hv, S = 64, 128
+
+    def step(ntok):
+        c = gq.gdn(hv, hv, 0, 262144, 524288, 786432, 790528, 800000, 0, 0, 1 / np.sqrt(S), gq.GDN_GATES, 1e-6, 1e-6, 0, 0,
+                   794624, 794688)
+        c[16 + 2:16 + 5] = [ntok, hv * S, hv]
+        return c
+    with gq.Context(act_floats=1 << 21, weight_bytes=1 << 16, state_rows=hv * S) as ctx:
+        assert ctx.run(step(8)) == 0, ctx.error()
+        free = _free_memory(gq)
+        for ntok in range(9, 33):
+            assert ctx.run(step(ntok)) == 0, ctx.error()
+        assert free - _free_memory(gq) < 4 << 20  # one buffer each would be 33 MB
