@@ -165,6 +165,7 @@ struct gemvq_ctx {
     float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens); the
     size_t attn_wide_n = 0;       // smaller ones before it, which captured graphs may still use
     std::vector<float *> attn_wide_old;
+    size_t scratch_max = ~size_t(0);  // largest allocation for scratch that a launch can do without (set at creation)
     int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
     float * ref_x = nullptr;      // the reference arithmetic's copy of a GEMM's token rows and norm weight
     int arith = GEMVQ_ARITH_CANONICAL;  // the arithmetic lists are compiled in (gemvq_set_arith)
@@ -247,6 +248,16 @@ constexpr size_t STAGE_BYTES = size_t(1) << 20;
 // Host copies of pageable memory run synchronously behind the work already queued on the stream, outside any
 // bound: every such copy first waits (bounded) for that work, so the copy itself has nothing to wait behind.
 int drain(gemvq_ctx * c, const char * what) { return wait_stream(c, what); }
+
+// Device memory for scratch whose launches have a form without it; NULL where there is none (no error of the context).
+void * optional_scratch(gemvq_ctx * c, size_t bytes) {
+    void * p = nullptr;
+    if (!c->usable || bytes > c->scratch_max) return nullptr;
+    hipSetDevice(c->device);
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
 
 int einval(gemvq_ctx * c, const std::string & what) {
     if (c) c->err = what;
@@ -979,10 +990,8 @@ struct Compiler {
     // not depend on the commands seen. NULL (they are formed in the step) without memory for it.
     float * gdn_prep() const {
         float *& p = c->gdn_prep[c->max_tok > GEMM_MAX_TOK];
-        if (!p && hipMalloc(&p, size_t(c->max_tok) * gdn_prep_row(GDN_MAX_HEADS, GDN_MAX_HEADS) * sizeof(float)) != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
-        }
+        const size_t n = size_t(c->max_tok) * gdn_prep_row(GDN_MAX_HEADS, GDN_MAX_HEADS);
+        if (!p) p = static_cast<float *>(optional_scratch(c, n * sizeof(float)));
         return p;
     }
 
@@ -1585,8 +1594,18 @@ gemvq_ctx * gemvq_ctx_create(int device, size_t act_floats, size_t weight_bytes,
         }
         polls = unsigned(p);
     }
+    size_t scratch_max = ~size_t(0);  // GEMVQ_SCRATCH_LIMIT, bytes (0: none of it, which tests use to reach those forms)
+    if (const char * v = std::getenv("GEMVQ_SCRATCH_LIMIT")) {
+        char * end = nullptr;
+        scratch_max = size_t(std::strtoull(v, &end, 10));
+        if (end == v || *end != '\0' || *v == '-') {
+            g_create_error = "gemvq_ctx_create: GEMVQ_SCRATCH_LIMIT must be a non-negative integer";
+            return nullptr;
+        }
+    }
     auto * c = new gemvq_ctx();
     c->device = device;
+    c->scratch_max = scratch_max;
     c->wait_ms = wait_ms;
     c->xch_polls = polls;
     hipError_t e = hipSetDevice(device);
@@ -1882,17 +1901,12 @@ int gemvq_run(gemvq_ctx * c, const uint32_t * cmds, unsigned n) {
 
 // Whether the lists compiled from now on may hold commands of up to GEMM_WIDE_TOK tokens (GEMM, CONV, GDN, GET_ROWS; ATTN: gq_attn_tokens): for
 // the prompt chunks of the model driver, which switches it on around its own lists. A caller's lists keep the limits of
-// the header.
+// the header. GEMVQ_EINVAL without memory for their scratch: the limits stay, the context is as before.
 __attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int on) {
     if (!c) return GEMVQ_EINVAL;
     if (on && !c->wide) {
-        if (!c->usable) return unusable(c);
-        hipSetDevice(c->device);
-        const hipError_t e = hipMalloc(&c->wide, Compiler::WIDE_BYTES);
-        if (e != hipSuccess) {
-            c->wide = nullptr;
-            return fail(c, e, "prompt chunk scratch");
-        }
+        c->wide = static_cast<uint8_t *>(optional_scratch(c, Compiler::WIDE_BYTES));
+        if (!c->wide) return GEMVQ_EINVAL;
     }
     c->max_tok = on ? GEMM_WIDE_TOK : GEMM_MAX_TOK;
     return 0;
@@ -1912,12 +1926,8 @@ __attribute__((visibility("hidden"))) int gq_attn_tokens(gemvq_ctx * c, int kv, 
     if (tok <= sets) return std::max(sets, 32);
     const size_t n = Compiler::attn_wide_floats(b, n_head, tok);
     if (c->attn_wide_n < n) {
-        hipSetDevice(c->device);
-        float * p = nullptr;
-        if (hipMalloc(&p, n * sizeof(float)) != hipSuccess) {
-            (void)hipGetLastError();
-            return std::max(sets, 32);
-        }
+        float * p = static_cast<float *>(optional_scratch(c, n * sizeof(float)));
+        if (!p) return std::max(sets, 32);
         if (c->attn_wide) c->attn_wide_old.push_back(c->attn_wide);
         c->attn_wide = p;
         c->attn_wide_n = n;

@@ -557,11 +557,12 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
     if (st) return st;
     const int np = int(m->prompt_ids.size());
     if (pos < 0 || pos + n > np - 1) return set_err(ctx, "gemvq_qwen35_prefill: positions past the last prompt token but one");
-    // chunks of the layout's rows; the reference arithmetic runs its commands token by token and keeps their limit
-    const int most = gemvq_arith(ctx) == GEMVQ_ARITH_REFERENCE ? int(GEMVQ_GEMM_MAX_TOK) : int(m->chunk);
+    // chunks of the layout's rows; the reference arithmetic runs its commands token by token and keeps their limit, and so
+    // does a prompt without memory for the scratch of longer chunks
+    int most = gemvq_arith(ctx) == GEMVQ_ARITH_REFERENCE ? int(GEMVQ_GEMM_MAX_TOK) : int(m->chunk);
     m->attn_batch = GEMVQ_GEMM_MAX_TOK;
+    if (most > int(GEMVQ_GEMM_MAX_TOK) && gq_wide_lists(ctx, 1)) most = GEMVQ_GEMM_MAX_TOK;
     if (most > int(GEMVQ_GEMM_MAX_TOK)) {
-        st = gq_wide_lists(ctx, 1);
         for (int il = 0; il < m->c.n_layer; ++il)  // (the layers' caches are alike)
             if (is_attn(m->c, il)) {
                 m->attn_batch = uint32_t(std::max(gq_attn_tokens(ctx, m->kv[il], m->c.n_head, most), int(GEMVQ_GEMM_MAX_TOK)));
@@ -580,7 +581,8 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
         if (!st && nt == most) {
             // full chunks replay one captured list: it reads the chunk's ids and positions from the slots just written
             // (the writes, the previous replay before them and this one run in order on the same stream)
-            if (m->chunk_graph >= 0 && m->chunk_graph_tok != most) {  // the arithmetic was switched: other chunks
+            // (the arithmetic was switched on the context, or the longer chunks' scratch could be had after all)
+            if (m->chunk_graph >= 0 && m->chunk_graph_tok != most) {
                 gemvq_graph_destroy(ctx, m->chunk_graph);
                 m->chunk_graph = -1;
             }

@@ -287,3 +287,33 @@ def test_prompt_chunks_of_many_tokens_equal_decode_steps(gq, q35, wtype, n_promp
         m.step(4)
         assert np.array_equal(m.tokens(n_prompt + 4), t_steps)
         assert np.array_equal(m.logits().view(np.uint32), l_steps.view(np.uint32))
+
+
+@pytest.mark.parametrize("limit", [0, 16 << 20])
+def test_prompt_without_memory_for_wide_chunks(gq, q35, monkeypatch, limit):
+    """Without memory for the scratch of longer prompt chunks the prefill runs in chunks of 32 (limit 0: none of the optional
+    scratch; 16 MiB: the chunks' own, not that of the DeltaNet norms ahead): states, cache, ids and the generation after it
+    equal the decode steps' bit for bit, and the context stays usable."""
+    n_prompt = 100
+    cfg = q35.Config(n_layer=4, n_embd=1024, n_ff=1536, n_vocab=1040, n_head=4, n_head_kv=1, head_dim=128, n_rot=32,
+                     ssm_k_heads=2, ssm_v_heads=4, n_ctx=n_prompt + 8)
+    prompt = q35.prompt_ids(cfg, n_prompt, seed=3)
+    monkeypatch.setenv("GEMVQ_SCRATCH_LIMIT", str(limit))
+    with q35.Model(q35.generate(cfg, seed=3)) as m:
+        m.reset(prompt)
+        m.step(n_prompt - 1)
+        want = _decode_state(m, cfg, n_prompt - 1)
+        m.step(4)
+        t_steps, l_steps = m.tokens(n_prompt + 4), m.logits()
+        for _ in range(2):
+            m.reset(prompt)
+            assert m.prefill(n_prompt - 1)
+            assert m.ctx.usable()
+            got = _decode_state(m, cfg, n_prompt - 1)
+            assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32)), "DeltaNet states"
+            for a, b in zip(got[1], want[1]):
+                assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), "KV cache"
+            assert np.array_equal(got[2], want[2]), "token ids"
+            m.step(4)
+            assert np.array_equal(m.tokens(n_prompt + 4), t_steps)
+            assert np.array_equal(m.logits().view(np.uint32), l_steps.view(np.uint32))

@@ -217,3 +217,12 @@ def test_wait_timeout_setting_is_validated(gq, libs, monkeypatch):
         assert b"GEMVQ_WAIT_TIMEOUT_MS" in lib.gemvq_last_error(None)
     assert lib.gemvq_set_wait_timeout(None, 5) == gq.EINVAL
     assert lib.gemvq_usable(None) == 0
+
+
+def test_scratch_limit_setting_is_validated(gq, libs, monkeypatch):
+    """The bound on optional scratch: a malformed GEMVQ_SCRATCH_LIMIT fails the create before any device call."""
+    lib = gq.hip_lib()
+    for bad in ("abc", "12x", "-5", ""):
+        monkeypatch.setenv("GEMVQ_SCRATCH_LIMIT", bad)
+        assert not lib.gemvq_ctx_create(0, 1024, 0, 0), bad
+        assert b"GEMVQ_SCRATCH_LIMIT" in lib.gemvq_last_error(None)
