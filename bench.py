@@ -373,7 +373,7 @@ def sequences(args) -> int:
         print(json.dumps({"sequences_decode": n, "tokens_per_s": round(tok_s, 1), "steps": args.steps,
                           "ms_per_step": round(dt * 1e3 / args.steps, 4), "launches_per_step": launches,
                           "weight_GBps_per_step": round(wbytes / (dt / args.steps) / 1e9, 1),
-                          "workload": "C5 model (32 layers, Q4_0 layers, Q6_K head: one GEMV per sequence), "
+                          "workload": "C5 model (32 layers, Q4_0 layers, Q6_K head), "
                                       "16-id prompts then timed lockstep steps", "data": "synthetic"}), flush=True)
         log(f"{n} sequences: {tok_s:.1f} tokens/s aggregate ({dt * 1e3 / args.steps:.3f} ms per step)")
     return 0
@@ -500,7 +500,7 @@ def main() -> int:
     prefill = None
     if not args.direct and args.prompt > 1:  # the same prompt positions again, batched (bit-identical state)
         m.reset(prompt[:args.prompt])
-        warm = m.prefill(min(32, args.prompt - 1))  # captures the full-chunk graph (once per model), untimed
+        warm = m.prefill(min(32, args.prompt - 1))  # untimed: the chunks' scratch (once per model)
         m.reset(prompt[:args.prompt])
         t = time.perf_counter()
         if warm and m.prefill(args.prompt - 1):
@@ -509,9 +509,8 @@ def main() -> int:
             prefill = {"positions": args.prompt - 1, "batched_tokens_per_s": round((args.prompt - 1) / t_pre, 1),
                        "decode_step_tokens_per_s": round((args.prompt - 1) / t_steps, 1),
                        "method": "chunks of up to 512 tokens: GEMM projections, conv and DeltaNet over the tokens in order, "
-                                 "attention over the chunk's tokens in one launch pair; full chunks replay one "
-                                 "captured graph (captured by an untimed first prefill); wall time of the whole "
-                                 "prefill call"}
+                                 "attention in batches of the chunk's tokens; full chunks replay one captured "
+                                 "graph; wall time of the whole prefill call, after an untimed one of 32 tokens"}
             log(f"prompt: {args.prompt - 1} positions batched in {t_pre:.3f} s ({prefill['batched_tokens_per_s']} tok/s) "
                 f"vs {t_steps:.3f} s as decode steps")
         else:

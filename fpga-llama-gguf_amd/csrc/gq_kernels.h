@@ -294,22 +294,29 @@ constexpr int GEMV_MAXK = 16384;  // GEMV columns at most
 constexpr int GEMM_MAX_TOK = 32;  // tokens of one GEMM command (two tiles of 16)
 constexpr int GEMM_WIDE_TOK = 512;  // tokens of a batched GEMV in the model driver's own lists (prompt chunks)
 // Q6_K GEMMs of at least this many tokens and weights take the matrix-core form, the others the small-token GEMV in launches
-// of up to 4 tokens (4096 x 4096, us at 2 / 3 / 4 / 8 / 32 tokens, quantization included: 17.6 / 17.5 / 17.3 / 17.4 / 19.7
-// against 18.5 / 23.4 / 25.8 / 46.3 / 169; 8192 x 4096 at 2 tokens 21.9 against 20.3). Below 2^24 weights, less than an
-// output head has, the difference at 3 and 4 tokens is 1 to 5 us, and the small-token form's launch counts are kept.
+// of up to 4 tokens. The bound on tokens is where the times cross for many weights (us at 2 / 3 / 4 / 8 / 32 tokens,
+// quantization included: 4096 x 4096 17.6 / 17.5 / 17.3 / 17.4 / 19.7 against 18.5 / 23.4 / 25.8 / 46.3 / 169; 8192 x 4096 at 2
+// tokens 21.9 against 20.3). The bound on weights is not: it was set for output heads, and commands on smaller matrices keep
+// their launches. There the matrix cores lose at 3 tokens up to about 2^21 weights (1024 x 1024 8.2 against 5.8) and win at
+// every size measured from 5 tokens on (5 / 32 tokens: 256 x 2048 9.3 / 10.8 against 14.3 / 81; 1024 x 4096 12.4 / 15.1 against
+// 23.7 / 140; 1024 x 12288 28.9 / 33.1 against 67.4 / 418).
 constexpr unsigned GEMM_KQ_TOK = 3;
 constexpr unsigned long long GEMM_KQ_SIZE = 1ull << 24;
 // Q4_0 SwiGLU pairs of 3 and 4 tokens: from this many weights a matrix on the matrix cores with their quantization launch (us
-// at 3 / 4 tokens: 9728 x 2560 15.1 / 15.1 against 16.6 / 18.0, 12288 x 4096 19.8 / 19.6 against 20.6 / 22.3, 4096 x 4096
-// 11.7 / 11.8 against 12.0 / 12.8). Q8_0 stays on the small-token GEMV (9728 x 2560 19.9 / 19.9 against 18.0 / 19.8).
+// at 3 / 4 tokens: 4096 x 4096 11.7 / 11.8 against 12.0 / 12.8, 9728 x 2560 15.1 / 15.1 against 16.6 / 18.0, 12288 x 4096 19.8 /
+// 19.6 against 20.6 / 22.3). Below, 3 tokens gain nothing (4096 x 2048 9.3 against 9.2, 2048 x 1024 7.4 against 6.8); 4 alone
+// would (9.2 against 10.9, 7.5 against 8.0). Q8_0 stays on the small-token GEMV (4096 x 4096 15.4 / 15.5 against 13.7 / 13.9,
+// 9728 x 2560 19.7 / 19.9 against 17.7 / 19.5, 12288 x 4096 29.8 / 29.7 against 25.7 / 26.8).
 constexpr unsigned GEMM_PAIR_TOK = 3;
 constexpr unsigned long long GEMM_PAIR_SIZE = 1ull << 24;
 // Token rows the activation scratch holds for n_tok tokens: whole tiles of 16, past 32 whole groups of 64.
 constexpr int gemm_pad(int n_tok) { return n_tok > 32 ? (n_tok + 63) / 64 * 64 : (n_tok + 15) / 16 * 16; }
 constexpr int ATTN_CHUNK = 64;
 // attn_tile_kernel's smallest head_dim (lanes are elements of the values) and token count: it and the combine after it cost
-// a launch more than attn_group_kernel, which is the faster for few tokens at short positions (head_dim 256, position 100:
-// 8 tokens 25 us against 29, 16 tokens 33 against 32, 32 tokens 47 against 38; 128: 28 / 24, 40 / 28, 64 / 34).
+// a launch more than attn_group_kernel, which is the faster for few tokens at short positions (us at position 100, 16 heads:
+// of 256, 8 tokens 20 against 24 by tiles, 12 24 / 25, 16 28 / 27, 32 42 / 33; of 128, 18 / 19, 21 / 19, 24 / 21, 37 / 24). The
+// position lies in device memory, so the rule is drawn at the short ones; at the end of a long cache the tiles are ahead from 2
+// tokens on (position 8000, heads of 256: 2 tokens 69 against 32, 8 tokens 144 against 57, 32 tokens 442 against 160).
 constexpr int ATTN_TILE_HD = 64, ATTN_TILE_TOK = 16;
 inline bool attn_tiled(const AttnArgs & a) { return a.head_dim >= ATTN_TILE_HD && !a.seq_ctx && a.n_tok >= ATTN_TILE_TOK; }
 constexpr int ATTN_MAXG = 8;  // q heads per KV head

@@ -200,10 +200,10 @@ def _decode_state(m, cfg, npos):
 
 @pytest.mark.parametrize("q4_1", [False, True])
 def test_batched_prefill_equals_decode_steps(gq, q35, q4_1):
-    """The batched prefill (GEMM commands over chunks of up to 32 prompt tokens, the conv and DeltaNet step over the
-    tokens in order, attention token by token) leaves the model where the decode steps do, bit for bit: DeltaNet
+    """The batched prefill (GEMM commands over the chunk's prompt tokens, the conv and DeltaNet step over the
+    tokens in order, attention in batches) leaves the model where the decode steps do, bit for bit: DeltaNet
     states, KV cache, token ids; and the generation that follows has identical tokens, logits and hidden state. C5
-    widths, 4 layers (3 DeltaNet + 1 attention); 44 prompt positions = chunks of 32 and 12; and a prefill split
+    widths, 4 layers (3 DeltaNet + 1 attention); 44 prompt positions, part of a chunk of 96; and a prefill split
     around decode steps. With q4_1, two layers' ffn_down are Q4_1 (the type mix of real Qwen3.5 Q4_0 files)."""
     cfg = q35.Config(n_layer=4, n_ctx=96)
     types = {f"blk.{il}.ffn_down.weight": gq.Q4_1 for il in (1, 3)} if q4_1 else None
@@ -255,11 +255,12 @@ def test_batched_prefill_declines_unbatchable_models(gq, q35):
 
 
 @pytest.mark.parametrize("wtype,n_prompt,outliers", [("q4_0", 34, False), ("q4_1", 66, False), ("q8_0", 130, False),
-                                                     ("q4_0", 517, False), ("q4_0", 100, True), ("q8_0", 66, True)])
+                                                     ("q4_0", 517, False), ("q4_0", 100, True), ("q8_0", 66, True),
+                                                     ("q8_0", 1030, False)])
 def test_prompt_chunks_of_many_tokens_equal_decode_steps(gq, q35, wtype, n_prompt, outliers):
     """Prompt chunks past 32 tokens (the batched GEMV over groups of 64 tokens, the token-parallel conv, attention in
-    batches of 32): one token past a batch or group, two and more groups, a full chunk of 512 and a remainder; with
-    activation outliers (norm weights of 2e3 in some columns) the steps that sum term by term. States, cache, ids and the
+    batches): one token past 32 or a group, two and more groups, a full chunk of 512 and a remainder, two full ones (replays
+    of one graph); with activation outliers (norm weights of 2e3 in some columns) the steps that sum term by term. States, cache, ids and the
     generation after it equal the decode steps' bit for bit."""
     cfg = q35.Config(n_layer=4, n_embd=1024, n_ff=1536, n_vocab=1040, n_head=4, n_head_kv=1, head_dim=128, n_rot=32,
                      ssm_k_heads=2, ssm_v_heads=4, n_ctx=n_prompt + 8, wtype=getattr(gq, wtype.upper()))
