@@ -161,9 +161,11 @@ struct gemvq_ctx {
     uint16_t * gemm_s = nullptr;  // and their Q8_1 block sums (for Q4_1 weights)
     float * gemm_b = nullptr;     // and their parts of the term bounds
     uint8_t * wide = nullptr;     // the same for a list of the model driver's prompt chunks (up to GEMM_WIDE_TOK rows)
-    float * gdn_prep[2] = {};     // norms and gates of a GDN command's tokens: of a caller's list, of a prompt chunk's
-    float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens); the
-    size_t attn_wide_n = 0;       // smaller ones before it, which captured graphs may still use
+    float * gdn_prep = nullptr;   // norms and gates of a GDN command's tokens, and the floats it holds; the smaller
+    size_t gdn_prep_n = 0;        // buffers before it, which captured graphs may still use
+    std::vector<float *> gdn_prep_old;
+    float * attn_wide = nullptr;  // attention partials and queries of a prompt chunk's batch (gq_attn_tokens), likewise
+    size_t attn_wide_n = 0;
     std::vector<float *> attn_wide_old;
     size_t scratch_max = ~size_t(0);  // largest allocation for scratch that a launch can do without (set at creation)
     int max_tok = GEMM_MAX_TOK;   // tokens a command of the list being compiled may hold (gq_wide_lists)
@@ -775,7 +777,7 @@ struct Compiler {
                                                 {k[5], uint64_t(k[5]) + uint64_t(sg) * (ntok - 1) + hv},
                                                 {k[6], uint64_t(k[6]) + uint64_t(sg) * (ntok - 1) + hv}};
                 if (ntok >= GDN_PREP_TOK && !seqs && !meet_any({{k[7], uint64_t(k[7]) + yz + hv * 128}}, reads))
-                    a.prep = gdn_prep();
+                    a.prep = gdn_prep(hk, hv);
                 if ((flags & GEMVQ_GDN_GATED) && ntok == 1 && fold_gated(cmds, n, next, k[7], hv * 128, k2[7], k2[6])) {
                     // the gated norm runs in the next GEMV's activation prologue: the step writes its raw output
                     // to scratch, and that GEMV writes the gated values to y as the norm would have
@@ -985,13 +987,19 @@ struct Compiler {
         return attn_wide_part(b, n_head, n_tok) + size_t(n_tok) * n_head * b.head_dim;
     }
 
-    // The buffer for the norms and gates of a GDN command's tokens, allocated once for the most tokens and heads that a command
-    // of the list may have (2 MiB; 32 MiB in the model driver's lists): commands run in order and share it, and its size does
-    // not depend on the commands seen. NULL (they are formed in the step) without memory for it.
-    float * gdn_prep() const {
-        float *& p = c->gdn_prep[c->max_tok > GEMM_MAX_TOK];
-        const size_t n = size_t(c->max_tok) * gdn_prep_row(GDN_MAX_HEADS, GDN_MAX_HEADS);
-        if (!p) p = static_cast<float *>(optional_scratch(c, n * sizeof(float)));
+    // The buffer for the norms and gates of a GDN command's tokens; NULL (they are formed in the step) without memory for it.
+    // Commands run in order and share it. It is made for the most tokens that a command of the list may have, whatever this
+    // one's count, and where a later list or more heads need a larger one at least doubles: all of them together stay below
+    // four times the largest need (17 KB a token at 32 value heads).
+    float * gdn_prep(uint32_t hk, uint32_t hv) const {
+        const size_t need = size_t(c->max_tok) * gdn_prep_row(int(hk), int(hv));
+        if (c->gdn_prep_n >= need) return c->gdn_prep;
+        const size_t n = std::max(need, 2 * c->gdn_prep_n);
+        float * p = static_cast<float *>(optional_scratch(c, n * sizeof(float)));
+        if (!p) return nullptr;
+        if (c->gdn_prep) c->gdn_prep_old.push_back(c->gdn_prep);
+        c->gdn_prep = p;
+        c->gdn_prep_n = n;
         return p;
     }
 
@@ -1671,7 +1679,8 @@ void gemvq_ctx_destroy(gemvq_ctx * c) {
     hipFree(c->gemm_s);
     hipFree(c->gemm_b);
     hipFree(c->wide);
-    for (float * p : c->gdn_prep) hipFree(p);
+    hipFree(c->gdn_prep);
+    for (float * p : c->gdn_prep_old) hipFree(p);
     hipFree(c->attn_wide);
     for (float * p : c->attn_wide_old) hipFree(p);
     hipFree(c->ref_x);
@@ -1899,16 +1908,17 @@ int gemvq_run(gemvq_ctx * c, const uint32_t * cmds, unsigned n) {
     return e == hipSuccess ? 0 : fail(c, e, "run");
 }
 
-// Whether the lists compiled from now on may hold commands of up to GEMM_WIDE_TOK tokens (GEMM, CONV, GDN, GET_ROWS; ATTN: gq_attn_tokens): for
-// the prompt chunks of the model driver, which switches it on around its own lists. A caller's lists keep the limits of
-// the header. GEMVQ_EINVAL without memory for their scratch: the limits stay, the context is as before.
-__attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int on) {
-    if (!c) return GEMVQ_EINVAL;
-    if (on && !c->wide) {
+// The lists compiled from now on may hold commands of up to `tokens` tokens (GEMM, CONV, GDN, GET_ROWS; ATTN:
+// gq_attn_tokens), at most GEMM_WIDE_TOK: for the prompt chunks of the model driver, which switches it on around its own
+// lists. A caller's lists keep the limits of the header (tokens = 0). GEMVQ_EINVAL without memory for their scratch: the limits
+// stay, the context is as before.
+__attribute__((visibility("hidden"))) int gq_wide_lists(gemvq_ctx * c, int tokens) {
+    if (!c || tokens > GEMM_WIDE_TOK) return GEMVQ_EINVAL;
+    if (tokens && !c->wide) {
         c->wide = static_cast<uint8_t *>(optional_scratch(c, Compiler::WIDE_BYTES));
         if (!c->wide) return GEMVQ_EINVAL;
     }
-    c->max_tok = on ? GEMM_WIDE_TOK : GEMM_MAX_TOK;
+    c->max_tok = std::max(tokens, GEMM_MAX_TOK);
     return 0;
 }
 

@@ -399,7 +399,7 @@ bool build_commands(gemvq_qwen35 & m, std::string & err) {
 }  // namespace
 
 extern "C" void gq_set_error(gemvq_ctx * ctx, const char * what);  // gq_runtime.hip
-extern "C" int gq_wide_lists(gemvq_ctx * ctx, int on);
+extern "C" int gq_wide_lists(gemvq_ctx * ctx, int tokens);
 extern "C" int gq_attn_tokens(gemvq_ctx * ctx, int kv, int n_head, int most);
 
 namespace {
@@ -561,7 +561,7 @@ int gemvq_qwen35_prefill(gemvq_qwen35 * m, int n) {
     // does a prompt without memory for the scratch of longer chunks
     int most = gemvq_arith(ctx) == GEMVQ_ARITH_REFERENCE ? int(GEMVQ_GEMM_MAX_TOK) : int(m->chunk);
     m->attn_batch = GEMVQ_GEMM_MAX_TOK;
-    if (most > int(GEMVQ_GEMM_MAX_TOK) && gq_wide_lists(ctx, 1)) most = GEMVQ_GEMM_MAX_TOK;
+    if (most > int(GEMVQ_GEMM_MAX_TOK) && gq_wide_lists(ctx, most)) most = GEMVQ_GEMM_MAX_TOK;
     if (most > int(GEMVQ_GEMM_MAX_TOK)) {
         for (int il = 0; il < m->c.n_layer; ++il)  // (the layers' caches are alike)
             if (is_attn(m->c, il)) {
